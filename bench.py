@@ -26,7 +26,7 @@ if ROOT not in sys.path:
 
 METRIC = "MCUPS + % HBM roofline (1 GPU); adjoint/forward cost ratio; batched vs plain"
 HBM_PEAK_GBS = 8000.0
-KERNELS = {0: "wave_uniform_k", 1: "wave_march_k", 7: "wave_row_k", 8: "wave_row_k", 9: "wave_row_k",
+KERNELS = {0: "wave_star_k", 1: "wave_march_k", 7: "wave_row_k", 8: "wave_row_k", 9: "wave_row_k",
            11: "wave_row2_k", 12: "wave_row2_k"}
 
 

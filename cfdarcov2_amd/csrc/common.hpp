@@ -69,6 +69,9 @@ struct cfd_ctx_s {
 
 namespace cfd {
 
+// Last-level cache (Infinity Cache) of an MI355X
+constexpr int64_t kLastLevelCacheBytes = int64_t(256) << 20;
+
 // Constant geometry of an exactly uniform hex mesh, per axis a = 0 (x), 1 (y), 2 (z).
 template <class T> struct UniformGeo {
     int64_t X, Y, Z;
@@ -155,10 +158,9 @@ struct cfd_mesh_s {
     // host copies of the reference-layout tables are rebuilt on demand
     std::vector<double> vertex_offsets;
     bool has_offsets = false;
-    // fused acoustic step on uniform meshes: variant 0 = per-thread kernel,
+    // fused acoustic step on uniform meshes: variant 0 = star form,
     // 1 = 2.5D marching tiles, 7-9 = row form, 11-12 = two-step row form (the
-    // variants of cfd_mesh_set_wave_shape); uniform meshes whose z extent
-    // suits the row form start on it
+    // variants of cfd_mesh_set_wave_shape); create_mesh picks the first one
     int wave_variant = 1;
     int wave_ty = 16;
     int wave_L = 32;

@@ -59,6 +59,13 @@ template <class T>
 void launch_wave_march(const cfd_mesh_s* m, void* const a[4], void* const b[4], double K, const void* Kf, double dt,
                        int64_t nsteps, int variant, int ty, int L, int remap, hipStream_t s);
 
+// Star form of the acoustic step (wave_star.hip): any extents and alignment.
+// Returns false (nothing launched) for meshes whose planes exceed its 32-bit
+// offsets.
+template <class T>
+bool launch_wave_star(const UniformGeo<T>& g, void* const* in, void* const* out, double K, const void* Kf, double dt,
+                      hipStream_t s);
+
 // Row form of the acoustic step (wave_row.hip): z extent a multiple of 4, at
 // most 256.  order: bit 0 XCD-contiguous tiles, bit 1 tiles last to first;
 // cache: bit 0 non-temporal stores, bit 1 non-temporal loads.  Returns false

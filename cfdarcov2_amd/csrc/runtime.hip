@@ -200,7 +200,15 @@ template <class T> static void create_mesh(cfd_mesh_s* m, const cfd_hex_desc& d)
             m->heat_nw = 12;
             m->heat_L = 16;
         }
-        if (wave_row_supported(d.nz)) {  // row forms, the fastest measured at 256^3
+        // Acoustic step.  While both states (8 fields) fit the last-level
+        // cache the star form is the fastest measured at every size and
+        // extent (us/step, star / best row form / best march tiles; FP32
+        // 48^3: 4.0 / 5.2 / 6.5, 128^3: 14.5 / 14.3 / 20.2, 200^3: 42.7 /
+        // 48.6 / 63.7; FP64 128^3: 23.0 / 26.5 / 28.3); its re-read rows cost
+        // it beyond (FP32 256^3: 155 / 71 / 140; FP64 200^3: 149 / 106 / 154).
+        if (8 * d.nx * d.ny * d.nz * int64_t(sizeof(T)) <= kLastLevelCacheBytes) {
+            m->wave_variant = 0;
+        } else if (wave_row_supported(d.nz)) {
             if constexpr (sizeof(T) == 4) {  // two steps per pass
                 m->wave_variant = 11;
                 m->wave_ty = 8;
@@ -212,6 +220,10 @@ template <class T> static void create_mesh(cfd_mesh_s* m, const cfd_hex_desc& d)
                 m->wave_L = 32;
                 m->wave_remap = 1;
             }
+        } else {  // z extents the row forms cannot take
+            m->wave_variant = 1;
+            m->wave_ty = 4;
+            m->wave_L = 16;
         }
         if constexpr (sizeof(T) == 4) m->ug32 = u; else m->ug64 = u;
     } else {

@@ -420,61 +420,9 @@ __global__ void __launch_bounds__(256) heat_general_k(GeneralGeo<T> g, const T* 
 }
 
 // ---------------------------------------------------------------------------
-// Fused acoustic step (uniform mesh), single pass per step.
-//   u' = dt*(-Gx(p)) + u, v' = dt*(-Gy(p)) + v, w' = dt*(-Gz(p)) + w
-//   p' = dt*(K*((Gx(u') + Gy(v')) + Gz(w'))) + p
-// p' needs u' at x+-1, v' at y+-1, w' at z+-1, which each thread recomputes
-// from p (distance 2) and the old velocities; the recomputation is bitwise
-// identical to the neighbour's own update, so the result equals the
-// sequential (Gauss-Seidel across equations) evaluation.  Walls: the normal
-// velocity's face value is zero; p is zero-gradient (neighbour = self).
+// Fused acoustic step.  Uniform meshes: wave_star.hip, wave_row.hip,
+// wave_row2.hip, wave_march.hip.
 // ---------------------------------------------------------------------------
-template <class T>
-__device__ inline T vel_update(const UniformGeo<T>& g, const T* __restrict__ p, const T* __restrict__ q,
-                               int64_t j, int64_t stride, bool lo_wall, bool hi_wall, int a, T dt) {
-    const T pc = p[j];
-    const T pl = lo_wall ? pc : p[j - stride];
-    const T ph = hi_wall ? pc : p[j + stride];
-    const T G = gg_pair_u(g, lin(pc, pl), lin(pc, ph), g.area[a]);
-    return dt * (-G) + q[j];
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) wave_uniform_k(UniformGeo<T> g, const T* __restrict__ p,
-                                                      const T* __restrict__ u, const T* __restrict__ v,
-                                                      const T* __restrict__ w, T* __restrict__ po,
-                                                      T* __restrict__ uo, T* __restrict__ vo, T* __restrict__ wo,
-                                                      T K, const T* __restrict__ Kf, T dt) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const int64_t sx = g.Y * g.Z, sy = g.Z, sz = 1;
-    const T* vel[3] = {u, v, w};
-    T* velo[3] = {uo, vo, wo};
-    const int64_t crd[3] = {c.x, c.y, c.z};
-    const int64_t ext[3] = {g.X, g.Y, g.Z};
-    const int64_t str[3] = {sx, sy, sz};
-    T S = T(0);
-    for (int a = 0; a < 3; ++a) {
-        const bool lo = crd[a] == 0, hi = crd[a] == ext[a] - 1;
-        const T qc = vel_update(g, p, vel[a], c.id, str[a], lo, hi, a, dt);
-        velo[a][c.id] = qc;
-        T f_lo = T(0), f_hi = T(0);  // wall faces carry zero normal velocity
-        if (!lo) {
-            const int64_t j = c.id - str[a];
-            const T ql = vel_update(g, p, vel[a], j, str[a], crd[a] - 1 == 0, false, a, dt);
-            f_lo = lin(qc, ql);
-        }
-        if (!hi) {
-            const int64_t j = c.id + str[a];
-            const T qh = vel_update(g, p, vel[a], j, str[a], false, crd[a] + 1 == ext[a] - 1, a, dt);
-            f_hi = lin(qc, qh);
-        }
-        const T G = gg_pair_u(g, f_lo, f_hi, g.area[a]);
-        S = (a == 0) ? G : S + G;
-    }
-    const T k = Kf ? Kf[c.id] : K;
-    po[c.id] = dt * (k * S) + p[c.id];
-}
 
 // General-mesh acoustic step.  Skewed face normals make every gradient
 // component depend on all six faces, so the step runs as two launches: the
@@ -653,19 +601,7 @@ void launch_wave(const cfd_mesh_s* m, void* const a[4], void* const b[4], double
         }
         return;
     }
-    if (m->wave_variant >= 1) {
-        launch_wave_march<T>(m, a, b, K, Kf, dt, nsteps, m->wave_variant, m->wave_ty, m->wave_L, m->wave_remap, s);
-        return;
-    }
-    const auto& g = ugeo<T>(m);
-    for (int64_t k = 0; k < nsteps; ++k) {
-        void* const* in = (k & 1) ? b : a;
-        void* const* out = (k & 1) ? a : b;
-        wave_uniform_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(
-            g, (const T*)in[0], (const T*)in[1], (const T*)in[2], (const T*)in[3], (T*)out[0], (T*)out[1],
-            (T*)out[2], (T*)out[3], T(K), (const T*)Kf, T(dt));
-        check_launch();
-    }
+    launch_wave_march<T>(m, a, b, K, Kf, dt, nsteps, m->wave_variant, m->wave_ty, m->wave_L, m->wave_remap, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -13,8 +13,8 @@
 // TYT rows to the same per TY rows without more threads per workgroup.
 // LDS planes are double-buffered (two barriers per plane) and the next plane's
 // global loads are issued before the current plane's arithmetic.  The
-// arithmetic is the sequence of the reference evaluation (see wave_uniform_k in
-// stencil.hip), so results equal the oracle bit for bit.
+// arithmetic is the sequence of the reference evaluation (see
+// wave_star.hip), so results equal the oracle bit for bit.
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
@@ -59,7 +59,7 @@ static void launch_one(const UniformGeo<T>& g, void* const* in, void* const* out
     CFD_HIP(hipGetLastError());
 }
 
-// Variant 1: tile_rows selects (threads in y) x (rows per thread): 4 = 4x1,
+// Variant 0: star form.  Variant 1: tile_rows selects (threads in y) x (rows per thread): 4 = 4x1,
 // 8 = 4x2, 16 = 4x4, 32 = 8x4.  Variants 7 to 9 take the row form
 // (wave_row.hip) and 11 and 12 the two-step row form (wave_row2.hip).
 template <class T>
@@ -85,6 +85,10 @@ void launch_wave_march(const cfd_mesh_s* m, void* const a[4], void* const b[4], 
     for (int64_t k = k0; k < nsteps; ++k) {
         void* const* in = (k & 1) ? b : a;
         void* const* out = (k & 1) ? a : b;
+        if (variant == 0) {
+            if (!launch_wave_star<T>(g, in, out, K, Kf, dt, s)) launch_one<T, 4, 1>(g, in, out, K, Kf, dt, L, 0, s);
+            continue;
+        }
         if (variant >= 7) {  // row form; misaligned fields take the 4-row march tile
             // remap bit 1: odd steps walk the tiles in reverse.  Cache policy:
             // 7 non-temporal stores, 8 plain, 9 non-temporal loads

@@ -398,7 +398,9 @@ int cfd_mesh_geometry(cfd_mesh_t mesh, cfd_geometry* out);
 /* Kernel shape of the fused acoustic step on uniform meshes (no counterpart
  * in the reference, whose JIT kernels use fixed 64-thread blocks,
  * src/fvm3d.cpp:1306-1308):
- *   0  one thread per cell (the form for small meshes);
+ *   0  star form: 16 bytes of consecutive z-cells per thread, neighbours'
+ *      velocities recomputed, no march (meshes whose fields stay in the
+ *      last-level cache; any extents);
  *   1  2.5D marching kernel, `tile_rows` (4, 8, 16 or 32) y-rows of 64 z-cells
  *      per workgroup carried by 4 (8 for 32) thread rows; any z extent;
  *   7  row form (z extent a multiple of 4 and at most 256): one wave per z row
@@ -416,8 +418,9 @@ int cfd_mesh_geometry(cfd_mesh_t mesh, cfd_geometry* out);
  * other step walk its tiles in reverse.  The row forms return
  * CFD_E_UNSUPPORTED for other z extents; other variant numbers (2 to 6 and 10
  * were forms the autotuner never chose) return CFD_E_INVALID.
- * Uniform meshes whose z extent suits the row form start on variant 11 (FP32)
- * or 7 (FP64).
+ * Uniform meshes start on variant 0 when both states (8 fields) fit 256 MiB,
+ * else on variant 11 (FP32) or 7 (FP64) where the z extent suits the row form
+ * and on variant 1 (4 rows, 16 planes) elsewhere.
  * All variants give bit-identical results.  Set by the autotuner
  * (cfdarcov2_amd/autotune.py). */
 int cfd_mesh_set_wave_shape(cfd_mesh_t mesh, int variant, int tile_rows, int chunk, int xcd_remap);
