@@ -101,6 +101,18 @@ template <class T> struct GeneralGeo {
     T dl;
 };
 
+// Geometry of a structured mesh whose every face is exactly normal to its axis
+// (any spacing that is not dyadic, or a graded lattice): the general mesh's
+// face arrays reduce to one width per cell layer and one alpha_d per face
+// layer, and only the volume is data per cell.  create_mesh compares the
+// general arrays with these values, so both give the same bits.
+template <class T> struct LatticeGeo {
+    const T* w[3];      // per axis: width of cell layer k; a face's area is the product of the other two
+    const T* alpha[3];  // per axis: alpha_d of face layer k = 0..n; at the walls, where the reference
+                        // multiplies a zero difference, any finite value (1)
+    const T* vol;       // per cell
+};
+
 // Finite-volume geometry of the Euler stepper: per face family the +axis unit
 // normal and the area of the face's vector area, and the cell volumes built from
 // the vector areas (built on first use).
@@ -153,6 +165,11 @@ struct cfd_mesh_s {
     cfd::UniformGeo<double> ug64{};
     cfd::GeneralGeo<float> gg32{};
     cfd::GeneralGeo<double> gg64{};
+    // general meshes whose faces are exactly axis-aligned (lat_block: the tables)
+    bool lattice = false;
+    cfd::LatticeGeo<float> lg32{};
+    cfd::LatticeGeo<double> lg64{};
+    void* lat_block = nullptr;
     void* dev_block = nullptr;     // one allocation holding all device geometry
     int64_t device_bytes = 0;
     // host copies of the reference-layout tables are rebuilt on demand

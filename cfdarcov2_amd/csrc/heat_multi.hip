@@ -9,7 +9,7 @@
 // s + 1 reads; at the walls a cell's outer neighbour is the cell itself, as in
 // the single-step kernel.  Cells near a box's sides are computed by several
 // workgroups (the redundant work that buys K - 1 fewer launches).  Each cell's
-// arithmetic is heat_uniform_cell's (stencil.hip), in the same order, so ns
+// arithmetic is heat_star_k's (ops_star.hip), in the same order, so ns
 // steps here equal ns single steps bit for bit.
 //
 // Threads: 64 lanes along z x 16 waves.  Every wave owns a fixed set of the

@@ -59,11 +59,20 @@ template <class T>
 void launch_wave_march(const cfd_mesh_s* m, void* const a[4], void* const b[4], double K, const void* Kf, double dt,
                        int64_t nsteps, int variant, int ty, int L, int remap, hipStream_t s);
 
-// Star form of the acoustic step (wave_star.hip): any extents and alignment.
-// Returns false (nothing launched) for meshes whose planes exceed its 32-bit
-// offsets.
+// Star forms (star.hpp; any extents and alignment): the acoustic step on
+// uniform meshes (wave_star.hip); one acoustic step on an axis-aligned lattice,
+// and the gradient, Laplacian and heat step on both (ops_star.hip)
 template <class T>
-bool launch_wave_star(const UniformGeo<T>& g, void* const* in, void* const* out, double K, const void* Kf, double dt,
+void launch_wave_lattice(const cfd_mesh_s* m, void* const* in, void* const* out, double K, const void* Kf, double dt,
+                         hipStream_t s);
+template <class T>
+void launch_grad_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s);
+template <class T> void launch_lapl_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s);
+template <class T>
+void launch_heat_star(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
+                      hipStream_t s);
+template <class T>
+void launch_wave_star(const UniformGeo<T>& g, void* const* in, void* const* out, double K, const void* Kf, double dt,
                       hipStream_t s);
 
 // Row form of the acoustic step (wave_row.hip): z extent a multiple of 4, at

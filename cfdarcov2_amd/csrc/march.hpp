@@ -290,7 +290,7 @@ template <class T, int TYT, int R> struct HeatLds {
 
 // One (zt, yt, xc) tile of the heat step dt * (alpha * lapl(T)) + T on a
 // uniform mesh, marching along x with T(x-1), T(x), T(x+1) in registers and the
-// plane's y/z neighbours in LDS.  The arithmetic is heat_uniform_k's
+// plane's y/z neighbours in LDS.  The arithmetic is heat_star_k's
 // (Grad2Var with neighbour = self on the walls), so the two agree bit for bit.
 template <class T, int TYT, int R, bool PW = false>
 __device__ inline void heat_march_tile(const UniformGeo<T>& g, const T* __restrict__ Tin, T* __restrict__ Tout,

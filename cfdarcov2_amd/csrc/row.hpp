@@ -413,7 +413,7 @@ __device__ inline void row_tile(const UniformGeo<T>& g, const T* __restrict__ p,
 // form: TY output waves of RW rows each and two halo waves (rows y0-1 and
 // y0+TY*RW) that only put their T row into the LDS plane; x neighbours in a
 // per-lane register queue, z neighbours in the lane's registers or the adjacent
-// lane's.  The arithmetic is heat_uniform_k's (Grad2Var with neighbour = self
+// lane's.  The arithmetic is heat_star_k's (Grad2Var with neighbour = self
 // on the walls).
 template <int TY, bool PW, bool XB, bool NTL>
 __device__ inline void heat_row_tile(const UniformGeo<float>& g, const float* __restrict__ Tin,
@@ -515,7 +515,7 @@ __device__ inline void heat_row_tile(const UniformGeo<float>& g, const float* __
 // the second on the output rows, which alone are stored.  Iteration x takes
 // the first step at plane x and the second at plane x-1, the second reading
 // the first's planes x-2 .. x from a register queue and its y-neighbours from
-// an LDS plane.  The arithmetic per cell is heat_uniform_k's.
+// an LDS plane.  The arithmetic per cell is heat_star_k's.
 template <class T, int NW, bool PW, bool XB, bool NTL>
 __device__ inline void heat_row2_tile(const UniformGeo<T>& g, const T* __restrict__ Tin, T* __restrict__ Tout,
                                       T alpha, T dt, int64_t x0, int64_t x1, int y0, int wv,

@@ -180,6 +180,68 @@ static void upload_general(cfd_mesh_s* m, const HexGeometry<T>& g, GeneralGeo<T>
     CFD_HIP(hipStreamSynchronize(s));
 }
 
+// Fills lg with the tables of LatticeGeo when every normal, area and interior
+// alpha_d of the mesh equals what the kernels form from them; returns false
+// otherwise.
+template <class T> static bool upload_lattice(cfd_mesh_s* m, const HexGeometry<T>& g, LatticeGeo<T>& lg, hipStream_t s) {
+    const int64_t ext[3] = {g.X, g.Y, g.Z};
+    const std::vector<T>* vert[3] = {&g.vx, &g.vy, &g.vz};
+    const int64_t vstr[3] = {(g.Y + 1) * (g.Z + 1), g.Z + 1, 1};
+    int64_t off[7] = {0};
+    for (int a = 0; a < 3; ++a) {
+        off[a + 1] = off[a] + ext[a];
+    }
+    for (int a = 0; a < 3; ++a) off[a + 4] = off[a + 3] + ext[a] + 1;
+    std::vector<T> host(size_t(off[6]), T(1));
+    T *w[3], *al[3];
+    for (int a = 0; a < 3; ++a) {
+        w[a] = host.data() + off[a];
+        al[a] = host.data() + off[3 + a];
+        for (int64_t k = 0; k < ext[a]; ++k) w[a][k] = (*vert[a])[size_t((k + 1) * vstr[a])] - (*vert[a])[size_t(k * vstr[a])];
+    }
+    // interior alpha_d of the layers from their first face
+    for (int64_t k = 1; k < g.X; ++k) al[0][k] = g.falpha[2][size_t(g.xface(k, 0, 0))];
+    for (int64_t k = 1; k < g.Y; ++k) al[1][k] = g.falpha[1][size_t(g.yface(0, k, 0))];
+    for (int64_t k = 1; k < g.Z; ++k) al[2][k] = g.falpha[0][size_t(g.zface(0, 0, k))];
+    int bad = 0;
+    for (int fam = 0; fam < 3; ++fam) {
+        const int axis = 2 - fam;
+        const int64_t nx = g.X + (axis == 0), ny = g.Y + (axis == 1), nz = g.Z + (axis == 2);
+#pragma omp parallel for schedule(static) reduction(+ : bad)
+        for (int64_t x = 0; x < nx; ++x) {
+            if (bad) continue;
+            for (int64_t y = 0; y < ny; ++y)
+                for (int64_t z = 0; z < nz; ++z) {
+                    const int64_t f = fam == 0 ? g.zface(x, y, z) : fam == 1 ? g.yface(x, y, z) : g.xface(x, y, z);
+                    const P3<T> n = HexGeometry<T>::axis_normal(g.fnorm(fam, f), 2 * fam);
+                    const T comp[3] = {n.x, n.y, n.z};
+                    for (int d = 0; d < 3; ++d) bad += !(comp[d] == (d == axis ? T(1) : T(0)));
+                    const T A = axis == 0 ? w[1][y] * w[2][z] : axis == 1 ? w[0][x] * w[2][z] : w[0][x] * w[1][y];
+                    bad += !(g.farea[fam][size_t(f)] == A && A > T(0) && std::isfinite(A));
+                    const int64_t k = axis == 0 ? x : axis == 1 ? y : z;
+                    if (k > 0 && k < ext[axis]) bad += !(g.falpha[fam][size_t(f)] == al[axis][k]);
+                    else bad += !std::isfinite(g.falpha[fam][size_t(f)]);
+                }
+        }
+        if (bad) return false;
+    }
+    const int64_t bytes = off[6] * int64_t(sizeof(T));
+    try {
+        m->lat_block = pool_alloc(m->ctx, bytes, s);
+    } catch (const Error&) {
+        return false;  // at the pool's limit the mesh does without the tables
+    }
+    m->device_bytes += bytes;
+    CFD_HIP(hipMemcpyAsync(m->lat_block, host.data(), size_t(bytes), hipMemcpyHostToDevice, s));
+    CFD_HIP(hipStreamSynchronize(s));
+    const T* dev = (const T*)m->lat_block;
+    for (int a = 0; a < 3; ++a) {
+        lg.w[a] = dev + off[a];
+        lg.alpha[a] = dev + off[3 + a];
+    }
+    return true;
+}
+
 template <class T> static void create_mesh(cfd_mesh_s* m, const cfd_hex_desc& d) {
     HexGeometry<T> g;
     build_hex_geometry<T>(g, d.nx, d.ny, d.nz, T(d.dx), T(d.dy), T(d.dz), d.vertex_offsets);
@@ -232,6 +294,12 @@ template <class T> static void create_mesh(cfd_mesh_s* m, const cfd_hex_desc& d)
         gg.dl = dl;
         upload_general(m, g, gg, nullptr);
         if constexpr (sizeof(T) == 4) m->gg32 = gg; else m->gg64 = gg;
+        LatticeGeo<T> lg{};
+        if (!d.force_general && upload_lattice(m, g, lg, nullptr)) {
+            lg.vol = gg.vol;
+            m->lattice = true;
+            if constexpr (sizeof(T) == 4) m->lg32 = lg; else m->lg64 = lg;
+        }
     }
 }
 
@@ -605,6 +673,7 @@ int cfd_mesh_destroy(cfd_mesh_t mesh) {
         drop_heat_graph(mesh);
         if (mesh->capture) (void)hipStreamDestroy(mesh->capture);
         if (mesh->dev_block) pool_free(mesh->ctx, mesh->dev_block, nullptr);
+        if (mesh->lat_block) pool_free(mesh->ctx, mesh->lat_block, nullptr);
         if (mesh->fv_block) pool_free(mesh->ctx, mesh->fv_block, nullptr);
         if (mesh->dev_block || mesh->fv_block) CFD_HIP(hipStreamSynchronize(nullptr));
         delete mesh;

@@ -23,34 +23,39 @@ namespace star {
 template <class T, int W> struct VecOf {
     typedef T type __attribute__((ext_vector_type(W), aligned(sizeof(T))));
 };
-template <class T> struct VecOf<T, 1> { typedef T type; };
 
-// W values at an element offset of a row-plane pointer.  The pointer is uniform
-// over the workgroup and the offset 32 bits wide (star_fits), so an address is
-// one register.
-template <class T, int W> __device__ inline void load(const T* base, uint32_t off, T (&v)[W]) {
-    using V = typename VecOf<T, W>::type;
-    const V r = *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + size_t(off * uint32_t(sizeof(T))));
+// Offsets within a plane.  The vector form keeps them in 32 bits (planes below
+// 4 GiB), so an address is a base uniform over the workgroup plus one
+// register; rows shorter than a vector and larger planes take W = 1 with 64.
+template <int W> struct OffOf { using type = uint32_t; };
+template <> struct OffOf<1> { using type = uint64_t; };
+template <int W> using Off = typename OffOf<W>::type;
+
+template <class T, class O> __device__ inline T load1(const T* base, O off) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + O(off * O(sizeof(T))));
+}
+// W values at an element offset from a uniform pointer
+template <class T, int W> __device__ inline void load(const T* base, Off<W> off, T (&v)[W]) {
     if constexpr (W == 1) {
-        v[0] = r;
+        v[0] = load1(base, off);
     } else {
+        using V = typename VecOf<T, W>::type;
+        const V r = *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + Off<W>(off * Off<W>(sizeof(T))));
 #pragma unroll
         for (int i = 0; i < W; ++i) v[i] = r[i];
     }
 }
-template <class T> __device__ inline T load1(const T* base, uint32_t off) {
-    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + size_t(off * uint32_t(sizeof(T))));
-}
-template <class T, int W> __device__ inline void store(T* base, uint32_t off, const T (&v)[W]) {
-    using V = typename VecOf<T, W>::type;
-    V r;
+template <class T, int W> __device__ inline void store(T* base, Off<W> off, const T (&v)[W]) {
+    char* const a = reinterpret_cast<char*>(base) + Off<W>(off * Off<W>(sizeof(T)));
     if constexpr (W == 1) {
-        r = v[0];
+        *reinterpret_cast<T*>(a) = v[0];
     } else {
+        using V = typename VecOf<T, W>::type;
+        V r;
 #pragma unroll
         for (int i = 0; i < W; ++i) r[i] = v[i];
+        *reinterpret_cast<V*>(a) = r;
     }
-    *reinterpret_cast<V*>(reinterpret_cast<char*>(base) + size_t(off * uint32_t(sizeof(T)))) = r;
 }
 
 // Launch geometry: workgroups of bx units x by rows of one x-plane, nzb x nyb
@@ -84,8 +89,11 @@ inline Plan make_plan(int64_t X, int64_t Y, int64_t Z, int W) {
 inline dim3 plan_grid(const Plan& p) { return dim3(unsigned((p.blocks + 7) / 8 * 8)); }
 inline dim3 plan_block(const Plan& p) { return dim3(unsigned(p.bx), unsigned(p.by)); }
 
-// Whether a plane's byte offsets fit 32 bits
-inline bool fits(int64_t Y, int64_t Z, size_t elem) { return Y * Z * int64_t(elem) < (int64_t(1) << 32); }
+// Whether rows and planes suit the vector form of T
+template <class T> constexpr int kWidth = 16 / int(sizeof(T));
+template <class T> inline bool vector_form(int64_t Y, int64_t Z) {
+    return Z >= kWidth<T> && Y * Z * int64_t(sizeof(T)) < (int64_t(1) << 32);
+}
 
 // The thread's place: plane x (uniform), row y, first cell z0; false without work.
 template <int W> __device__ inline bool place(const Plan& p, int& x, int& y, int& z0) {
@@ -99,6 +107,105 @@ template <int W> __device__ inline bool place(const Plan& p, int& x, int& y, int
     if (y >= p.Y || zi * W >= p.Z) return false;
     z0 = min(zi * W, p.Z - W);
     return true;
+}
+
+// Element offsets of a thread's cells and of their six neighbours, clamped to
+// the mesh: a neighbour beyond a wall is the cell itself (the reference rule).
+template <int W> struct Offsets {
+    int64_t x0, xm1, xp1;           // planes
+    Off<W> o0, ym1, yp1, zm1, zp1;  // within a plane: the W cells, rows y-1 and y+1, cells z0-1 and z0+W
+};
+template <int W> __device__ inline Offsets<W> offsets(const Plan& p, int x, int y, int z0) {
+    using O = Off<W>;
+    Offsets<W> o;
+    const int64_t SX = int64_t(p.Y) * p.Z;
+    o.x0 = int64_t(x) * SX;
+    o.xm1 = x >= 1 ? o.x0 - SX : o.x0;
+    o.xp1 = x + 1 < p.X ? o.x0 + SX : o.x0;
+    const O uz = O(p.Z);
+    o.o0 = O(y) * uz + O(z0);
+    o.ym1 = y >= 1 ? o.o0 - uz : o.o0;
+    o.yp1 = y + 1 < p.Y ? o.o0 + uz : o.o0;
+    o.zm1 = z0 >= 1 ? o.o0 - 1 : o.o0;
+    const O last = o.o0 + O(W - 1);
+    o.zp1 = z0 + W < p.Z ? last + 1 : last;
+    return o;
+}
+
+// The values of a field that a seven-point stencil of W cells reads; r holds
+// the row with one cell on each side (r[j] is cell z0 - 1 + j).
+template <class T, int W> struct Star7 {
+    T xm[W], xp[W], ym[W], yp[W], r[W + 2];
+    __device__ T c(int i) const { return r[i + 1]; }
+};
+template <class T, int W> __device__ inline Star7<T, W> load7(const T* __restrict__ f, const Offsets<W>& o) {
+    Star7<T, W> s;
+    T c[W];
+    const T* const f0 = f + o.x0;
+    load<T, W>(f0, o.o0, c);
+    load<T, W>(f + o.xm1, o.o0, s.xm);
+    load<T, W>(f + o.xp1, o.o0, s.xp);
+    load<T, W>(f0, o.ym1, s.ym);
+    load<T, W>(f0, o.yp1, s.yp);
+    s.r[0] = load1(f0, o.zm1);
+    s.r[W + 1] = load1(f0, o.zp1);
+#pragma unroll
+    for (int i = 0; i < W; ++i) s.r[i + 1] = c[i];
+    return s;
+}
+
+// Geometry of a thread's cells on an axis-aligned lattice (LatticeGeo).
+template <class T, int W> struct LatticeCells {
+    T wx, wy, wz[W];
+    T V[W];
+    T ax[2], ay[2], az[W + 1];  // alpha_d of the lower and upper faces (az: of the W + 1 z-faces)
+    __device__ T area(int a, int i) const { return a == 0 ? wy * wz[i] : a == 1 ? wx * wz[i] : wx * wy; }
+};
+template <class T, int W, bool ALPHA>
+__device__ inline LatticeCells<T, W> load_lattice(const LatticeGeo<T>& g, const Offsets<W>& o, int x, int y, int z0) {
+    LatticeCells<T, W> c;
+    load<T, W>(g.vol + o.x0, o.o0, c.V);
+    c.wx = g.w[0][x];
+    c.wy = g.w[1][y];
+    load<T, W>(g.w[2], Off<W>(z0), c.wz);
+    if constexpr (ALPHA) {
+        T lo[W];
+        c.ax[0] = g.alpha[0][x];
+        c.ax[1] = g.alpha[0][x + 1];
+        c.ay[0] = g.alpha[1][y];
+        c.ay[1] = g.alpha[1][y + 1];
+        load<T, W>(g.alpha[2], Off<W>(z0), lo);
+#pragma unroll
+        for (int i = 0; i < W; ++i) c.az[i] = lo[i];
+        c.az[W] = g.alpha[2][z0 + W];
+    }
+    return c;
+}
+
+// Six face values of a cell, lower and upper per axis
+template <class T> struct Faces {
+    T lo[3], hi[3];
+};
+
+// f * 0, which is not 0 where f is infinite or NaN
+template <class T> __device__ inline T zero_of(T lo, T hi) {
+    if constexpr (sizeof(T) == 4) return __builtin_fmaf(hi, T(0), lo * T(0));
+    else return __builtin_fma(hi, T(0), lo * T(0));
+}
+
+// Gauss sum of component a on a lattice, outward (the gradient's) or axis
+// normals (the Laplacian's).  The reference sums all six faces, the other
+// axes' with a zero normal component: they add nothing to a finite sum and
+// make it NaN where a face value is not finite.
+template <class T, int W, bool OUTWARD>
+__device__ inline T lattice_gauss(const LatticeCells<T, W>& c, const Faces<T>& f, int a, int i) {
+    const int b = a == 0 ? 1 : 0, d = a == 2 ? 1 : 2;
+    const T A = c.area(a, i);
+    const T zeros = zero_of(f.lo[b], f.hi[b]) + zero_of(f.lo[d], f.hi[d]);
+    T acc = T(0) + (OUTWARD ? -f.lo[a] : f.lo[a]) * A;
+    acc = acc + f.hi[a] * A;
+    acc = acc + zeros;
+    return acc / c.V[i];
 }
 
 }  // namespace star

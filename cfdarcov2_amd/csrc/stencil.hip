@@ -1,8 +1,10 @@
 // Stencil kernels of the explicit finite-volume step on the structured hex
 // mesh: Green-Gauss gradient, Laplacian, stabilisation, and the fused heat and
-// acoustic steps.  Two geometry forms:
+// acoustic steps.  Three geometry forms:
 //   uniform  - exactly uniform meshes; geometry is a handful of constants and
 //              neighbours are implicit, so only state crosses HBM;
+//   lattice  - axis-aligned faces (any spacing): widths and alpha_d per cell
+//              layer, volume per cell (ops_star.hip);
 //   general  - per-face SoA geometry (face families z, y, x) for perturbed
 //              meshes; neighbours are still implicit (structured topology).
 // All arithmetic follows the reference operation order (see the oracle and
@@ -93,47 +95,9 @@ template <class T> __device__ inline T gg_pair_u(const UniformGeo<T>& g, T f_lo,
 template <class T> __device__ inline T lin(T c, T nb) { return (c + nb) * T(0.5); }
 
 // ---------------------------------------------------------------------------
-// GradVar / Grad2Var / StabVar operator kernels
+// GradVar / Grad2Var / StabVar operator kernels (the gradient and Laplacian of
+// uniform meshes and axis-aligned lattices: ops_star.hip)
 // ---------------------------------------------------------------------------
-
-template <class T>
-__global__ void __launch_bounds__(256) grad_uniform_k(UniformGeo<T> g, const T* __restrict__ phi,
-                                                      T* __restrict__ out, int mask, int wall_axis) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = phi[c.id];
-    T res = T(0);
-    for (int a = 0; a < 3; ++a) {
-        if (!(mask & (1 << a))) continue;
-        T f_lo = lin(pc, phi[nb_lo(g, c, a)]);
-        T f_hi = lin(pc, phi[nb_hi(g, c, a)]);
-        if (wall_axis == a) {
-            if (at_lo(g, c, a)) f_lo = T(0);
-            if (at_hi(g, c, a)) f_hi = T(0);
-        }
-        res = res + gg_pair_u(g, f_lo, f_hi, g.area[a]);
-    }
-    out[c.id] = res;
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) lapl_uniform_k(UniformGeo<T> g, const T* __restrict__ phi,
-                                                      T* __restrict__ out, int mask) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = phi[c.id];
-    T res = T(0);
-    for (int a = 0; a < 3; ++a) {
-        if (!(mask & (1 << a))) continue;
-        const T al_lo = at_lo(g, c, a) ? g.alpha_b[a] : g.alpha[a];
-        const T al_hi = at_hi(g, c, a) ? g.alpha_b[a] : g.alpha[a];
-        const T s_lo = (-pc + phi[nb_lo(g, c, a)]) * al_lo;
-        const T s_hi = (-pc + phi[nb_hi(g, c, a)]) * al_hi;
-        // axis normals are +1 on both faces of the pair
-        res = res + udiv(g, s_lo * g.area[a] + s_hi * g.area[a]);
-    }
-    out[c.id] = res;
-}
 
 // One axis d of StabVar on a uniform mesh (src/fvm3d.cpp:909-936), added to
 // res.  Second stage: upwind face values phi + (len * g_d) * n_out_d, jump
@@ -371,35 +335,6 @@ __global__ void __launch_bounds__(256) stab_general_k(GeneralGeo<T> g, const T* 
 // Fused heat step: T' = dt * (alpha * lapl(T)) + T   (DtVar::extract order,
 // src/fvm3d.cpp:690-692, with lapl = ((0 + L_x) + L_y) + L_z).
 // ---------------------------------------------------------------------------
-template <class T, bool PW>
-__device__ inline void heat_uniform_cell(const UniformGeo<T>& g, const T* __restrict__ Tin, T* __restrict__ Tout,
-                                         T alpha, const T* __restrict__ alpha_f, T dt) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = Tin[c.id];
-    T L = T(0);
-    for (int a = 0; a < 3; ++a) {
-        const T al_lo = at_lo(g, c, a) ? g.alpha_b[a] : g.alpha[a];
-        const T al_hi = at_hi(g, c, a) ? g.alpha_b[a] : g.alpha[a];
-        const T s_lo = (-pc + Tin[nb_lo(g, c, a)]) * al_lo;
-        const T s_hi = (-pc + Tin[nb_hi(g, c, a)]) * al_hi;
-        const T num = s_lo * g.area[a] + s_hi * g.area[a];
-        // a power-of-two volume divides exactly, so the product is the same number
-        if constexpr (PW) L = L + num * g.inv_vol;
-        else L = L + num / g.vol;
-    }
-    const T k = alpha_f ? alpha_f[c.id] : alpha;
-    Tout[c.id] = dt * (k * L) + pc;
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) heat_uniform_k(UniformGeo<T> g, const T* __restrict__ Tin,
-                                                      T* __restrict__ Tout, T alpha, const T* __restrict__ alpha_f,
-                                                      T dt) {
-    if (g.vol_pow2) heat_uniform_cell<T, true>(g, Tin, Tout, alpha, alpha_f, dt);
-    else heat_uniform_cell<T, false>(g, Tin, Tout, alpha, alpha_f, dt);
-}
-
 template <class T>
 __global__ void __launch_bounds__(256) heat_general_k(GeneralGeo<T> g, const T* __restrict__ Tin,
                                                       T* __restrict__ Tout, T alpha, const T* __restrict__ alpha_f,
@@ -484,9 +419,8 @@ template <> const GeneralGeo<double>& ggeo<double>(const cfd_mesh_s* m) { return
 inline void check_launch() { CFD_HIP(hipGetLastError()); }
 
 template <class T> void launch_grad(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s) {
-    if (m->uniform) {
-        const auto& g = ugeo<T>(m);
-        grad_uniform_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, (T*)out, mask, wall);
+    if (m->uniform || m->lattice) {
+        launch_grad_star<T>(m, phi, out, mask, wall, s);
     } else {
         const auto& g = ggeo<T>(m);
         grad_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, (T*)out, mask, wall);
@@ -495,9 +429,8 @@ template <class T> void launch_grad(const cfd_mesh_s* m, const void* phi, void* 
 }
 
 template <class T> void launch_lapl(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s) {
-    if (m->uniform) {
-        const auto& g = ugeo<T>(m);
-        lapl_uniform_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, (T*)out, mask);
+    if (m->uniform || m->lattice) {
+        launch_lapl_star<T>(m, phi, out, mask, s);
     } else {
         const auto& g = ggeo<T>(m);
         lapl_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, (T*)out, mask);
@@ -571,9 +504,8 @@ void launch_heat(const cfd_mesh_s* m, void* Ta, void* Tb, double alpha, const vo
     for (int64_t k = k0; k < nsteps; ++k) {
         const T* in = (const T*)((k & 1) ? Tb : Ta);
         T* out = (T*)((k & 1) ? Ta : Tb);
-        if (m->uniform) {
-            const auto& g = ugeo<T>(m);
-            heat_uniform_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, in, out, T(alpha), (const T*)af, T(dt));
+        if (m->uniform || m->lattice) {
+            launch_heat_star<T>(m, in, out, alpha, af, dt, s);
         } else {
             const auto& g = ggeo<T>(m);
             heat_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, in, out, T(alpha), (const T*)af, T(dt));
@@ -590,6 +522,10 @@ void launch_wave(const cfd_mesh_s* m, void* const a[4], void* const b[4], double
         for (int64_t k = 0; k < nsteps; ++k) {
             void* const* in = (k & 1) ? b : a;
             void* const* out = (k & 1) ? a : b;
+            if (m->lattice) {
+                launch_wave_lattice<T>(m, in, out, K, Kf, dt, s);
+                continue;
+            }
             wave_vel_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(
                 g, (const T*)in[0], (const T*)in[1], (const T*)in[2], (const T*)in[3], (T*)out[1], (T*)out[2],
                 (T*)out[3], T(dt));
@@ -607,7 +543,7 @@ void launch_wave(const cfd_mesh_s* m, void* const a[4], void* const b[4], double
 // ---------------------------------------------------------------------------
 // Adjoint of the heat step on uniform meshes (no reference counterpart).
 // The step is H = I + dt K L, K = diag(k) with k the constant alpha or the
-// alpha field, L the Laplacian of heat_uniform_cell.  On a uniform mesh L is
+// alpha field, L the Laplacian of heat_star_k.  On a uniform mesh L is
 // symmetric (an interior face couples its two cells with the same
 // alpha_d A / V, a wall face couples nothing), so H^T = I + dt L K:
 //   constant alpha:  H^T = H, the forward kernels themselves;
@@ -616,7 +552,7 @@ void launch_wave(const cfd_mesh_s* m, void* const a[4], void* const b[4], double
 // the forward states T_{t-1} recomputed from checkpoints.
 // ---------------------------------------------------------------------------
 
-// L(k o f) at cell c (L(f) when kf is null), heat_uniform_cell's operation
+// L(k o f) at cell c (L(f) when kf is null), heat_star_k's operation
 // order; on a wall the neighbour is the cell itself and its term is zero
 template <class T, bool PW>
 __device__ inline T lapl_scaled(const UniformGeo<T>& g, const Cell& c, const T* __restrict__ f,

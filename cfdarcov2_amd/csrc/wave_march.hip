@@ -86,7 +86,7 @@ void launch_wave_march(const cfd_mesh_s* m, void* const a[4], void* const b[4], 
         void* const* in = (k & 1) ? b : a;
         void* const* out = (k & 1) ? a : b;
         if (variant == 0) {
-            if (!launch_wave_star<T>(g, in, out, K, Kf, dt, s)) launch_one<T, 4, 1>(g, in, out, K, Kf, dt, L, 0, s);
+            launch_wave_star<T>(g, in, out, K, Kf, dt, s);
             continue;
         }
         if (variant >= 7) {  // row form; misaligned fields take the 4-row march tile

@@ -41,3 +41,91 @@ def test_wave_star(hip_ctx, oracle_lib, n, shift, dtype):
         for name, g, r in zip("puvw", got, ref):
             assert np.array_equal(g.cpu().numpy(), r), f"field {name}, K field {kf is not None}"
     gm.close()
+
+
+def _mesh(hip_ctx, oracle_lib, n, kind, dtype):
+    """(star mesh, the same mesh in general form, oracle) of a uniform, decimal or graded lattice."""
+    from cfdarcov2_amd import capi
+    off, d = None, (0.125, 0.25, 0.5) if kind == "dyadic" else (0.1, 0.3, 0.7)
+    if kind == "graded":  # vertex layers moved along their own axis
+        g = np.meshgrid(*[0.05 * s * (np.arange(k + 1) % 3) for k, s in zip(n, d)], indexing="ij")
+        off = np.stack([a.ravel() for a in g], axis=1)
+    gm = capi.HexMesh(hip_ctx, *n, *d, dtype=dtype, vertex_offsets=off)
+    gg = capi.HexMesh(hip_ctx, *n, *d, dtype=dtype, vertex_offsets=off, force_general=True)
+    assert gg.info().uniform == 0
+    if kind == "dyadic":
+        assert gm.info().uniform == 1
+    elif min(n) > 3:  # (one or two layers can be exactly uniform) the lattice's tables are there
+        assert gm.info().uniform == 0 and gm.info().device_bytes > gg.info().device_bytes
+    return gm, gg, oracle_lib.OracleMesh(*n, *d, dtype=dtype, perturb=off)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["dyadic", "decimal", "graded"])
+@pytest.mark.parametrize("n", EXTENTS, ids=lambda n: "x".join(map(str, n)))
+def test_operators_and_heat_star(hip_ctx, oracle_lib, n, kind, dtype):
+    gm, gg, om = _mesh(hip_ctx, oracle_lib, n, kind, dtype)
+    rng = np.random.default_rng(5)
+    phi = rng.standard_normal(om.N).astype(dtype)
+    af = (1e-3 * (1 + rng.random(om.N))).astype(dtype)
+    for shift in (0, 1):
+        t, out = _view(phi, dtype, shift), _view(phi, dtype, shift)
+        for mask in (1, 2, 4, 7, 0):
+            for wall in (-1, 0, 1, 2):
+                assert np.array_equal(gm.grad(t, mask, wall, out=out).cpu().numpy(), om.grad(phi, mask, wall)), (mask, wall)
+            assert np.array_equal(gm.lapl(t, mask, out=out).cpu().numpy(), om.lapl(phi, mask)), mask
+        for a in (None, af):
+            A, B = _view(phi, dtype, shift), _view(phi, dtype, shift)
+            got = gm.heat_run(A, B, 2e-3, 0.5, 5, alpha_field=None if a is None else _view(a, dtype, shift))
+            assert np.array_equal(got.cpu().numpy(), om.heat_run(phi, 2e-3, 0.5, 5, alpha_field=a)), a is None
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["decimal", "graded"])
+@pytest.mark.parametrize("n", EXTENTS, ids=lambda n: "x".join(map(str, n)))
+def test_lattice_equals_general_form(hip_ctx, oracle_lib, n, kind, dtype):
+    """Every operator and step on a lattice against the general form of the
+    same mesh, with infinities, NaN and values near the ends of the range
+    among the cells: the same bits, NaN in the same places."""
+    gm, gg, om = _mesh(hip_ctx, oracle_lib, n, kind, dtype)
+    if gm.info().uniform:
+        pytest.skip("one or two layers per axis: exactly uniform, no lattice tables")
+    rng = np.random.default_rng(6)
+    tiny, big = np.finfo(dtype).smallest_subnormal, np.finfo(dtype).max
+    fields = []
+    for special in (None, (np.inf, np.nan, big, -big, tiny, -0.0)):
+        f = [rng.standard_normal(om.N).astype(dtype) for _ in range(4)]
+        if special:
+            for a in f:
+                a[rng.integers(om.N, size=max(1, om.N // 40))] = rng.choice(special)
+        fields.append(f)
+    K = (-(0.5 + rng.random(om.N))).astype(dtype)
+
+    def same(a, b):
+        return np.array_equal(a.cpu().numpy(), b.cpu().numpy(), equal_nan=True)
+
+    for f in fields:
+        t = _view(f[0], dtype, 0)
+        for mask in (1, 6, 7):
+            assert same(gm.grad(t, mask, -1), gg.grad(t, mask, -1)) and same(gm.grad(t, mask, 2), gg.grad(t, mask, 2))
+            assert same(gm.lapl(t, mask), gg.lapl(t, mask))
+            assert same(gm.stab(t, mask), gg.stab(t, mask))
+        for m in (3, 4):
+            x = [_view(f[0], dtype, 0) for _ in range(4)]
+            assert same(gm.heat_run(x[0], x[1], 2e-3, 0.5, m), gg.heat_run(x[2], x[3], 2e-3, 0.5, m))
+        for kf in (None, _view(K, dtype, 0)):
+            A, C = [[_view(a, dtype, 0) for a in f] for _ in range(2)]
+            B, D = [[torch.empty_like(a) for a in A] for _ in range(2)]
+            for g, r in zip(gm.wave_run(A, B, -1.0, 0.02, 3, K_field=kf), gg.wave_run(C, D, -1.0, 0.02, 3, K_field=kf)):
+                assert same(g, r)
+
+
+def test_perturbed_mesh_is_no_lattice(hip_ctx):
+    """One vertex moved by one unit in the last place: the general form."""
+    from cfdarcov2_amd import capi
+    n, d = (5, 4, 6), (0.1, 0.3, 0.7)
+    off = np.zeros(((n[0] + 1) * (n[1] + 1) * (n[2] + 1), 3))
+    off[2 * 5 * 7 + 2 * 7 + 3, 1] = 2.0 ** -40
+    gm = capi.HexMesh(hip_ctx, *n, *d, dtype="f64", vertex_offsets=off)
+    gg = capi.HexMesh(hip_ctx, *n, *d, dtype="f64", vertex_offsets=off, force_general=True)
+    assert gm.info().device_bytes == gg.info().device_bytes
