@@ -10,8 +10,8 @@
 // Both run the row tile of the fused step (row.hpp): one wave per z row, four
 // cells per lane, TY output waves and two halo waves per workgroup marching x
 // over L planes.  MODE 1 is the fused step's arithmetic, so it equals the
-// oracle bit for bit; MODES 2 and 3 are the per-thread transposed kernel's
-// (adjoint.hip) operation for operation, so the two forms agree bit for bit.
+// oracle bit for bit; MODES 2 and 3 are the star form's
+// (adj_star.hip) operation for operation, so the two forms agree bit for bit.
 #include <hip/hip_runtime.h>
 
 #include <vector>
@@ -109,11 +109,18 @@ bool aligned4(const void* p, size_t elem) { return (reinterpret_cast<uintptr_t>(
 // Output rows of the row tile for `m`'s adjoint shape
 template <class T> int adj_row_tile_rows(const cfd_mesh_s* m) { return m->adj_ty; }
 
-// Whether the row form takes this mesh and these fields (16-byte aligned rows
-// in FP32, 32-byte in FP64).
+// Whether a run takes the row form: it was set, or no form was set and both
+// states (8 fields) exceed the last-level cache (without the K gradient) or
+// half of it (with it: the recomputed segment's fields want room too), and the
+// fields are aligned (16-byte rows in FP32, 32-byte in FP64).  Measured
+// us/step, star / row form (4 rows, 8 planes): transposed step 128^3 FP32
+// 15.7 / 17.0, 160^3 FP64 51.8 / 67.7, 192^3 FP64 135 / 101; with the K
+// gradient 160^3 FP32 72.9 / 83.0, 128^3 FP64 73.4 / 70.0, 192^3 FP32 137 / 125.
 template <class T>
-bool adj_row_usable(const cfd_mesh_s* m, const void* const* fields, int n) {
-    if (m->adj_form != 1 || !m->uniform || !wave_row_supported(m->Z)) return false;
+bool adj_row_usable(const cfd_mesh_s* m, const void* const* fields, int n, bool grad_K) {
+    if (!m->uniform || !wave_row_supported(m->Z)) return false;
+    const int64_t room = grad_K ? kLastLevelCacheBytes / 2 - 1 : kLastLevelCacheBytes;
+    if (m->adj_form == 0 || (m->adj_form < 0 && 8 * m->N * int64_t(sizeof(T)) <= room)) return false;
     for (int i = 0; i < n; ++i)
         if (fields[i] && !aligned4(fields[i], sizeof(T))) return false;
     return true;
@@ -158,7 +165,7 @@ void launch_wave_row_aux(const cfd_mesh_s* m, int mode, const void* const in[4],
 }
 
 #define CFD_AUX_INSTANTIATE(T)                                                                                   \
-    template bool adj_row_usable<T>(const cfd_mesh_s*, const void* const*, int);                                \
+    template bool adj_row_usable<T>(const cfd_mesh_s*, const void* const*, int, bool);                          \
     template std::vector<uint64_t> adj_row_tile_sensors<T>(const cfd_mesh_s*, const SensorList&);              \
     template void launch_wave_row_aux<T>(const cfd_mesh_s*, int, const void* const[4], void* const[4], double,  \
                                          const void*, double, const SensorList*, const row::RowAux<T>&, int,     \

@@ -19,9 +19,7 @@
 //
 // Sensor traces: the forward kernel writes p' at up to 64 sensor cells, the
 // adjoint kernel adds the trace gradients of the previous step to nu_p there.
-// The sensor list is a kernel argument; each wave tests it against its own row
-// of 64 z-cells with scalar instructions, so cells without sensors pay nothing
-// but that scan.
+// Kernels: adj_star.hip (form 0) and adj_row.hip (form 1).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,11 +29,19 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "row.hpp"
+#include "star_wave.hpp"
 
 namespace cfd {
 
+// star form (adj_star.hip)
+star::SensorSet sensor_set(const cfd_mesh_s* m, const SensorList& l);
+template <class T>
+void launch_wave_star_aux(const cfd_mesh_s* m, int mode, const void* const in[4], void* const out[4], double K,
+                          const void* Kf, double dt, const star::SensorSet& sens, const star::WaveAux<T>& aux,
+                          hipStream_t s);
+
 // row form (adj_row.hip)
-template <class T> bool adj_row_usable(const cfd_mesh_s* m, const void* const* fields, int n);
+template <class T> bool adj_row_usable(const cfd_mesh_s* m, const void* const* fields, int n, bool grad_K);
 template <class T>
 void launch_wave_row_aux(const cfd_mesh_s* m, int mode, const void* const in[4], void* const out[4], double K,
                          const void* Kf, double dt, const SensorList* sens, const row::RowAux<T>& aux, int rev,
@@ -71,161 +77,6 @@ template <class T> static DevSensors upload_sensors(const cfd_mesh_s* m, const S
     return d;
 }
 
-namespace {
-
-template <class T> __device__ inline T a_lin(T c, T nb) { return (c + nb) * T(0.5); }
-// Green-Gauss face pair ((-f_lo) A + f_hi A) / V; with PW the volume is an
-// exact power of two and the division is the (bit-identical) product with 1/V.
-template <bool PW, class T> __device__ inline T a_pair(T f_lo, T f_hi, T A, const UniformGeo<T>& g) {
-    const T t_lo = (-f_lo) * A;
-    const T t_hi = f_hi * A;
-    if constexpr (PW) return (t_lo + t_hi) * g.inv_vol;
-    else return (t_lo + t_hi) / g.vol;
-}
-
-struct TCell {
-    int64_t x, y, z, id;
-    bool valid;
-};
-
-template <class T> __device__ inline TCell tcell(const UniformGeo<T>& g) {
-    TCell c;
-    c.z = int64_t(blockIdx.x) * 64 + threadIdx.x;
-    c.y = int64_t(blockIdx.y) * 4 + threadIdx.y;
-    c.x = blockIdx.z;
-    c.valid = c.z < g.Z && c.y < g.Y;
-    c.id = (c.x * g.Y + c.y) * g.Z + c.z;
-    return c;
-}
-
-// Sensor j of the wave holding this thread's row, or -1.  `row` and `z0` are
-// wave-uniform; the loop runs on the scalar unit.
-__device__ inline int sensor_of(const SensorList& s, int row, int z0, int z) {
-    int hit = -1;
-    for (int j = 0; j < s.n; ++j) {
-        if (s.row[j] == row && s.z[j] >= z0 && s.z[j] < z0 + 64) {
-            if (s.z[j] == z) hit = j;
-        }
-    }
-    return hit;
-}
-
-__device__ inline int wave_row(int64_t x, int64_t Y) {
-    return __builtin_amdgcn_readfirstlane(int(x * Y) + int(blockIdx.y) * 4 + int(threadIdx.y));
-}
-
-// velocity update of cell j along axis a from p (reference boundary rule)
-template <bool PW, class T>
-__device__ inline T fwd_vel(const UniformGeo<T>& g, const T* __restrict__ p, const T* __restrict__ q, int64_t j,
-                            int64_t stride, bool lo, bool hi, int a, T dt) {
-    const T pc = p[j];
-    const T pl = lo ? pc : p[j - stride];
-    const T ph = hi ? pc : p[j + stride];
-    const T G = a_pair<PW>(a_lin(pc, pl), a_lin(pc, ph), g.area[a], g);
-    return dt * (-G) + q[j];
-}
-
-}  // namespace
-
-// Forward step with optional sensor recording: bitwise the same arithmetic as
-// the per-thread fused acoustic kernel.
-template <class T, bool PW>
-__global__ void __launch_bounds__(256) wave_trace_k(UniformGeo<T> g, const T* __restrict__ p,
-                                                    const T* __restrict__ u, const T* __restrict__ v,
-                                                    const T* __restrict__ w, T* __restrict__ po,
-                                                    T* __restrict__ uo, T* __restrict__ vo, T* __restrict__ wo, T K,
-                                                    const T* __restrict__ Kf, T dt, SensorList sens,
-                                                    T* __restrict__ trace) {
-    const TCell c = tcell(g);
-    const int row = wave_row(c.x, g.Y);
-    if (!c.valid) return;
-    const T* vel[3] = {u, v, w};
-    T* velo[3] = {uo, vo, wo};
-    const int64_t crd[3] = {c.x, c.y, c.z};
-    const int64_t ext[3] = {g.X, g.Y, g.Z};
-    const int64_t str[3] = {g.Y * g.Z, g.Z, 1};
-    T S = T(0);
-    for (int a = 0; a < 3; ++a) {
-        const bool lo = crd[a] == 0, hi = crd[a] == ext[a] - 1;
-        const T qc = fwd_vel<PW>(g, p, vel[a], c.id, str[a], lo, hi, a, dt);
-        velo[a][c.id] = qc;
-        T f_lo = T(0), f_hi = T(0);
-        if (!lo) f_lo = a_lin(qc, fwd_vel<PW>(g, p, vel[a], c.id - str[a], str[a], crd[a] - 1 == 0, false, a, dt));
-        if (!hi) f_hi = a_lin(qc, fwd_vel<PW>(g, p, vel[a], c.id + str[a], str[a], false, crd[a] + 1 == ext[a] - 1, a, dt));
-        const T G = a_pair<PW>(f_lo, f_hi, g.area[a], g);
-        S = (a == 0) ? G : S + G;
-    }
-    const T k = Kf ? Kf[c.id] : K;
-    const T pn = dt * (k * S) + p[c.id];
-    po[c.id] = pn;
-    if (trace) {
-        const int j = sensor_of(sens, row, int(blockIdx.x) * 64, int(c.z));
-        if (j >= 0) trace[j] = pn;
-    }
-}
-
-// adjoint velocity of cell j along axis a: mu = lam_a - G_a(q), q = (dt k) lam_p
-template <bool PW, class T>
-__device__ inline T adj_vel(const UniformGeo<T>& g, const T* __restrict__ lp, const T* __restrict__ la, T K,
-                            const T* __restrict__ Kf, int64_t j, int64_t stride, bool lo, bool hi, int a, T dt) {
-    auto q = [&](int64_t i) { return (dt * (Kf ? Kf[i] : K)) * lp[i]; };
-    const T qc = q(j);
-    const T ql = lo ? qc : q(j - stride);
-    const T qh = hi ? qc : q(j + stride);
-    const T G = a_pair<PW>(a_lin(qc, ql), a_lin(qc, qh), g.area[a], g);
-    return la[j] - G;
-}
-
-// One transposed step lam_t -> lam_{t-1}.  src (nullable): trace gradients of
-// step t-1, added at the sensors.  vel_t/gK (nullable): the forward
-// velocities of step t and the K-gradient accumulator.
-template <class T, bool PW>
-__global__ void __launch_bounds__(256) wave_adj_k(UniformGeo<T> g, const T* __restrict__ lp,
-                                                  const T* __restrict__ lu, const T* __restrict__ lv,
-                                                  const T* __restrict__ lw, T* __restrict__ op,
-                                                  T* __restrict__ ou, T* __restrict__ ov, T* __restrict__ ow, T K,
-                                                  const T* __restrict__ Kf, T dt, SensorList sens,
-                                                  const T* __restrict__ src, const T* __restrict__ ut,
-                                                  const T* __restrict__ vt, const T* __restrict__ wt,
-                                                  T* __restrict__ gK) {
-    const TCell c = tcell(g);
-    const int row = wave_row(c.x, g.Y);
-    if (!c.valid) return;
-    const T* lam[3] = {lu, lv, lw};
-    T* outv[3] = {ou, ov, ow};
-    const T* velt[3] = {ut, vt, wt};
-    const int64_t crd[3] = {c.x, c.y, c.z};
-    const int64_t ext[3] = {g.X, g.Y, g.Z};
-    const int64_t str[3] = {g.Y * g.Z, g.Z, 1};
-    T S = T(0), St = T(0);
-    for (int a = 0; a < 3; ++a) {
-        const bool lo = crd[a] == 0, hi = crd[a] == ext[a] - 1;
-        const T mc = adj_vel<PW>(g, lp, lam[a], K, Kf, c.id, str[a], lo, hi, a, dt);
-        outv[a][c.id] = mc;
-        T f_lo = T(0), f_hi = T(0);
-        if (!lo) f_lo = a_lin(mc, adj_vel<PW>(g, lp, lam[a], K, Kf, c.id - str[a], str[a], crd[a] - 1 == 0, false, a, dt));
-        if (!hi)
-            f_hi = a_lin(mc, adj_vel<PW>(g, lp, lam[a], K, Kf, c.id + str[a], str[a], false, crd[a] + 1 == ext[a] - 1, a, dt));
-        const T G = a_pair<PW>(f_lo, f_hi, g.area[a], g);
-        S = (a == 0) ? G : S + G;
-        if (gK) {  // forward divergence of step t, as the forward computes it
-            const T vc = velt[a][c.id];
-            const T tl = lo ? T(0) : a_lin(vc, velt[a][c.id - str[a]]);
-            const T th = hi ? T(0) : a_lin(vc, velt[a][c.id + str[a]]);
-            const T Gt = a_pair<PW>(tl, th, g.area[a], g);
-            St = (a == 0) ? Gt : St + Gt;
-        }
-    }
-    const T lpc = lp[c.id];
-    if (gK) gK[c.id] = gK[c.id] + (lpc * dt) * St;
-    T np = dt * S + lpc;
-    if (src) {
-        const int j = sensor_of(sens, row, int(blockIdx.x) * 64, int(c.z));
-        if (j >= 0) np = np + src[j];
-    }
-    op[c.id] = np;
-}
-
 // lam_p[sensor j] += src[j]
 template <class T> __global__ void scatter_add_k(T* __restrict__ lp, SensorList sens, const T* __restrict__ src) {
     const int j = threadIdx.x;
@@ -234,16 +85,6 @@ template <class T> __global__ void scatter_add_k(T* __restrict__ lp, SensorList 
         lp[cell] = lp[cell] + src[j];
     }
 }
-
-namespace {
-const dim3 kBlk(64, 4, 1);
-template <class T> dim3 tgrid(const UniformGeo<T>& g) {
-    return dim3(unsigned((g.Z + 63) / 64), unsigned((g.Y + 3) / 4), unsigned(g.X));
-}
-template <class T> const UniformGeo<T>& ug(const cfd_mesh_s* m) {
-    if constexpr (sizeof(T) == 4) return m->ug32; else return m->ug64;
-}
-}  // namespace
 
 SensorList make_sensors(const cfd_mesh_s* m, const int64_t* cells, int n) {
     CFD_REQUIRE(n >= 0 && n <= kMaxSensors, "sensor count must be in [0, 64]");
@@ -261,30 +102,6 @@ SensorList make_sensors(const cfd_mesh_s* m, const int64_t* cells, int n) {
         s.z[j] = int(cells[j] % m->Z);
     }
     return s;
-}
-
-template <class T>
-void launch_wave_trace_step(const cfd_mesh_s* m, const void* const in[4], void* const out[4], double K,
-                            const void* Kf, double dt, const SensorList& sens, void* trace, hipStream_t s) {
-    const UniformGeo<T>& g = ug<T>(m);
-    auto* kern = g.vol_pow2 ? wave_trace_k<T, true> : wave_trace_k<T, false>;
-    kern<<<tgrid(g), kBlk, 0, s>>>(g, (const T*)in[0], (const T*)in[1], (const T*)in[2], (const T*)in[3],
-                                   (T*)out[0], (T*)out[1], (T*)out[2], (T*)out[3], T(K), (const T*)Kf, T(dt), sens,
-                                   (T*)trace);
-}
-
-template <class T>
-void launch_wave_adj_step(const cfd_mesh_s* m, const void* const in[4], void* const out[4], double K,
-                          const void* Kf, double dt, const SensorList& sens, const void* src,
-                          const void* const velt[3], void* gK, hipStream_t s) {
-    const UniformGeo<T>& g = ug<T>(m);
-    const T* vt[3] = {nullptr, nullptr, nullptr};
-    if (gK)
-        for (int a = 0; a < 3; ++a) vt[a] = (const T*)velt[a];
-    auto* kern = g.vol_pow2 ? wave_adj_k<T, true> : wave_adj_k<T, false>;
-    kern<<<tgrid(g), kBlk, 0, s>>>(g, (const T*)in[0], (const T*)in[1], (const T*)in[2], (const T*)in[3],
-                                   (T*)out[0], (T*)out[1], (T*)out[2], (T*)out[3], T(K), (const T*)Kf, T(dt), sens,
-                                   (const T*)src, vt[0], vt[1], vt[2], (T*)gK);
 }
 
 template <class T> void launch_scatter_add(void* lp, const SensorList& sens, const void* src, hipStream_t s) {
@@ -305,10 +122,11 @@ void run_wave_traces(const cfd_mesh_s* m, void* const a[4], void* const b[4], do
                      hipStream_t s) {
     const size_t field = size_t(m->N) * sizeof(T);
     const void* fields[9] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3], Kf};
-    const bool rowf = adj_row_usable<T>(m, fields, 9);
+    const bool rowf = adj_row_usable<T>(m, fields, 9, false);
     auto trace_row = [&](int64_t t) -> T* { return traces ? (T*)traces + t * sens.n : nullptr; };
     const DevSensors ds = rowf ? upload_sensors<T>(m, sens, s) : DevSensors{};
     const SensorList* dsens = ds.list;
+    const star::SensorSet set = rowf ? star::SensorSet{} : sensor_set(m, sens);
     try {
         for (int64_t t = 0; t < nsteps; ++t) {
             void* const* in = (t & 1) ? b : a;
@@ -323,7 +141,8 @@ void run_wave_traces(const cfd_mesh_s* m, void* const a[4], void* const b[4], do
                 const row::RowAux<T> aux{T(0), tr, nullptr, nullptr, nullptr, nullptr, ds.tiles};
                 launch_wave_row_aux<T>(m, 1, (const void* const*)in, out, K, Kf, dt, dsens, aux, int(t & 1), s);
             } else {
-                launch_wave_trace_step<T>(m, (const void* const*)in, out, K, Kf, dt, sens, tr, s);
+                const star::WaveAux<T> aux{tr, nullptr, 1, nullptr, nullptr, nullptr};
+                launch_wave_star_aux<T>(m, 1, (const void* const*)in, out, K, Kf, dt, set, aux, s);
             }
         }
         CFD_HIP(hipGetLastError());
@@ -405,7 +224,7 @@ static void run_wave_adjoint_row(const cfd_mesh_s* m, void* const la[4], void* c
 // step's trace gradients); on return the adjoint of the initial state is in
 // adj_a when nsteps is even, adj_b when odd.  grad_K (nullable) accumulates
 // dL/dK per cell and needs the checkpoints: each segment of `every` steps is
-// recomputed from its checkpoint, keeping the segment's velocities.
+// recomputed from its checkpoint.
 template <class T>
 void run_wave_adjoint(const cfd_mesh_s* m, void* const la[4], void* const lb[4], double K, const void* Kf,
                       double dt, int64_t nsteps, const SensorList& sens, const void* tgrad, const void* ckpt,
@@ -415,73 +234,68 @@ void run_wave_adjoint(const cfd_mesh_s* m, void* const la[4], void* const lb[4],
     if (tgrad && nsteps >= 1) launch_scatter_add<T>(la[0], sens, (const T*)tgrad + (nsteps - 1) * sens.n, s);
     {
         const void* fields[10] = {la[0], la[1], la[2], la[3], lb[0], lb[1], lb[2], lb[3], gK, ckpt};
-        if (!Kf && adj_row_usable<T>(m, fields, 10)) {
+        if (!Kf && adj_row_usable<T>(m, fields, 10, gK != nullptr)) {
             run_wave_adjoint_row<T>(m, la, lb, K, dt, nsteps, sens, tgrad, ckpt, every, gK, s);
             return;
         }
     }
-    void* ws = nullptr;       // recomputed velocities of one segment: every x 3 fields
-    void* pbuf = nullptr;     // recomputed pressures (ping-pong)
-    if (gK) {
-        ws = pool_alloc(m->ctx, int64_t(every) * 3 * int64_t(field), s);
-        pbuf = pool_alloc(m->ctx, 2 * int64_t(field), s);
-    }
+    // With grad_K each segment is recomputed forward, keeping every step's
+    // divergence S (one field per step); the state ping-pongs between two
+    // buffers and the segment's last step stores S alone.
+    const int states = every == 1 ? 0 : every == 2 ? 1 : 2;
+    void* ws = nullptr;  // S of each step of one segment
+    void* st = nullptr;  // recomputed states
+    const star::SensorSet set = sensor_set(m, sens);
     try {
+        if (gK) {
+            ws = pool_alloc(m->ctx, every * int64_t(field), s);
+            if (states) st = pool_alloc(m->ctx, states * 4 * int64_t(field), s);
+        }
         int64_t done = 0;
-        auto adj_step = [&](int64_t t, const void* const velt[3]) {
+        auto adj_step = [&](int64_t t, const void* s_in) {
             void* const* in = (done & 1) ? lb : la;
             void* const* out = (done & 1) ? la : lb;
-            const void* src = (tgrad && t >= 2) ? (const void*)((const T*)tgrad + (t - 2) * sens.n) : nullptr;
-            launch_wave_adj_step<T>(m, (const void* const*)in, out, K, Kf, dt, sens, src, velt, gK, s);
+            const T* src = (tgrad && t >= 2) ? (const T*)tgrad + (t - 2) * sens.n : nullptr;
+            const star::WaveAux<T> aux{nullptr, nullptr, 1, src, (const T*)s_in, (T*)gK};
+            launch_wave_star_aux<T>(m, 2, (const void* const*)in, out, K, Kf, dt, set, aux, s);
             ++done;
         };
         int64_t t = nsteps;
         while (t >= 1) {
             if (!gK) {
-                const void* none[3] = {nullptr, nullptr, nullptr};
-                adj_step(t, none);
+                adj_step(t, nullptr);
                 --t;
                 continue;
             }
             const int64_t seg = (t - 1) / every, t0 = seg * every, len = t - t0;
             const char* ck = (const char*)ckpt + size_t(seg) * 4 * field;
             for (int64_t k = 0; k < len; ++k) {  // state t0+k -> t0+k+1
+                const bool last = k + 1 == len;
                 const void* in[4];
                 void* out[4];
-                if (k == 0) {
-                    for (int f = 0; f < 4; ++f) in[f] = ck + f * field;
-                } else {
-                    in[0] = (char*)pbuf + size_t(k & 1) * field;
-                    for (int f = 0; f < 3; ++f) in[1 + f] = (char*)ws + (size_t(k - 1) * 3 + f) * field;
+                for (int f = 0; f < 4; ++f) {
+                    in[f] = k == 0 ? (const void*)(ck + f * field)
+                                   : (const void*)((char*)st + (size_t((k - 1) & 1) * 4 + f) * field);
+                    out[f] = last ? nullptr : (void*)((char*)st + (size_t(k & 1) * 4 + f) * field);
                 }
-                out[0] = (char*)pbuf + size_t((k + 1) & 1) * field;
-                for (int f = 0; f < 3; ++f) out[1 + f] = (char*)ws + (size_t(k) * 3 + f) * field;
-                launch_wave_trace_step<T>(m, in, out, K, Kf, dt, sens, nullptr, s);
+                const star::WaveAux<T> aux{nullptr, (T*)((char*)ws + size_t(k) * field), last ? 0 : 1,
+                                           nullptr, nullptr, nullptr};
+                launch_wave_star_aux<T>(m, 1, in, out, K, Kf, dt, set, aux, s);
             }
-            for (int64_t tt = t; tt > t0; --tt) {
-                const int64_t k = tt - t0 - 1;
-                const void* velt[3];
-                for (int f = 0; f < 3; ++f) velt[f] = (char*)ws + (size_t(k) * 3 + f) * field;
-                adj_step(tt, velt);
-            }
+            for (int64_t tt = t; tt > t0; --tt) adj_step(tt, (char*)ws + size_t(tt - t0 - 1) * field);
             t = t0;
         }
         CFD_HIP(hipGetLastError());
     } catch (...) {
         pool_free(m->ctx, ws, s);
-        pool_free(m->ctx, pbuf, s);
+        pool_free(m->ctx, st, s);
         throw;
     }
     pool_free(m->ctx, ws, s);
-    pool_free(m->ctx, pbuf, s);
+    pool_free(m->ctx, st, s);
 }
 
 #define CFD_ADJ_INSTANTIATE(T)                                                                                  \
-    template void launch_wave_trace_step<T>(const cfd_mesh_s*, const void* const[4], void* const[4], double,   \
-                                            const void*, double, const SensorList&, void*, hipStream_t);        \
-    template void launch_wave_adj_step<T>(const cfd_mesh_s*, const void* const[4], void* const[4], double,     \
-                                          const void*, double, const SensorList&, const void*,                  \
-                                          const void* const[3], void*, hipStream_t);                            \
     template void launch_scatter_add<T>(void*, const SensorList&, const void*, hipStream_t);                   \
     template void run_wave_traces<T>(const cfd_mesh_s*, void* const[4], void* const[4], double, const void*,   \
                                      double, int64_t, const SensorList&, void*, void*, int64_t, hipStream_t);   \

@@ -20,13 +20,6 @@ struct SensorList {
 };
 SensorList make_sensors(const cfd_mesh_s* m, const int64_t* cells, int n);
 
-template <class T>
-void launch_wave_trace_step(const cfd_mesh_s* m, const void* const in[4], void* const out[4], double K,
-                            const void* Kf, double dt, const SensorList& sens, void* trace, hipStream_t s);
-template <class T>
-void launch_wave_adj_step(const cfd_mesh_s* m, const void* const in[4], void* const out[4], double K,
-                          const void* Kf, double dt, const SensorList& sens, const void* src,
-                          const void* const velt[3], void* gK, hipStream_t s);
 template <class T> void launch_scatter_add(void* lp, const SensorList& sens, const void* src, hipStream_t s);
 template <class T>
 void run_wave_traces(const cfd_mesh_s* m, void* const a[4], void* const b[4], double K, const void* Kf, double dt,

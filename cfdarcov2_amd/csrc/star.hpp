@@ -9,7 +9,8 @@
 // Any extents: rows need not start on 16-byte boundaries (global memory takes
 // multi-word accesses at element alignment), and the last unit of a row whose
 // extent is not a multiple of W is moved back to end with the row, so the
-// cells it shares with the unit before are computed twice with equal results.
+// cells it shares with the unit before are computed twice with equal results
+// (a kernel that updates a field in place must leave them to one of the two).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -95,8 +96,9 @@ template <class T> inline bool vector_form(int64_t Y, int64_t Z) {
     return Z >= kWidth<T> && Y * Z * int64_t(sizeof(T)) < (int64_t(1) << 32);
 }
 
-// The thread's place: plane x (uniform), row y, first cell z0; false without work.
-template <int W> __device__ inline bool place(const Plan& p, int& x, int& y, int& z0) {
+// The thread's place: plane x (uniform), row y, first cell z0; false without
+// work.  The first *skip of its cells belong to the unit before as well.
+template <int W> __device__ inline bool place(const Plan& p, int& x, int& y, int& z0, int* skip = nullptr) {
     const int lin = int((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
     if (lin >= p.blocks) return false;
     const int row = p.nzb == 1 ? lin : lin / p.nzb;
@@ -106,6 +108,7 @@ template <int W> __device__ inline bool place(const Plan& p, int& x, int& y, int
     const int zi = zb * p.bx + int(threadIdx.x);
     if (y >= p.Y || zi * W >= p.Z) return false;
     z0 = min(zi * W, p.Z - W);
+    if (skip) *skip = zi * W - z0;
     return true;
 }
 

@@ -317,15 +317,16 @@ int cfd_heat_adjoint(cfd_mesh_t mesh, void* adj_a, void* adj_b, double alpha, co
                      const void* checkpoints, int64_t every, void* grad_alpha, void* stream);
 
 /* Kernel form of cfd_wave_traces / cfd_wave_adjoint (no reference
- * counterpart): form 0 = one thread per cell; form 1 = row form (uniform
- * meshes whose z extent is a multiple of 4 and at most 256, else
- * CFD_E_UNSUPPORTED) with `tile_rows` (4 or 8; 4 in FP64) output waves and
- * `chunk` x-planes per workgroup.  The row form's forward records the traces in the
- * fused step itself; its transposed step needs a constant K (runs with a K
- * field take form 0 for the transposed steps) and its K gradient keeps one
- * divergence field per recomputed step instead of three velocity fields.
- * Both forms give bit-identical traces and gradients.  Uniform meshes that allow it start on form 1 (4 waves, 8
- * planes). */
+ * counterpart): form 0 = star form (any extents, constant K or a K field);
+ * form 1 = row form (uniform meshes whose z extent is a multiple of 4 and at
+ * most 256, else CFD_E_UNSUPPORTED) with `tile_rows` (4 or 8; 4 in FP64)
+ * output waves and `chunk` x-planes per workgroup.  The row form's transposed
+ * step needs a constant K (runs with a K field take form 0 for the transposed
+ * steps).  Both record the traces in the step itself, keep one divergence
+ * field per recomputed step for the K gradient and give bit-identical traces
+ * and gradients.  Until a form is set, a run takes form 0 while both states (8
+ * fields) fit 256 MiB (with the K gradient: half of that) and form 1 (4 waves,
+ * 8 planes) beyond, where the mesh allows it. */
 int cfd_mesh_set_adjoint_shape(cfd_mesh_t mesh, int form, int tile_rows, int chunk);
 
 /* ---- batched ensemble (FP32 uniform meshes; no reference counterpart) -----

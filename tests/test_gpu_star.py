@@ -129,3 +129,41 @@ def test_perturbed_mesh_is_no_lattice(hip_ctx):
     gm = capi.HexMesh(hip_ctx, *n, *d, dtype="f64", vertex_offsets=off)
     gg = capi.HexMesh(hip_ctx, *n, *d, dtype="f64", vertex_offsets=off, force_general=True)
     assert gm.info().device_bytes == gg.info().device_bytes
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("every", [1, 2, 3, 9])
+@pytest.mark.parametrize("n", EXTENTS[1:] + [(600, 2, 5)], ids=lambda n: "x".join(map(str, n)))
+def test_adjoint_star(hip_ctx, n, every, dtype):
+    """Traces and gradients (K field and constant K, checkpoint segments of
+    one to all steps, sensors in the first and last cells) against autograd
+    through the plain FP64 stepper.  Bound: 7 steps forward and back of some
+    30 roundings each, eps * 420 = 2.5e-5 in FP32 and 5e-14 in FP64."""
+    from cfdarcov2_amd import adjoint, capi
+    from tests import torch_wave
+    d, steps, dt = (0.125, 0.125, 0.125), 7, 0.04
+    N = n[0] * n[1] * n[2]
+    rng = np.random.default_rng(N)
+    sens = np.unique(np.concatenate([[0, N - 1, N // 2], rng.integers(N, size=min(N, 20))]))
+    p0 = rng.standard_normal(N).astype(dtype)
+    Kf = (-(0.5 + rng.random(N))).astype(dtype)
+    g = rng.standard_normal((steps, sens.size)).astype(dtype)
+    gm = capi.HexMesh(hip_ctx, *n, *d, dtype=dtype)
+    gm.set_adjoint_shape(0, 4, 8)
+    for field in (True, False):
+        pr = adjoint.WaveProblem(gm, sens, dt, steps, K=-0.75, every=every)
+        tp = torch.from_numpy(p0).cuda().requires_grad_(True)
+        tk = torch.from_numpy(Kf).cuda().requires_grad_(True) if field else None
+        tr = adjoint.wave_traces(tp, tk, pr)
+        got = [tr.detach(), *torch.autograd.grad(tr, [tp, tk] if field else [tp], torch.from_numpy(g).cuda())]
+        if not field:  # the K gradient at a constant K
+            _, _, ck = adjoint.forward_traces(pr, tp, checkpoints=True)
+            got.append(adjoint.adjoint(pr, torch.from_numpy(g).cuda(), None, ck, want_K=True)[1])
+        rp = torch.from_numpy(p0).double().requires_grad_(True)
+        rk = (torch.from_numpy(Kf).double() if field else torch.full((N,), -0.75, dtype=torch.float64)).requires_grad_(True)
+        rt = torch_wave.traces(rp, rk, dt, steps, torch.from_numpy(sens), n, d)
+        ref = [rt.detach(), *torch.autograd.grad(rt, [rp, rk], torch.from_numpy(g).double())]
+        for a, b in zip(got, ref):
+            err = (a.cpu().double() - b).norm() / max(float(b.norm()), 1e-30)
+            assert err < (2.5e-5 if dtype == np.float32 else 5e-14), (field, float(err))
+    gm.close()
