@@ -14,8 +14,8 @@
 // Time step, all on the device: the step kernel reads dt from a rotating slot,
 // and from the cell's new state computes V / sum_f A_f (|u.n_f| + a), reduces
 // the block minimum and folds it into the next slot with one atomic minimum
-// per block (non-negative floats order like their bit patterns).  A third slot
-// is reset to +inf for the step after, so the loop needs no host round trip.
+// per block.  A third slot is reset to +inf for the step after, so the loop
+// needs no host round trip.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -126,9 +126,18 @@ template <class T> __device__ inline T local_dt_faces(T V, const Prim<T>& q, con
     return V / s;
 }
 
+// The next time step is the minimum over all cells, folded with atomics.  All
+// workgroups on one address would queue there (12 ns each, measured: 100 us
+// for the 8,192 workgroups of a per-cell kernel at 512x64x64), so a slot is a
+// set of kDtSlots values on cache lines of their own, workgroups spread over
+// them, and every wave that needs the minimum reads the whole set, one value
+// per lane.  Non-negative floats order like their bit patterns.
+constexpr int kDtSlots = 64, kDtStride = 32;  // values, elements between them
+constexpr int kDtSet = kDtSlots * kDtStride;
+
 // minimum over the block (64 x blockDim.y threads, one wave per y row), folded
-// into *slot by thread (0, 0) with one atomic per block
-template <class T> __device__ inline void block_min_into(T v, Bits<T>* slot) {
+// into the set by thread (0, 0) with one atomic per block
+template <class T> __device__ inline void block_min_into(T v, Bits<T>* set) {
     __shared__ T red[16];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
@@ -138,9 +147,24 @@ template <class T> __device__ inline void block_min_into(T v, Bits<T>* slot) {
     if (lane == 0 && wave == 0) {
         T m = red[0];
         for (int w = 1; w < int(blockDim.y); ++w) m = fmin(m, red[w]);
-        if (m < std::numeric_limits<T>::infinity()) atomicMin(slot, to_bits(m));
+        const unsigned wg = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        if (m < std::numeric_limits<T>::infinity()) atomicMin(set + (wg % kDtSlots) * kDtStride, to_bits(m));
     }
 }
+
+// the minimum of a set (every lane of a wave takes part)
+template <class T> __device__ inline T set_min(const Bits<T>* set) {
+    Bits<T> b = set[int(threadIdx.x) * kDtStride];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const Bits<T> c = to_bits(__shfl_xor(from_bits(b), o, 64));
+        b = c < b ? c : b;
+    }
+    return from_bits(b);
+}
+
+// thread (0..63, 0) of the first workgroup clears a set
+template <class T> __device__ inline void set_reset(Bits<T>* set) { set[int(threadIdx.x) * kDtStride] = inf_bits<T>(); }
 
 template <class T>
 __global__ void __launch_bounds__(256) euler_dt_k(FvGeo<T> g, EIn<T> in, T gamma, Bits<T>* slot) {
@@ -165,10 +189,10 @@ __global__ void __launch_bounds__(256) euler_step_k(FvGeo<T> g, EIn<T> in, EOut<
     const int64_t z = int64_t(blockIdx.x) * 64 + threadIdx.x;
     const int64_t y = int64_t(blockIdx.y) * 4 + threadIdx.y;
     const int64_t x = blockIdx.z;
-    const T dt = cfl * from_bits(*dt_cur);
-    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
-        *dt_reset = inf_bits<T>();
-        if (dt_hist) dt_hist[step] = dt;
+    const T dt = cfl * set_min<T>(dt_cur);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.y == 0) {
+        set_reset<T>(dt_reset);
+        if (dt_hist && threadIdx.x == 0) dt_hist[step] = dt;
     }
     T loc = std::numeric_limits<T>::infinity();
     if (z < g.Z && y < g.Y) {
@@ -263,10 +287,10 @@ __global__ void __launch_bounds__(64 * TY) euler_march_k(FvGeo<T> g, EIn<T> in, 
     const int64_t col = valid ? y * Z + z : 0;
     const int64_t x0 = xc * L;
     const int64_t x1 = (x0 + L < X) ? x0 + L : X;
-    const T dt = cfl * from_bits(*dt_cur);
-    if (lin == 0 && lz == 0 && ly == 0) {
-        *dt_reset = inf_bits<T>();
-        if (dt_hist) dt_hist[step] = dt;
+    const T dt = cfl * set_min<T>(dt_cur);
+    if (lin == 0 && ly == 0) {
+        set_reset<T>(dt_reset);
+        if (dt_hist && lz == 0) dt_hist[step] = dt;
     }
     const int own = (ly + 1) * PZ + (lz + 1);
     // halo cells: row -1 (ly 0) / row TY (ly 1) at this column, column -1
@@ -334,27 +358,46 @@ __global__ void __launch_bounds__(64 * TY) euler_march_k(FvGeo<T> g, EIn<T> in, 
         rusanov(Ul, ql, Uc, qc, fg[4][0], fg[4][1], fg[4][2], fg[4][3], Gxl);
     }
     T loc = std::numeric_limits<T>::infinity();
+    // Everything a plane reads is loaded one plane ahead (the state of plane
+    // x + 1, the halo cells, the face geometry), so no plane waits for a load
+    // that it has just issued.
+    const uint32_t bhy = hy_col >= 0 ? uint32_t(hy_col) * uint32_t(sizeof(T)) : 0;
+    const uint32_t bhz = hz_col >= 0 ? uint32_t(hz_col) * uint32_t(sizeof(T)) : 0;
+    T Uy[5] = {}, Uz[5] = {}, Uf[5] = {}, fn[6][4] = {}, Vn = T(1);
+    auto fetch = [&](int64_t x) {
+        if (valid && x + 1 < X) load(x + 1, bcol, Uf);
+        if (hy_col >= 0) load(x, bhy, Uy);
+        if (hz_col >= 0) load(x, bhz, Uz);
+        if (valid) {
+            face4(2, (x + 1) * SX, bcol, fn[5]);
+            face4(1, x * (Y + 1) * Z, bcol, fn[2]);
+            face4(1, x * (Y + 1) * Z + Z, bcol, fn[3]);
+            const int64_t fz = x * Y * (Z + 1);
+            face4(0, fz, bzf, fn[0]);
+            face4(0, fz + 1, bzf, fn[1]);
+            Vn = at(g.vol + x * SX, bcol);
+        }
+    };
+    if (x0 < x1) fetch(x0);
     int b = 0;
 #pragma unroll 1
     for (int64_t x = x0; x < x1; ++x, b ^= 1) {
         T* S[10];
 #pragma unroll
         for (int k = 0; k < 10; ++k) S[k] = sh[b][k];
-        if (valid && x + 1 < X) {
-            load(x + 1, bcol, Un);
-            qn = prim(gamma, Un);
-        }
-        if (hy_col >= 0) {
-            T Uh[5];
-            load(x, uint32_t(hy_col) * uint32_t(sizeof(T)), Uh);
-            put(S, hy_slot, Uh, prim(gamma, Uh));
-        }
-        if (hz_col >= 0) {
-            T Uh[5];
-            load(x, uint32_t(hz_col) * uint32_t(sizeof(T)), Uh);
-            put(S, hz_slot, Uh, prim(gamma, Uh));
-        }
+        const T V = Vn;
+#pragma unroll
+        for (int f = 0; f < 6; ++f)
+            if (f != 4)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) fg[f][k] = fn[f][k];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) Un[k] = Uf[k];
+        if (valid && x + 1 < X) qn = prim(gamma, Un);
+        if (hy_col >= 0) put(S, hy_slot, Uy, prim(gamma, Uy));
+        if (hz_col >= 0) put(S, hz_slot, Uz, prim(gamma, Uz));
         if (valid) put(S, own, Uc, qc);
+        if (x + 1 < x1) fetch(x + 1);
         __syncthreads();
         if (valid) {
             T Um[5], G1[5], G2[5], acc[5];
@@ -362,7 +405,6 @@ __global__ void __launch_bounds__(64 * TY) euler_march_k(FvGeo<T> g, EIn<T> in, 
             // net = ((Gx+ - Gx-) + (Gy+ - Gy-)) + (Gz+ - Gz-), accumulated one
             // axis at a time; the upper x flux becomes the next plane's lower.
             // The six faces' geometry stays in registers for the next dt.
-            face4(2, (x + 1) * SX, bcol, fg[5]);
             if (x == X - 1) {
                 mirror(Uc, qc, 0, Um, qm);
                 rusanov(Uc, qc, Um, qm, fg[5][0], fg[5][1], fg[5][2], fg[5][3], G1);
@@ -375,27 +417,21 @@ __global__ void __launch_bounds__(64 * TY) euler_march_k(FvGeo<T> g, EIn<T> in, 
                 Gxl[k] = G1[k];
             }
             // y faces
-            face4(1, x * (Y + 1) * Z, bcol, fg[2]);
             if (y == 0) mirror(Uc, qc, 1, Um, qm);
             else get(S, own - PZ, Um, qm);
             rusanov(Um, qm, Uc, qc, fg[2][0], fg[2][1], fg[2][2], fg[2][3], G1);
-            face4(1, x * (Y + 1) * Z + Z, bcol, fg[3]);
             if (y == Y - 1) mirror(Uc, qc, 1, Um, qm);
             else get(S, own + PZ, Um, qm);
             rusanov(Uc, qc, Um, qm, fg[3][0], fg[3][1], fg[3][2], fg[3][3], G2);
 #pragma unroll
             for (int k = 0; k < 5; ++k) acc[k] = acc[k] + (G2[k] - G1[k]);
             // z faces
-            const int64_t fz = x * Y * (Z + 1);
-            face4(0, fz, bzf, fg[0]);
             if (z == 0) mirror(Uc, qc, 2, Um, qm);
             else get(S, own - 1, Um, qm);
             rusanov(Um, qm, Uc, qc, fg[0][0], fg[0][1], fg[0][2], fg[0][3], G1);
-            face4(0, fz + 1, bzf, fg[1]);
             if (z == Z - 1) mirror(Uc, qc, 2, Um, qm);
             else get(S, own + 1, Um, qm);
             rusanov(Uc, qc, Um, qm, fg[1][0], fg[1][1], fg[1][2], fg[1][3], G2);
-            const T V = at(g.vol + x * SX, bcol);
             const T iV = T(1) / V;
             T Unew[5];
 #pragma unroll
@@ -416,7 +452,8 @@ __global__ void __launch_bounds__(64 * TY) euler_march_k(FvGeo<T> g, EIn<T> in, 
 }
 
 template <class B> __global__ void fill_bits_k(B* p, int n, B v) {
-    if (int(threadIdx.x) < n) p[threadIdx.x] = v;
+    const int i = int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x);
+    if (i < n) p[i] = v;
 }
 
 // Device geometry of the stepper, built on first use from the mesh's vertices.
@@ -456,12 +493,12 @@ template <class T>
 void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamma, double cfl, int64_t nsteps,
                   void* dt_hist, hipStream_t s) {
     const FvGeo<T>& g = fv_geometry<T>(m, s);
-    Bits<T>* slots = (Bits<T>*)pool_alloc(m->ctx, 3 * sizeof(Bits<T>), s);
+    Bits<T>* slots = (Bits<T>*)pool_alloc(m->ctx, 3 * kDtSet * sizeof(Bits<T>), s);
     try {
         const dim3 block(64, 4, 1);
         const dim3 grid(unsigned((m->Z + 63) / 64), unsigned((m->Y + 3) / 4), unsigned(m->X));
         const Bits<T> inf = sizeof(T) == 4 ? Bits<T>(0x7f800000u) : Bits<T>(0x7ff0000000000000ull);
-        fill_bits_k<Bits<T>><<<1, 64, 0, s>>>(slots, 3, inf);
+        fill_bits_k<Bits<T>><<<3 * kDtSet / 256, 256, 0, s>>>(slots, 3 * kDtSet, inf);
         EIn<T> in{};
         EOut<T> out{};
         for (int k = 0; k < 5; ++k) in.u[k] = (const T*)a[k];
@@ -480,9 +517,9 @@ void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamm
                 in.u[k] = (const T*)src[k];
                 out.u[k] = (T*)dst[k];
             }
-            Bits<T>* cur = slots + (st % 3);
-            Bits<T>* nxt = slots + ((st + 1) % 3);
-            Bits<T>* rst = slots + ((st + 2) % 3);
+            Bits<T>* cur = slots + (st % 3) * kDtSet;
+            Bits<T>* nxt = slots + ((st + 1) % 3) * kDtSet;
+            Bits<T>* rst = slots + ((st + 2) % 3) * kDtSet;
             if (m->euler_variant == 0) {
                 euler_step_k<T><<<grid, block, 0, s>>>(g, in, out, T(gamma), T(cfl), cur, nxt, rst, (T*)dt_hist,
                                                        st);
@@ -557,10 +594,10 @@ __global__ void __launch_bounds__(256) ueuler_step_k(UnstructGeo<T> g, EIn<T> in
                                                     const Bits<T>* dt_cur, Bits<T>* dt_next, Bits<T>* dt_reset,
                                                     T* dt_hist, int64_t step) {
     const int64_t i = ucell();
-    const T dt = cfl * from_bits(*dt_cur);
-    if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
-        *dt_reset = inf_bits<T>();
-        if (dt_hist) dt_hist[step] = dt;
+    const T dt = cfl * set_min<T>(dt_cur);
+    if (blockIdx.x == 0 && threadIdx.y == 0) {
+        set_reset<T>(dt_reset);
+        if (dt_hist && threadIdx.x == 0) dt_hist[step] = dt;
     }
     T loc = std::numeric_limits<T>::infinity();
     if (i < g.N) {
@@ -657,12 +694,12 @@ template <class T>
 void launch_ueuler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamma, double cfl, int64_t nsteps,
                    void* dt_hist, hipStream_t s) {
     const UnstructGeo<T>& g = ufv_geometry<T>(m, s);
-    Bits<T>* slots = (Bits<T>*)pool_alloc(m->ctx, 3 * sizeof(Bits<T>), s);
+    Bits<T>* slots = (Bits<T>*)pool_alloc(m->ctx, 3 * kDtSet * sizeof(Bits<T>), s);
     try {
         const dim3 block(64, 4, 1);
         const dim3 grid(unsigned((m->N + 255) / 256));
         const Bits<T> inf = sizeof(T) == 4 ? Bits<T>(0x7f800000u) : Bits<T>(0x7ff0000000000000ull);
-        fill_bits_k<Bits<T>><<<1, 64, 0, s>>>(slots, 3, inf);
+        fill_bits_k<Bits<T>><<<3 * kDtSet / 256, 256, 0, s>>>(slots, 3 * kDtSet, inf);
         EIn<T> in{};
         EOut<T> out{};
         for (int k = 0; k < 5; ++k) in.u[k] = (const T*)a[k];
@@ -675,8 +712,8 @@ void launch_ueuler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gam
                 in.u[k] = (const T*)src[k];
                 out.u[k] = (T*)dst[k];
             }
-            ueuler_step_k<T><<<grid, block, 0, s>>>(g, in, out, T(gamma), T(cfl), slots + (st % 3),
-                                                    slots + ((st + 1) % 3), slots + ((st + 2) % 3), (T*)dt_hist, st);
+            ueuler_step_k<T><<<grid, block, 0, s>>>(g, in, out, T(gamma), T(cfl), slots + (st % 3) * kDtSet,
+                                                    slots + ((st + 1) % 3) * kDtSet, slots + ((st + 2) % 3) * kDtSet, (T*)dt_hist, st);
             CFD_HIP(hipGetLastError());
         }
     } catch (...) {
