@@ -123,6 +123,15 @@ template <class T> struct FvGeo {
     const T* vol;
 };
 
+// The same geometry of a mesh whose vector-area normals are exactly the unit
+// vectors: areas and volume as constants (vol null), or areas as products of
+// the layer widths and the volume per cell.
+template <class T> struct FvAxis {
+    T A[3], V;
+    const T* w[3];
+    const T* vol;
+};
+
 // Connectivity of an unstructured hex mesh (cfd_mesh_create_unstructured), in
 // the caller's numbering.
 struct UConn {
@@ -201,9 +210,10 @@ struct cfd_mesh_s {
     const void* hg_af = nullptr;
     double hg_alpha = 0, hg_dt = 0;
     int hg_shape[3] = {-1, 0, 0};
-    // Euler stepper: variant 0 = one thread per cell, 1 = 2.5D march with
-    // `euler_ty` rows x 64 columns x `euler_L` planes per workgroup
-    int euler_variant = 1;
+    // Euler stepper: variant 0 = one thread per cell, 1 = march with
+    // `euler_ty` x 64 cells x `euler_L` planes per workgroup, -1 = variant 1
+    // with a tile by the mesh's size
+    int euler_variant = -1;
     int euler_ty = 4;
     int euler_L = 16;
     // adjoint of the acoustic step (cfd_wave_traces / cfd_wave_adjoint):
@@ -226,4 +236,10 @@ struct cfd_mesh_s {
     cfd::FvGeo<double> fv64{};
     void* fv_block = nullptr;
     int64_t fv_bytes = 0;
+    // 0 = not looked at, 1 = axis-aligned (fa32 / fa64, the volumes in
+    // fa_block where they differ), 2 = faces of any direction
+    int fv_axis = 0;
+    cfd::FvAxis<float> fa32{};
+    cfd::FvAxis<double> fa64{};
+    void* fa_block = nullptr;
 };

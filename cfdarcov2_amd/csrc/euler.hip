@@ -43,6 +43,13 @@ template <class T> struct EOut { T* u[5]; };
 
 template <class T> struct Prim { T ux, uy, uz, p, a; };
 
+// the rotating dt sets of one step
+template <class T> struct EulerSlots {
+    const Bits<T>* cur;
+    Bits<T>* next;
+    Bits<T>* reset;
+};
+
 // a * b + c rounded once (the fused multiply-add the scheme's rounding is
 // defined with; the oracle uses std::fma in the same places)
 template <class T> __device__ inline T fmul_add(T a, T b, T c) {
@@ -451,48 +458,487 @@ __global__ void __launch_bounds__(64 * TY) euler_march_k(FvGeo<T> g, EIn<T> in, 
     block_min_into(loc, dt_next);
 }
 
+// ---------------------------------------------------------------------------
+// The Rusanov step as a march along x over tiles of consecutive cells of a
+// plane (variant 1 where a row is at most half a tile).
+//
+// A workgroup owns B consecutive cells c = y*Z + z of each of its L planes, so
+// any Z fills its lanes (tiles of whole 64-cell columns leave 45% of them idle
+// at Z = 70).  Each cell's state and primitives go to LDS once per plane with
+// Z halo cells on either side, at most one per thread; the y and z neighbours
+// are the slots Z and 1 away, a wall's neighbour is the cell itself with the
+// normal momentum's sign flipped.  The flux between planes x and x+1 is carried
+// in registers, and all a plane reads is loaded one plane ahead.  Every face
+// flux is evaluated with the lower cell as L, as in euler_step_k, so both give
+// the same bits.
+//
+// GEO 0: face normals, areas and volumes per face and cell (FvGeo).
+// GEO 1 / 2: axis-aligned meshes (FvAxis), whose normals are exactly the unit
+// vectors: constants for the areas and the volume (1), or areas as products of
+// layer widths and the volume per cell (2).  A cell's two fluxes along an axis
+// then share its own flux vector and wave speed.
+// ---------------------------------------------------------------------------
+namespace {
+
+template <class T, int GEO> struct TileGeo { using type = FvAxis<T>; };
+template <class T> struct TileGeo<T, 0> { using type = FvGeo<T>; };
+
+// a slot's state and primitives, moved as pairs
+template <class T> struct Pair { typedef T type __attribute__((ext_vector_type(2))); };
+constexpr int kSlot = 10;
+
+template <class T> __device__ inline void put10(T* slot, const T (&U)[5], const Prim<T>& q) {
+    using P = typename Pair<T>::type;
+    P* const d = reinterpret_cast<P*>(slot);
+    d[0] = P{U[0], U[1]};
+    d[1] = P{U[2], U[3]};
+    d[2] = P{U[4], q.ux};
+    d[3] = P{q.uy, q.uz};
+    d[4] = P{q.p, q.a};
+}
+template <class T> __device__ inline void get10(const T* slot, T (&U)[5], Prim<T>& q) {
+    using P = typename Pair<T>::type;
+    const P* const d = reinterpret_cast<const P*>(slot);
+    const P a = d[0], b = d[1], c = d[2], e = d[3], f = d[4];
+    U[0] = a[0]; U[1] = a[1]; U[2] = b[0]; U[3] = b[1]; U[4] = c[0];
+    q.ux = c[1]; q.uy = e[0]; q.uz = e[1]; q.p = f[0]; q.a = f[1];
+}
+
+template <class T> __device__ inline T at(const T* base, uint32_t boff) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + boff);
+}
+
+
+template <class T, int GEO>
+__device__ inline void axis_faces(T Ax, T Ay, T Az, T (&f)[6][4]) {
+#pragma unroll
+    for (int fc = 0; fc < 6; ++fc) {
+        const int a = 2 - (fc >> 1);
+        f[fc][0] = T(a == 0);
+        f[fc][1] = T(a == 1);
+        f[fc][2] = T(a == 2);
+        f[fc][3] = a == 0 ? Ax : a == 1 ? Ay : Az;
+    }
+}
+
+}  // namespace
+
+template <class T, int B, int GEO>
+__global__ void __launch_bounds__(B) euler_tile_k(typename TileGeo<T, GEO>::type g, EIn<T> in, EOut<T> out, int64_t X,
+                                                  int Y, int Z, T gamma, T cfl, const Bits<T>* dt_cur,
+                                                  Bits<T>* dt_next, Bits<T>* dt_reset, T* dt_hist, int64_t step, int L,
+                                                  int ntile) {
+    extern __shared__ __align__(16) char lds_raw[];
+    T* const lds = reinterpret_cast<T*>(lds_raw);
+    const int NS = B + 2 * Z;  // slots of one plane; two planes, used in turn
+    const int plane = Y * Z;
+    const int64_t SX = plane;
+    const int lin = blockIdx.x;
+    const int tile = lin % ntile;
+    const int64_t x0 = int64_t(lin / ntile) * L;
+    const int64_t x1 = (x0 + L < X) ? x0 + L : X;
+    const int tid = threadIdx.y * 64 + threadIdx.x;
+    const int c0 = tile * B, c = c0 + tid;
+    const bool valid = c < plane;
+    const int y = valid ? c / Z : 0, z = valid ? c - y * Z : 0;
+    const bool zlo = z == 0, zhi = z == Z - 1, ylo = y == 0, yhi = y == Y - 1;
+    const T dt = cfl * set_min<T>(dt_cur);
+    if (lin == 0 && threadIdx.y == 0) {
+        set_reset<T>(dt_reset);
+        if (dt_hist && threadIdx.x == 0) dt_hist[step] = dt;
+    }
+    const int own = (Z + tid) * kSlot;
+    // the neighbours' slots, the cell's own at a wall
+    const int szl = zlo ? own : own - kSlot, szh = zhi ? own : own + kSlot;
+    const int syl = ylo ? own : own - Z * kSlot, syh = yhi ? own : own + Z * kSlot;
+    // halo cell of this thread: Z cells before the tile, Z cells after it
+    const int hc = tid < Z ? c0 - Z + tid : c0 + B + tid - Z;
+    const bool halo = tid < 2 * Z && hc >= 0 && hc < plane;
+    const int hslot = (tid < Z ? tid : B + tid) * kSlot;
+    // addresses: a pointer uniform over the workgroup and a 32-bit byte offset
+    // per lane (the launcher checks that a plane fits)
+    const uint32_t bc = uint32_t(valid ? c : 0) * uint32_t(sizeof(T));
+    const uint32_t bh = uint32_t(halo ? hc : 0) * uint32_t(sizeof(T));
+    const uint32_t bzf = uint32_t(y * (Z + 1) + z) * uint32_t(sizeof(T));
+    auto load = [&](int64_t p, uint32_t boff, T (&U)[5]) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) U[k] = at(in.u[k] + p * SX, boff);
+    };
+    auto face4 = [&](int fam, int64_t first, uint32_t boff, T (&o)[4]) {
+        if constexpr (GEO == 0) {
+            o[0] = at(g.n[fam][0] + first, boff);
+            o[1] = at(g.n[fam][1] + first, boff);
+            o[2] = at(g.n[fam][2] + first, boff);
+            o[3] = at(g.A[fam] + first, boff);
+        }
+    };
+
+    T fg[6][4] = {};
+    T wyz = T(0), wy = T(0), wz = T(0);
+    if constexpr (GEO == 1) axis_faces<T, GEO>(g.A[0], g.A[1], g.A[2], fg);
+    if constexpr (GEO == 2) {
+        wy = g.w[1][y];
+        wz = g.w[2][z];
+        wyz = wy * wz;
+    }
+    T Uc[5] = {}, Gxl[5] = {};
+    Prim<T> qc{};
+    T Uh[5] = {}, Uf[5] = {}, fn[6][4] = {}, Vn = T(1);
+    auto fetch = [&](int64_t x) {  // for plane x: its halo cell and geometry, the state of plane x + 1
+        if (valid && x + 1 < X) load(x + 1, bc, Uf);
+        if (halo) load(x, bh, Uh);
+        if (valid) {
+            if constexpr (GEO == 0) {
+                face4(2, (x + 1) * SX, bc, fn[5]);
+                face4(1, x * int64_t(Y + 1) * Z, bc, fn[2]);
+                face4(1, x * int64_t(Y + 1) * Z + Z, bc, fn[3]);
+                const int64_t fz = x * int64_t(Y) * (Z + 1);
+                face4(0, fz, bzf, fn[0]);
+                face4(0, fz + 1, bzf, fn[1]);
+            }
+            if constexpr (GEO != 1) Vn = at(g.vol + x * SX, bc);
+        }
+    };
+    T Ul[5] = {};
+    if (valid) {  // warm-up: state of plane x0 and the flux through its lower x-face
+        load(x0, bc, Uc);
+        if (x0 > 0) load(x0 - 1, bc, Ul);
+        face4(2, x0 * SX, bc, fg[4]);
+    }
+    fetch(x0);
+    if constexpr (GEO == 2) axis_faces<T, GEO>(wyz, T(0), T(0), fg);
+    {
+        qc = prim(gamma, Uc);
+        Prim<T> ql = qc;
+        if (x0 == 0) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) Ul[k] = Uc[k];
+            Ul[1] = -Uc[1];
+            ql.ux = -qc.ux;
+        } else {
+            ql = prim(gamma, Ul);
+        }
+        rusanov(Ul, ql, Uc, qc, fg[4][0], fg[4][1], fg[4][2], fg[4][3], Gxl);
+    }
+    T loc = std::numeric_limits<T>::infinity();
+    int b = 0;
+#pragma unroll 1
+    for (int64_t x = x0; x < x1; ++x, b ^= 1) {
+        T* const S = lds + b * NS * kSlot;
+        T V = Vn;
+        if constexpr (GEO == 1) V = g.V;
+        if constexpr (GEO == 0) {
+#pragma unroll
+            for (int f = 0; f < 6; ++f)
+                if (f != 4)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) fg[f][k] = fn[f][k];
+        }
+        if constexpr (GEO == 2) {
+            const T wx = g.w[0][x];
+            axis_faces<T, GEO>(wyz, wx * wz, wx * wy, fg);
+        }
+        T Un[5];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) Un[k] = Uf[k];
+        if (halo) put10(S + hslot, Uh, prim(gamma, Uh));
+        put10(S + own, Uc, qc);
+        if (x + 1 < x1) fetch(x + 1);
+        __syncthreads();
+        if (valid) {
+            T Um[5], G1[5], G2[5], acc[5];
+            Prim<T> qn, qm;
+            // net = ((Gx+ - Gx-) + (Gy+ - Gy-)) + (Gz+ - Gz-), accumulated one
+            // axis at a time; the upper x flux becomes the next plane's lower
+            if (x == X - 1) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) Un[k] = Uc[k];
+                Un[1] = -Uc[1];
+                qn = qc;
+                qn.ux = -qc.ux;
+            } else {
+                qn = prim(gamma, Un);
+            }
+            rusanov(Uc, qc, Un, qn, fg[5][0], fg[5][1], fg[5][2], fg[5][3], G1);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                acc[k] = G1[k] - Gxl[k];
+                Gxl[k] = G1[k];
+            }
+            get10(S + syl, Um, qm);
+            if (ylo) { Um[2] = -Um[2]; qm.uy = -qm.uy; }
+            rusanov(Um, qm, Uc, qc, fg[2][0], fg[2][1], fg[2][2], fg[2][3], G1);
+            get10(S + syh, Um, qm);
+            if (yhi) { Um[2] = -Um[2]; qm.uy = -qm.uy; }
+            rusanov(Uc, qc, Um, qm, fg[3][0], fg[3][1], fg[3][2], fg[3][3], G2);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) acc[k] = acc[k] + (G2[k] - G1[k]);
+            get10(S + szl, Um, qm);
+            if (zlo) { Um[3] = -Um[3]; qm.uz = -qm.uz; }
+            rusanov(Um, qm, Uc, qc, fg[0][0], fg[0][1], fg[0][2], fg[0][3], G1);
+            get10(S + szh, Um, qm);
+            if (zhi) { Um[3] = -Um[3]; qm.uz = -qm.uz; }
+            rusanov(Uc, qc, Um, qm, fg[1][0], fg[1][1], fg[1][2], fg[1][3], G2);
+            const T iV = T(1) / V;
+            T Unew[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                const T net = acc[k] + (G2[k] - G1[k]);
+                Unew[k] = fmul_add(-(dt * net), iV, Uc[k]);
+                *reinterpret_cast<T*>(reinterpret_cast<char*>(out.u[k] + x * SX) + bc) = Unew[k];
+            }
+            loc = fmin(loc, local_dt_faces(V, prim(gamma, Unew), fg));
+#pragma unroll
+            for (int k = 0; k < 5; ++k) Uc[k] = Un[k];
+            qc = qn;
+            if constexpr (GEO == 0) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) fg[4][k] = fg[5][k];
+            }
+        }
+    }
+    block_min_into(loc, dt_next);
+}
+
+// the time step of the initial state on an axis-aligned mesh
+template <class T, int GEO>
+__global__ void __launch_bounds__(256) euler_dt_axis_k(FvAxis<T> g, EIn<T> in, int Y, int Z, T gamma, Bits<T>* slot) {
+    const int c = int(blockIdx.x) * 256 + int(threadIdx.y) * 64 + int(threadIdx.x);
+    const int64_t x = blockIdx.y;
+    T loc = std::numeric_limits<T>::infinity();
+    if (c < Y * Z) {
+        const int64_t i = x * (int64_t(Y) * Z) + c;
+        T U[5], fg[6][4], V = g.V;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) U[k] = in.u[k][i];
+        if constexpr (GEO == 1) {
+            axis_faces<T, GEO>(g.A[0], g.A[1], g.A[2], fg);
+        } else {
+            const int y = c / Z, z = c - y * Z;
+            const T wx = g.w[0][x], wy = g.w[1][y], wz = g.w[2][z];
+            axis_faces<T, GEO>(wy * wz, wx * wz, wx * wy, fg);
+            V = g.vol[i];
+        }
+        loc = local_dt_faces(V, prim(gamma, U), fg);
+    }
+    block_min_into(loc, slot);
+}
+
+template <class T>
+static void launch_euler_dt_axis(const cfd_mesh_s* m, const FvAxis<T>& g, const EIn<T>& in, T gamma, Bits<T>* slot,
+                          hipStream_t s) {
+    const dim3 grid(unsigned((m->Y * m->Z + 255) / 256), unsigned(m->X));
+    if (g.vol) euler_dt_axis_k<T, 2><<<grid, dim3(64, 4), 0, s>>>(g, in, int(m->Y), int(m->Z), gamma, slot);
+    else euler_dt_axis_k<T, 1><<<grid, dim3(64, 4), 0, s>>>(g, in, int(m->Y), int(m->Z), gamma, slot);
+    CFD_HIP(hipGetLastError());
+}
+
+static bool euler_tile_supported(const cfd_mesh_s* m, int rows) {
+    return 2 * m->Z <= 64 * rows && m->Y * (m->Z + 1) * 8 < (int64_t(1) << 31);
+}
+
+// Tile and chunk by size: the time of a step goes as the rounds of workgroups
+// the chip needs times the planes of one, L and about 1.7 more for its start,
+// at the builds' waves per SIMD (FP32 2, FP64 1; axis-aligned 4 and 2).  The
+// smallest product was the fastest shape measured, or within 4% of it, at all
+// of 512x64x64, 300x40x70, 242x18x21, 80x33x27 and 45x70x76, both precisions,
+// all geometries (FP32 us/step against 4 rows x 16 planes throughout:
+// perturbed 40.5 / 43.8, 25.4 / 35.4, 8.8 / 32.8, 8.7 / 33.5, 11.9 / 35.0).
+// Equal products go to the larger tile (fewer halo cells) on meshes of 2^19
+// cells and more.
+static void euler_tile_shape(const cfd_mesh_s* m, bool axis, int& rows, int& L) {
+    const bool f32 = m->dtype == CFD_F32;
+    const int waves = (f32 ? 2 : 1) * (axis ? 2 : 1);
+    const bool large = m->N >= (int64_t(1) << 19);
+    const bool any = euler_tile_supported(m, f32 ? 8 : 4);
+    double best = std::numeric_limits<double>::infinity();
+    for (int k = 0; k < 3; ++k) {
+        const int r = large ? 8 >> k : (k == 0 ? 4 : k == 1 ? 8 : 2);
+        if ((r == 8 && !f32) || (any && !euler_tile_supported(m, r))) continue;
+        const int64_t B = 64 * r;
+        const int64_t tiles = any ? (m->Y * m->Z + B - 1) / B : ((m->Z + 63) / 64) * ((m->Y + r - 1) / r);
+        const int64_t room = 256 * 4 * waves / r;
+        for (int l = 32; l >= 1; l /= 2) {
+            const int64_t wg = tiles * ((m->X + l - 1) / l);
+            const double t = double((wg + room - 1) / room) * (l + 1.7);
+            if (t < best) {
+                best = t;
+                rows = r;
+                L = l;
+            }
+        }
+    }
+}
+
+// One step; rows = 2, 4 or 8 (FP32) gives tiles of 64 * rows cells.  Exactly
+// one of `faces` and `axis` is given.
+template <class T>
+static void launch_euler_tile(const cfd_mesh_s* m, const FvGeo<T>* faces, const FvAxis<T>* axis, const EIn<T>& in,
+                       const EOut<T>& out, T gamma, T cfl, const EulerSlots<T>& sl, T* dt_hist, int64_t step, int rows,
+                       int L, hipStream_t s) {
+    const int B = 64 * rows, Z = int(m->Z);
+    const int64_t ntile = (m->Y * m->Z + B - 1) / B;
+    const int64_t nwg = ntile * ((m->X + L - 1) / L);
+    CFD_REQUIRE(nwg < (int64_t(1) << 31), "euler march grid too large");
+    const size_t lds = size_t(2) * (B + 2 * Z) * kSlot * sizeof(T);
+    auto run = [&](auto kern, const auto& g) {
+        if (lds > 65536)
+            CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        int(lds)));
+        kern<<<dim3(unsigned(nwg)), dim3(64, unsigned(rows)), lds, s>>>(g, in, out, m->X, int(m->Y), Z, gamma, cfl,
+                                                                       sl.cur, sl.next, sl.reset, dt_hist, step, L,
+                                                                       int(ntile));
+        CFD_HIP(hipGetLastError());
+    };
+    auto with_rows = [&](auto r) {
+        constexpr int BB = 64 * decltype(r)::value;
+        if (faces) run(euler_tile_k<T, BB, 0>, *faces);
+        else if (axis->vol) run(euler_tile_k<T, BB, 2>, *axis);
+        else run(euler_tile_k<T, BB, 1>, *axis);
+    };
+    switch (rows) {
+        case 2: with_rows(std::integral_constant<int, 2>{}); break;
+        case 4: with_rows(std::integral_constant<int, 4>{}); break;
+        case 8:
+            if constexpr (sizeof(T) == 4) {
+                with_rows(std::integral_constant<int, 8>{});
+                break;
+            }
+            [[fallthrough]];
+        default: throw Error(CFD_E_INVALID, "euler tiles have 2, 4 or 8 (2 or 4 in FP64) times 64 cells");
+    }
+}
+
 template <class B> __global__ void fill_bits_k(B* p, int n, B v) {
     const int i = int(blockIdx.x) * int(blockDim.x) + int(threadIdx.x);
     if (i < n) p[i] = v;
 }
 
-// Device geometry of the stepper, built on first use from the mesh's vertices.
-template <class T> static FvGeo<T>& fv_geometry(cfd_mesh_s* m, hipStream_t s) {
-    FvGeo<T>& fv = [&]() -> FvGeo<T>& {
-        if constexpr (sizeof(T) == 4) return m->fv32; else return m->fv64;
-    }();
-    if (m->fv_block) return fv;
+// Device geometry of the stepper, built on first use from the mesh's vertices:
+// the stepper's host arrays, then on the device either what an axis-aligned
+// mesh needs of them or all of them.
+template <class T> struct FvHost {
     HexGeometry<T> g;
-    build_hex_geometry<T>(g, m->X, m->Y, m->Z, T(m->dx), T(m->dy), T(m->dz),
-                          m->has_offsets ? m->vertex_offsets.data() : nullptr);
-    std::vector<T> host;
+    std::vector<T> v;
     int64_t off_fam[3], off_vol;
-    build_fv_geometry<T>(g, host, off_fam, off_vol);
-    const int64_t bytes = int64_t(host.size() * sizeof(T));
+};
+
+template <class T> static void build_fv_host(const cfd_mesh_s* m, FvHost<T>& h) {
+    build_hex_geometry<T>(h.g, m->X, m->Y, m->Z, T(m->dx), T(m->dy), T(m->dz),
+                          m->has_offsets ? m->vertex_offsets.data() : nullptr);
+    build_fv_geometry<T>(h.g, h.v, h.off_fam, h.off_vol);
+}
+
+static void* fv_upload(cfd_mesh_s* m, const void* host, int64_t bytes, hipStream_t s) {
     void* dev = pool_alloc(m->ctx, bytes, s);
-    hipError_t e = hipMemcpyAsync(dev, host.data(), size_t(bytes), hipMemcpyHostToDevice, s);
+    hipError_t e = hipMemcpyAsync(dev, host, size_t(bytes), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         pool_free(m->ctx, dev, s);
         CFD_HIP(e);
     }
-    T* d = (T*)dev;
+    return dev;
+}
+
+template <class T> static FvGeo<T>& fv_of(cfd_mesh_s* m) {
+    if constexpr (sizeof(T) == 4) return m->fv32; else return m->fv64;
+}
+template <class T> static FvAxis<T>& fa_of(cfd_mesh_s* m) {
+    if constexpr (sizeof(T) == 4) return m->fa32; else return m->fa64;
+}
+
+template <class T> static void upload_faces(cfd_mesh_s* m, const FvHost<T>& h, hipStream_t s) {
+    const int64_t bytes = int64_t(h.v.size() * sizeof(T));
+    const T* d = (const T*)(m->fv_block = fv_upload(m, h.v.data(), bytes, s));
+    m->fv_bytes = bytes;
+    FvGeo<T>& fv = fv_of<T>(m);
     fv.X = m->X; fv.Y = m->Y; fv.Z = m->Z;
     for (int fam = 0; fam < 3; ++fam) {
-        const int64_t nf = g.nf[fam];
-        for (int k = 0; k < 3; ++k) fv.n[fam][k] = d + off_fam[fam] + k * nf;
-        fv.A[fam] = d + off_fam[fam] + 3 * nf;
+        const int64_t nf = h.g.nf[fam];
+        for (int k = 0; k < 3; ++k) fv.n[fam][k] = d + h.off_fam[fam] + k * nf;
+        fv.A[fam] = d + h.off_fam[fam] + 3 * nf;
     }
-    fv.vol = d + off_vol;
-    m->fv_block = dev;
-    m->fv_bytes = bytes;
-    return fv;
+    fv.vol = d + h.off_vol;
+}
+
+template <class T> static const FvGeo<T>& fv_geometry(cfd_mesh_s* m, hipStream_t s) {
+    if (!m->fv_block) {
+        FvHost<T> h;
+        build_fv_host(m, h);
+        upload_faces(m, h, s);
+    }
+    return fv_of<T>(m);
+}
+
+// The axis-aligned form, or null.  Every normal must be a unit vector exactly,
+// and the areas (and the volume of a uniform mesh) what the kernels form.
+template <class T> static const FvAxis<T>* fv_axis(cfd_mesh_s* m, hipStream_t s) {
+    FvAxis<T>& fa = fa_of<T>(m);
+    if (m->fv_axis) return m->fv_axis == 1 ? &fa : nullptr;
+    if (!m->uniform && !m->lattice) {
+        m->fv_axis = 2;
+        return nullptr;
+    }
+    FvHost<T> h;
+    build_fv_host(m, h);
+    const HexGeometry<T>& g = h.g;
+    const int64_t vs[3] = {(g.Y + 1) * (g.Z + 1), g.Z + 1, 1}, ext[3] = {g.X, g.Y, g.Z};
+    const std::vector<T>* vert[3] = {&g.vx, &g.vy, &g.vz};
+    std::vector<T> w[3];
+    for (int a = 0; a < 3; ++a)
+        for (int64_t k = 0; k < ext[a]; ++k)
+            w[a].push_back((*vert[a])[size_t((k + 1) * vs[a])] - (*vert[a])[size_t(k * vs[a])]);
+    int bad = 0;
+    FvAxis<T> f{};
+    for (int fam = 0; fam < 3 && !bad; ++fam) {
+        const int axis = 2 - fam;
+        const T* d = h.v.data() + h.off_fam[fam];
+        const int64_t nf = g.nf[fam];
+        f.A[axis] = d[3 * nf];
+        const int64_t nx = g.X + (axis == 0), ny = g.Y + (axis == 1), nz = g.Z + (axis == 2);
+#pragma omp parallel for schedule(static) reduction(+ : bad)
+        for (int64_t x = 0; x < nx; ++x)
+            for (int64_t y = 0; y < ny; ++y)
+                for (int64_t z = 0; z < nz; ++z) {
+                    const int64_t i = fam == 0 ? g.zface(x, y, z) : fam == 1 ? g.yface(x, y, z) : g.xface(x, y, z);
+                    for (int k = 0; k < 3; ++k) bad += !(d[k * nf + i] == (k == axis ? T(1) : T(0)));
+                    const T A = m->uniform ? f.A[axis]
+                              : axis == 0 ? w[1][y] * w[2][z] : axis == 1 ? w[0][x] * w[2][z] : w[0][x] * w[1][y];
+                    bad += !(d[3 * nf + i] == A);
+                }
+    }
+    const T* vol = h.v.data() + h.off_vol;
+    f.V = vol[0];
+    if (m->uniform)
+        for (int64_t i = 0; i < g.N; ++i) bad += !(vol[i] == f.V);
+    if (bad) {
+        m->fv_axis = 2;
+        if (!m->fv_block) upload_faces(m, h, s);
+        return nullptr;
+    }
+    if (!m->uniform) {
+        m->fa_block = fv_upload(m, vol, g.N * int64_t(sizeof(T)), s);
+        f.vol = (const T*)m->fa_block;
+        const LatticeGeo<T>& lg = [&]() -> const LatticeGeo<T>& {
+            if constexpr (sizeof(T) == 4) return m->lg32; else return m->lg64;
+        }();
+        for (int a = 0; a < 3; ++a) f.w[a] = lg.w[a];
+    }
+    fa = f;
+    m->fv_axis = 1;
+    return &fa;
 }
 
 template <class T>
 void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamma, double cfl, int64_t nsteps,
                   void* dt_hist, hipStream_t s) {
-    const FvGeo<T>& g = fv_geometry<T>(m, s);
+    int ty = m->euler_ty, L = m->euler_L;
+    const bool march = m->euler_variant != 0, chosen = m->euler_variant < 0;
+    const FvAxis<T>* axis = nullptr;
+    if (march && euler_tile_supported(m, chosen ? (sizeof(T) == 4 ? 8 : 4) : ty)) axis = fv_axis<T>(m, s);
+    if (chosen) euler_tile_shape(m, axis != nullptr, ty, L);
+    const bool tile = march && euler_tile_supported(m, ty);
+    const FvGeo<T>* faces = axis ? nullptr : &fv_geometry<T>(m, s);
     Bits<T>* slots = (Bits<T>*)pool_alloc(m->ctx, 3 * kDtSet * sizeof(Bits<T>), s);
     try {
         const dim3 block(64, 4, 1);
@@ -502,11 +948,11 @@ void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamm
         EIn<T> in{};
         EOut<T> out{};
         for (int k = 0; k < 5; ++k) in.u[k] = (const T*)a[k];
-        euler_dt_k<T><<<grid, block, 0, s>>>(g, in, T(gamma), slots);
+        if (axis) launch_euler_dt_axis<T>(m, *axis, in, T(gamma), slots, s);
+        else euler_dt_k<T><<<grid, block, 0, s>>>(*faces, in, T(gamma), slots);
         CFD_HIP(hipGetLastError());
-        const int ty = m->euler_ty, L = m->euler_L;
         const int nzt = int((m->Z + 63) / 64), nyt = int((m->Y + ty - 1) / ty);
-        CFD_REQUIRE(m->euler_variant == 0 || m->Y * (m->Z + 1) * int64_t(sizeof(T)) < (int64_t(1) << 32),
+        CFD_REQUIRE(!march || m->Y * (m->Z + 1) * int64_t(sizeof(T)) < (int64_t(1) << 32),
                     "Euler march: a plane of this mesh exceeds 32-bit byte offsets (use the per-thread form)");
         const int64_t nwg = int64_t(nzt) * nyt * ((m->X + L - 1) / L);
         CFD_REQUIRE(nwg < (int64_t(1) << 31), "euler march grid too large");
@@ -520,15 +966,20 @@ void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamm
             Bits<T>* cur = slots + (st % 3) * kDtSet;
             Bits<T>* nxt = slots + ((st + 1) % 3) * kDtSet;
             Bits<T>* rst = slots + ((st + 2) % 3) * kDtSet;
-            if (m->euler_variant == 0) {
-                euler_step_k<T><<<grid, block, 0, s>>>(g, in, out, T(gamma), T(cfl), cur, nxt, rst, (T*)dt_hist,
+            if (!march) {
+                euler_step_k<T><<<grid, block, 0, s>>>(*faces, in, out, T(gamma), T(cfl), cur, nxt, rst, (T*)dt_hist,
                                                        st);
+                continue;
+            }
+            if (tile) {
+                launch_euler_tile<T>(m, faces, axis, in, out, T(gamma), T(cfl), EulerSlots<T>{cur, nxt, rst},
+                                     (T*)dt_hist, st, ty, L, s);
                 continue;
             }
             const dim3 mgrid{unsigned(nwg), 1u, 1u};
 #define CFD_EULER_MARCH(TYV)                                                                                    \
-    euler_march_k<T, TYV><<<mgrid, dim3(64, TYV), 0, s>>>(g, in, out, T(gamma), T(cfl), cur, nxt, rst, (T*)dt_hist, \
-                                                         st, L, nzt, nyt)
+    euler_march_k<T, TYV><<<mgrid, dim3(64, TYV), 0, s>>>(*faces, in, out, T(gamma), T(cfl), cur, nxt, rst,     \
+                                                         (T*)dt_hist, st, L, nzt, nyt)
             switch (ty) {
                 case 2: CFD_EULER_MARCH(2); break;
                 case 4: CFD_EULER_MARCH(4); break;

@@ -675,7 +675,8 @@ int cfd_mesh_destroy(cfd_mesh_t mesh) {
         if (mesh->dev_block) pool_free(mesh->ctx, mesh->dev_block, nullptr);
         if (mesh->lat_block) pool_free(mesh->ctx, mesh->lat_block, nullptr);
         if (mesh->fv_block) pool_free(mesh->ctx, mesh->fv_block, nullptr);
-        if (mesh->dev_block || mesh->fv_block) CFD_HIP(hipStreamSynchronize(nullptr));
+        if (mesh->fa_block) pool_free(mesh->ctx, mesh->fa_block, nullptr);
+        if (mesh->dev_block || mesh->fv_block || mesh->fa_block) CFD_HIP(hipStreamSynchronize(nullptr));
         delete mesh;
     });
 }

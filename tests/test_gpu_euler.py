@@ -162,3 +162,60 @@ def test_sod_full_size_properties(hip_ctx):
     rho_ex, _, _ = riemann_exact.sod(x_c, t)
     assert np.mean(np.abs(rho_x - rho_ex)) < 0.01
     gm.close()
+
+
+# Cells-in-a-row tiles of the march: planes that fill a tile, end inside one or
+# need several, rows of one cell and of half a tile, chunks of one plane to
+# more than the mesh; on perturbed (face arrays), decimal (layer widths) and
+# dyadic (constants) meshes.
+TILE_CASES = [((9, 16, 32), (1, 2, 1)), ((7, 13, 20), (1, 2, 3)), ((6, 1, 1), (1, 4, 2)), ((5, 130, 1), (1, 2, 4)),
+              ((12, 9, 64), (1, 2, 16)), ((4, 11, 128), (1, 4, 2)), ((3, 9, 200), (1, 8, 5)), ((17, 24, 23), None),
+              ((40, 12, 300), None)]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["perturbed", "decimal", "dyadic"])
+@pytest.mark.parametrize("n,shape", TILE_CASES, ids=lambda v: "x".join(map(str, v)) if v else "auto")
+def test_euler_tiles(hip_ctx, oracle_lib, n, shape, kind, dtype):
+    if dtype == np.float64 and shape and shape[1] == 8:
+        shape = (1, 4, shape[2])
+    d = (0.125, 0.25, 0.125) if kind == "dyadic" else (0.1, 0.07, 0.09)
+    off = workloads.perturbed_vertex_offsets(*n, *d, seed=4, frac=0.2) if kind == "perturbed" else None
+    om = oracle_lib.OracleMesh(*n, *d, dtype=dtype, perturb=off)
+    rng = np.random.default_rng(9)
+    U0 = np.empty((5, om.N), dtype=dtype)
+    U0[0] = 1.0 + 0.5 * rng.random(om.N)
+    U0[1:4] = 0.2 * rng.standard_normal((3, om.N))
+    U0[4] = 3.0 + rng.random(om.N)
+    ref, ref_dt = om.euler_run(U0, 1.4, 0.3, 5)
+    got, got_dt = _gpu_run(hip_ctx, n, d, off, dtype, U0, 1.4, 0.3, 5, shape)
+    assert np.all(np.isfinite(ref))
+    assert np.array_equal(got_dt, ref_dt)
+    assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("kind", ["decimal", "dyadic"])
+def test_euler_axis_aligned_equals_face_arrays(hip_ctx, kind):
+    """Axis-aligned geometry against the face arrays of the same mesh (forced
+    general), with infinite and NaN cells: the same values, NaN in the same
+    places."""
+    from cfdarcov2_amd import capi
+    n, d = (14, 9, 12), (0.125,) * 3 if kind == "dyadic" else (0.1, 0.07, 0.09)
+    N = n[0] * n[1] * n[2]
+    rng = np.random.default_rng(1)
+    for special in (None, np.inf, -np.inf, np.nan):
+        for field in range(5) if special is not None else (0,):
+            U0 = np.stack([1.0 + 0.3 * rng.random(N), *(0.2 * rng.standard_normal((3, N))), 3.0 + rng.random(N)])
+            if special is not None:
+                U0[field, rng.integers(N, size=3)] = special
+            res = []
+            for force in (False, True):
+                gm = capi.HexMesh(hip_ctx, *n, *d, dtype="f64", force_general=force)
+                A = [torch.from_numpy(U0[k].copy()).cuda() for k in range(5)]
+                B = [torch.empty_like(a) for a in A]
+                hist = torch.empty(3, dtype=torch.float64, device="cuda")
+                out = gm.euler_run(A, B, 1.4, 0.3, 3, hist)
+                res.append([t.cpu().numpy() for t in out] + [hist.cpu().numpy()])
+                gm.close()
+            for k, (x, y) in enumerate(zip(*res)):
+                assert np.array_equal(x, y, equal_nan=True), (special, field, k)
