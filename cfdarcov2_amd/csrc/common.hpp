@@ -145,22 +145,29 @@ struct UConn {
 
 // Device geometry of an unstructured hex mesh, cells and faces in the mesh's
 // (reordered) numbering.  Per (cell, local face) arrays are fc-major (6 x N).
+// A face's normal and area are one record of four values, so a cell gathers
+// them with one or two 16-byte loads instead of four 4- or 8-byte ones.
 template <class T> struct UnstructGeo {
     int64_t N, F;
     const int32_t* nbr;    // neighbour across the face, -1 on the boundary
-    const int32_t* face;   // face id
-    const int8_t* osign;   // outward normal of the face = osign * its normal
-    const T* fn[3];        // per face: normal (first three vertices)
-    const T* area;
-    const T* alpha;        // alpha_d (the same from both cells)
+    const int32_t* face;   // face id; the top bit is set where the cell's outward normal is minus the face's
+    const T* rec;          // per face: normal (first three vertices), area
+    const T* alpha;        // per face: alpha_d (the same from both cells)
     const T* vol;          // per cell
     const T* len;          // per (fc, cell), fc-major: centre-to-face distance
     // the Rusanov stepper's geometry, built on its first use (null before):
     // per face the +axis unit vector-area normal and area, per cell the volume
-    const T* sn[3] = {nullptr, nullptr, nullptr};
-    const T* sa = nullptr;
+    const T* srec = nullptr;
     const T* svol = nullptr;
 };
+
+constexpr int32_t kFaceId = 0x7fffffff;  // the face id without its sign bit
+
+// record f of an array of four values per face
+template <class T> struct FaceRec { typedef T type __attribute__((ext_vector_type(4), aligned(16))); };
+template <class T> __device__ inline typename FaceRec<T>::type face_rec(const T* rec, int32_t f) {
+    return reinterpret_cast<const typename FaceRec<T>::type*>(rec)[f & kFaceId];
+}
 
 }  // namespace cfd
 
@@ -229,6 +236,7 @@ struct cfd_mesh_s {
     bool unstructured = false;
     cfd::UConn uconn;
     std::vector<int64_t> cell_perm, cell_iperm, face_perm;
+    std::vector<int64_t> face_dev;  // caller's face of each place in the device arrays
     cfd::UnstructGeo<float> uu32{};
     cfd::UnstructGeo<double> uu64{};
     // Euler stepper geometry (device block allocated on first use)

@@ -1013,16 +1013,20 @@ void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamm
 // connectivity.
 // ---------------------------------------------------------------------------
 
-__device__ inline int64_t ucell() { return int64_t(blockIdx.x) * 256 + threadIdx.y * 64 + threadIdx.x; }
+// each XCD (round-robin dispatch) takes a contiguous run of blocks
+__device__ inline int64_t ucell() {
+    const int b = int((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+    return int64_t(b) * 256 + threadIdx.y * 64 + threadIdx.x;
+}
 
 // V / sum over fc = 0..5 of A_f (|u.n_f| + a), the faces through the ids
 template <class T> __device__ inline T ulocal_dt(const UnstructGeo<T>& g, int64_t i, const Prim<T>& q) {
     T s = T(0);
 #pragma unroll
     for (int fc = 0; fc < 6; ++fc) {
-        const int32_t f = g.face[int64_t(fc) * g.N + i];
-        const T un = un_of(q.ux, q.uy, q.uz, g.sn[0][f], g.sn[1][f], g.sn[2][f]);
-        s = fmul_add(g.sa[f], fabs(un) + q.a, s);
+        const auto r = face_rec(g.srec, g.face[int64_t(fc) * g.N + i]);
+        const T un = un_of(q.ux, q.uy, q.uz, r[0], r[1], r[2]);
+        s = fmul_add(r[3], fabs(un) + q.a, s);
     }
     return g.svol[i] / s;
 }
@@ -1076,10 +1080,9 @@ __global__ void __launch_bounds__(256) ueuler_step_k(UnstructGeo<T> g, EIn<T> in
                     for (int k = 0; k < 5; ++k) Un[k] = in.u[k][nb];
                 }
                 const Prim<T> qn = prim(gamma, Un);
-                const int32_t f = g.face[k6];
-                const T nx = g.sn[0][f], ny = g.sn[1][f], nz = g.sn[2][f], A = g.sa[f];
-                if (side == 1) rusanov(Ui, qi, Un, qn, nx, ny, nz, A, Gp[side]);
-                else rusanov(Un, qn, Ui, qi, nx, ny, nz, A, Gp[side]);
+                const auto r = face_rec(g.srec, g.face[k6]);
+                if (side == 1) rusanov<T>(Ui, qi, Un, qn, r[0], r[1], r[2], r[3], Gp[side]);
+                else rusanov<T>(Un, qn, Ui, qi, r[0], r[1], r[2], r[3], Gp[side]);
             }
 #pragma unroll
             for (int k = 0; k < 5; ++k) {
@@ -1118,8 +1121,8 @@ template <class T> const UnstructGeo<T>& ufv_geometry(cfd_mesh_s* m, hipStream_t
     const int64_t N = c.N, F = c.F;
     std::vector<T> host(size_t(4 * F + N));
     for (int64_t n = 0; n < F; ++n) {
-        const int64_t f = m->face_perm[n];
-        for (int k = 0; k < 4; ++k) host[size_t(k * F + n)] = sv[size_t(k * F + f)];
+        const int64_t f = m->face_dev[n];
+        for (int k = 0; k < 4; ++k) host[size_t(4 * n + k)] = sv[size_t(k * F + f)];
     }
     for (int64_t n = 0; n < N; ++n) host[size_t(4 * F + n)] = svol[size_t(m->cell_perm[n])];
     const int64_t bytes = int64_t(host.size() * sizeof(T));
@@ -1131,8 +1134,7 @@ template <class T> const UnstructGeo<T>& ufv_geometry(cfd_mesh_s* m, hipStream_t
         CFD_HIP(e);
     }
     const T* d = static_cast<const T*>(dev);
-    for (int k = 0; k < 3; ++k) u.sn[k] = d + k * F;
-    u.sa = d + 3 * F;
+    u.srec = d;
     u.svol = d + 4 * F;
     m->fv_block = dev;
     m->fv_bytes = bytes;
@@ -1148,7 +1150,7 @@ void launch_ueuler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gam
     Bits<T>* slots = (Bits<T>*)pool_alloc(m->ctx, 3 * kDtSet * sizeof(Bits<T>), s);
     try {
         const dim3 block(64, 4, 1);
-        const dim3 grid(unsigned((m->N + 255) / 256));
+        const dim3 grid(unsigned((m->N + 2047) / 2048 * 8));
         const Bits<T> inf = sizeof(T) == 4 ? Bits<T>(0x7f800000u) : Bits<T>(0x7ff0000000000000ull);
         fill_bits_k<Bits<T>><<<3 * kDtSet / 256, 256, 0, s>>>(slots, 3 * kDtSet, inf);
         EIn<T> in{};

@@ -4,9 +4,10 @@
 //
 // Device layout (cells and faces in the mesh's reordered numbering):
 //   per (local face fc, cell), fc-major, int32: the neighbour across the face
-//   (-1 on the boundary) and the face id; int8: the sign that turns the face
-//   normal into the cell's outward normal;
-//   per face: the normal (first three vertices), area and alpha_d;
+//   (-1 on the boundary) and the face id, its top bit set where the face
+//   normal points into the cell;
+//   per face: the normal (first three vertices) and area as one record of
+//   four values, and alpha_d;
 //   per cell: the volume; per (fc, cell): the centre-to-face distance (the
 //   stabilisation's upwind extrapolation).
 // Each cell reads its own six faces and neighbours and writes only itself:
@@ -16,6 +17,14 @@
 // the reference semantics bit for bit whatever the numbering.  Reverse
 // Cuthill-McKee numbering keeps the six neighbours of a cell, and so the
 // gathered values, within a few cache lines of the cell's own.
+//
+// Bound by the gathers: 96^3 FP64 moves 186 algorithmic bytes per cell and
+// heat step (ids, records, alpha, volume, state) at 6.5 TB/s from the
+// last-level cache.  us/step at 96^3, heat / acoustic, FP64 (FP32): blocks in
+// launch order, faces by their lowest cell, one array per component 43.6 / 86.6
+// (26.2 / 55.2); contiguous runs of blocks per XCD, so a face's second gather
+// hits that L2, 29.6 / 64.1 (20.9 / 45.3); faces by local index and cell,
+// normal and area in one record 25.4 / 59.0 (16.5 / 37.2).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,31 +40,43 @@ namespace {
 
 constexpr int kUBlock = 256;
 
-template <class T> __device__ inline T ugauss(const UnstructGeo<T>& g, const T (&fv)[6], const int32_t (&f)[6],
-                                              const int8_t (&sg)[6], int d, int64_t i, bool axis) {
+// The thread's cell.  Each XCD (round-robin dispatch) takes a contiguous run
+// of blocks, so cells a matrix bandwidth apart meet in one L2.
+__device__ inline int64_t ucell_of_thread() {
+    const int b = int((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+    return int64_t(b) * kUBlock + threadIdx.x;
+}
+
+// a cell's six faces: neighbours, face ids (with the sign bit), normal and area
+template <class T> struct UFaces {
+    int32_t nb[6], f[6];
+    typename FaceRec<T>::type r[6];
+};
+template <class T> __device__ inline void uload(const UnstructGeo<T>& g, int64_t i, UFaces<T>& c) {
+#pragma unroll
+    for (int fc = 0; fc < 6; ++fc) {
+        const int64_t k = int64_t(fc) * g.N + i;
+        c.nb[fc] = g.nbr[k];
+        c.f[fc] = g.face[k];
+    }
+#pragma unroll
+    for (int fc = 0; fc < 6; ++fc) c.r[fc] = face_rec(g.rec, c.f[fc]);
+}
+
+template <class T> __device__ inline T ugauss(const UnstructGeo<T>& g, const T (&fv)[6], const UFaces<T>& c, int d,
+                                              int64_t i, bool axis) {
     // sum over fc = 0..5 of (fv * n) * area from 0, then / V; n is the axis
     // normal (+n on fc 2, 3, -n on the others) or the outward normal
     T acc = T(0);
 #pragma unroll
     for (int fc = 0; fc < 6; ++fc) {
-        const T n = g.fn[d][f[fc]];
-        const bool neg = axis ? !(fc == 2 || fc == 3) : sg[fc] < 0;
+        const T n = d == 0 ? c.r[fc][0] : d == 1 ? c.r[fc][1] : c.r[fc][2];
+        const bool neg = axis ? !(fc == 2 || fc == 3) : c.f[fc] < 0;
         T t = fv[fc] * (neg ? -n : n);
-        t = t * g.area[f[fc]];
+        t = t * c.r[fc][3];
         acc = acc + t;
     }
     return acc / g.vol[i];
-}
-
-template <class T> __device__ inline void uload(const UnstructGeo<T>& g, int64_t i, int32_t (&nb)[6], int32_t (&f)[6],
-                                                int8_t (&sg)[6]) {
-#pragma unroll
-    for (int fc = 0; fc < 6; ++fc) {
-        const int64_t k = int64_t(fc) * g.N + i;
-        nb[fc] = g.nbr[k];
-        f[fc] = g.face[k];
-        sg[fc] = g.osign[k];
-    }
 }
 
 }  // namespace
@@ -66,44 +87,42 @@ template <class T> __device__ inline void uload(const UnstructGeo<T>& g, int64_t
 template <class T>
 __global__ void __launch_bounds__(kUBlock) ugrad_k(UnstructGeo<T> g, const T* __restrict__ phi, T* __restrict__ out,
                                                    int mask, int wall) {
-    const int64_t i = int64_t(blockIdx.x) * kUBlock + threadIdx.x;
+    const int64_t i = ucell_of_thread();
     if (i >= g.N) return;
-    int32_t nb[6], f[6];
-    int8_t sg[6];
-    uload(g, i, nb, f, sg);
+    UFaces<T> c;
+    uload(g, i, c);
     const T pc = phi[i];
     T fv[6];
 #pragma unroll
     for (int fc = 0; fc < 6; ++fc) {
-        const bool bnd = nb[fc] < 0;
-        fv[fc] = (wall >= 0 && bnd && (fc >> 1) == 2 - wall) ? T(0) : (pc + (bnd ? pc : phi[nb[fc]])) * T(0.5);
+        const bool bnd = c.nb[fc] < 0;
+        fv[fc] = (wall >= 0 && bnd && (fc >> 1) == 2 - wall) ? T(0) : (pc + (bnd ? pc : phi[c.nb[fc]])) * T(0.5);
     }
     T res = T(0);
     for (int d = 0; d < 3; ++d)
-        if (mask & (1 << d)) res = res + ugauss(g, fv, f, sg, d, i, false);
+        if (mask & (1 << d)) res = res + ugauss(g, fv, c, d, i, false);
     out[i] = res;
 }
 
 // Grad2Var: (-phi_c + phi_nb) * alpha_d, axis-normal Gauss sum per selected axis.
 template <class T> __device__ inline T ulapl_cell(const UnstructGeo<T>& g, const T* __restrict__ phi, int64_t i,
                                                   int mask) {
-    int32_t nb[6], f[6];
-    int8_t sg[6];
-    uload(g, i, nb, f, sg);
+    UFaces<T> c;
+    uload(g, i, c);
     const T pc = phi[i];
     T fv[6];
 #pragma unroll
-    for (int fc = 0; fc < 6; ++fc) fv[fc] = (-pc + (nb[fc] < 0 ? pc : phi[nb[fc]])) * g.alpha[f[fc]];
+    for (int fc = 0; fc < 6; ++fc) fv[fc] = (-pc + (c.nb[fc] < 0 ? pc : phi[c.nb[fc]])) * g.alpha[c.f[fc] & kFaceId];
     T res = T(0);
     for (int d = 0; d < 3; ++d)
-        if (mask & (1 << d)) res = res + ugauss(g, fv, f, sg, d, i, true);
+        if (mask & (1 << d)) res = res + ugauss(g, fv, c, d, i, true);
     return res;
 }
 
 template <class T>
 __global__ void __launch_bounds__(kUBlock) ulapl_k(UnstructGeo<T> g, const T* __restrict__ phi, T* __restrict__ out,
                                                    int mask) {
-    const int64_t i = int64_t(blockIdx.x) * kUBlock + threadIdx.x;
+    const int64_t i = ucell_of_thread();
     if (i >= g.N) return;
     out[i] = ulapl_cell(g, phi, i, mask);
 }
@@ -112,7 +131,7 @@ __global__ void __launch_bounds__(kUBlock) ulapl_k(UnstructGeo<T> g, const T* __
 template <class T>
 __global__ void __launch_bounds__(kUBlock) uheat_k(UnstructGeo<T> g, const T* __restrict__ Tin, T* __restrict__ Tout,
                                                    T alpha, const T* __restrict__ alpha_f, T dt) {
-    const int64_t i = int64_t(blockIdx.x) * kUBlock + threadIdx.x;
+    const int64_t i = ucell_of_thread();
     if (i >= g.N) return;
     const T L = ulapl_cell(g, Tin, i, 7);
     const T k = alpha_f ? alpha_f[i] : alpha;
@@ -127,7 +146,7 @@ template <class T> const UnstructGeo<T>& ugeo_u(const cfd_mesh_s* m) {
 template <class T> UnstructGeo<T>& ugeo_u(cfd_mesh_s* m) {
     if constexpr (sizeof(T) == 4) return m->uu32; else return m->uu64;
 }
-dim3 ugrid(int64_t N) { return dim3(unsigned((N + kUBlock - 1) / kUBlock)); }
+dim3 ugrid(int64_t N) { return dim3(unsigned((N + 8 * kUBlock - 1) / (8 * kUBlock) * 8)); }
 
 }  // namespace
 
@@ -145,18 +164,17 @@ template <class T> void launch_ulapl(const cfd_mesh_s* m, const void* phi, void*
 template <class T>
 __global__ void __launch_bounds__(kUBlock) ustab_grad_k(UnstructGeo<T> g, const T* __restrict__ phi,
                                                         T* __restrict__ gx, T* __restrict__ gy, T* __restrict__ gz) {
-    const int64_t i = int64_t(blockIdx.x) * kUBlock + threadIdx.x;
+    const int64_t i = ucell_of_thread();
     if (i >= g.N) return;
-    int32_t nb[6], f[6];
-    int8_t sg[6];
-    uload(g, i, nb, f, sg);
+    UFaces<T> c;
+    uload(g, i, c);
     const T pc = phi[i];
     T fv[6];
 #pragma unroll
-    for (int fc = 0; fc < 6; ++fc) fv[fc] = (pc + (nb[fc] < 0 ? pc : phi[nb[fc]])) * T(0.5);
-    gx[i] = ugauss(g, fv, f, sg, 0, i, false);
-    gy[i] = ugauss(g, fv, f, sg, 1, i, false);
-    gz[i] = ugauss(g, fv, f, sg, 2, i, false);
+    for (int fc = 0; fc < 6; ++fc) fv[fc] = (pc + (c.nb[fc] < 0 ? pc : phi[c.nb[fc]])) * T(0.5);
+    gx[i] = ugauss(g, fv, c, 0, i, false);
+    gy[i] = ugauss(g, fv, c, 1, i, false);
+    gz[i] = ugauss(g, fv, c, 2, i, false);
 }
 
 // StabVar, second stage (include/grad_utils.hpp:38-80, src/fvm3d.cpp:915-936):
@@ -169,17 +187,17 @@ template <class T>
 __global__ void __launch_bounds__(kUBlock) ustab_k(UnstructGeo<T> g, const T* __restrict__ phi,
                                                    const T* __restrict__ gx, const T* __restrict__ gy,
                                                    const T* __restrict__ gz, T* __restrict__ out, int mask) {
-    const int64_t i = int64_t(blockIdx.x) * kUBlock + threadIdx.x;
+    const int64_t i = ucell_of_thread();
     if (i >= g.N) return;
-    int32_t nb[6], f[6];
-    int8_t sg[6];
-    uload(g, i, nb, f, sg);
+    UFaces<T> c;
+    uload(g, i, c);
     const T* const gd[3] = {gx, gy, gz};
-    auto upwind = [&](int d, int64_t c, int fc) {
-        const int64_t k = int64_t(fc) * g.N + c;
-        const T n = g.fn[d][g.face[k]];
-        const T na = g.osign[k] < 0 ? -n : n;
-        return phi[c] + g.len[k] * gd[d][c] * na;
+    auto upwind = [&](int d, int64_t j, int fc) {
+        const int64_t k = int64_t(fc) * g.N + j;
+        const int32_t f = g.face[k];
+        const T n = g.rec[4 * int64_t(f & kFaceId) + d];
+        const T na = f < 0 ? -n : n;
+        return phi[j] + g.len[k] * gd[d][j] * na;
     };
     T res = T(0);
     for (int d = 0; d < 3; ++d) {
@@ -187,12 +205,12 @@ __global__ void __launch_bounds__(kUBlock) ustab_k(UnstructGeo<T> g, const T* __
         T fv[6];
 #pragma unroll
         for (int fc = 0; fc < 6; ++fc) {
-            const int64_t c = nb[fc] < 0 ? i : int64_t(nb[fc]);
+            const int64_t j = c.nb[fc] < 0 ? i : int64_t(c.nb[fc]);
             const T own = upwind(d, i, fc);
-            const T col = upwind(d, c, fc ^ 1);
+            const T col = upwind(d, j, fc ^ 1);
             fv[fc] = T(0.5) * (own - col);
         }
-        res = res + ugauss(g, fv, f, sg, d, i, true);
+        res = res + ugauss(g, fv, c, d, i, true);
     }
     out[i] = res;
 }
@@ -209,20 +227,19 @@ __global__ void __launch_bounds__(kUBlock) uwave_vel_k(UnstructGeo<T> g, const T
                                                        const T* __restrict__ u, const T* __restrict__ v,
                                                        const T* __restrict__ w, T* __restrict__ uo,
                                                        T* __restrict__ vo, T* __restrict__ wo, T dt) {
-    const int64_t i = int64_t(blockIdx.x) * kUBlock + threadIdx.x;
+    const int64_t i = ucell_of_thread();
     if (i >= g.N) return;
-    int32_t nb[6], f[6];
-    int8_t sg[6];
-    uload(g, i, nb, f, sg);
+    UFaces<T> c;
+    uload(g, i, c);
     const T pc = p[i];
     T fv[6];
 #pragma unroll
-    for (int fc = 0; fc < 6; ++fc) fv[fc] = (pc + (nb[fc] < 0 ? pc : p[nb[fc]])) * T(0.5);
+    for (int fc = 0; fc < 6; ++fc) fv[fc] = (pc + (c.nb[fc] < 0 ? pc : p[c.nb[fc]])) * T(0.5);
     const T* const vin[3] = {u, v, w};
     T* const vout[3] = {uo, vo, wo};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const T gd = T(0) + ugauss(g, fv, f, sg, d, i, false);
+        const T gd = T(0) + ugauss(g, fv, c, d, i, false);
         vout[d][i] = dt * (-gd) + vin[d][i];
     }
 }
@@ -232,11 +249,10 @@ __global__ void __launch_bounds__(kUBlock) uwave_pres_k(UnstructGeo<T> g, const 
                                                         const T* __restrict__ u, const T* __restrict__ v,
                                                         const T* __restrict__ w, T* __restrict__ po, T K,
                                                         const T* __restrict__ Kf, T dt) {
-    const int64_t i = int64_t(blockIdx.x) * kUBlock + threadIdx.x;
+    const int64_t i = ucell_of_thread();
     if (i >= g.N) return;
-    int32_t nb[6], f[6];
-    int8_t sg[6];
-    uload(g, i, nb, f, sg);
+    UFaces<T> c;
+    uload(g, i, c);
     const T* const vel[3] = {u, v, w};
     T div[3];
 #pragma unroll
@@ -246,10 +262,10 @@ __global__ void __launch_bounds__(kUBlock) uwave_pres_k(UnstructGeo<T> g, const 
         T fv[6];
 #pragma unroll
         for (int fc = 0; fc < 6; ++fc) {
-            const bool bnd = nb[fc] < 0;
-            fv[fc] = (bnd && (fc >> 1) == 2 - d) ? T(0) : (qc + (bnd ? qc : q[nb[fc]])) * T(0.5);
+            const bool bnd = c.nb[fc] < 0;
+            fv[fc] = (bnd && (fc >> 1) == 2 - d) ? T(0) : (qc + (bnd ? qc : q[c.nb[fc]])) * T(0.5);
         }
-        div[d] = T(0) + ugauss(g, fv, f, sg, d, i, false);
+        div[d] = T(0) + ugauss(g, fv, c, d, i, false);
     }
     const T S = (div[0] + div[1]) + div[2];
     const T k = Kf ? Kf[i] : K;
@@ -294,9 +310,9 @@ void launch_uheat(const cfd_mesh_s* m, void* Ta, void* Tb, double alpha, const v
     }
 }
 
-// Geometry, numbering and upload of an unstructured mesh.  Device block:
-// nbr (6N int32), face (6N int32), then per face fn (3F), area (F), alpha (F),
-// then vol (N), len (6N), then osign (6N int8).
+// Geometry, numbering and upload of an unstructured mesh.  Device block: the
+// faces' records (4F), alpha (F), vol (N), len (6N), then nbr and face (6N
+// int32 each).
 template <class T> void create_unstructured(cfd_mesh_s* m, int reorder) {
     const UConn& c = m->uconn;
     check_uconn(c);
@@ -312,41 +328,74 @@ template <class T> void create_unstructured(cfd_mesh_s* m, int reorder) {
     m->cell_iperm.assign(N, 0);
     for (int64_t n = 0; n < N; ++n) m->cell_iperm[m->cell_perm[n]] = n;
     m->face_perm = face_order(c, m->cell_iperm);
-    std::vector<int64_t> face_iperm(F);
-    for (int64_t n = 0; n < F; ++n) face_iperm[m->face_perm[n]] = n;
-
-    const size_t ib = 6 * size_t(N) * sizeof(int32_t);
-    const size_t tb = (5 * size_t(F) + 7 * size_t(N)) * sizeof(T);
-    const size_t sb = 6 * size_t(N);
-    const int64_t bytes = int64_t(2 * ib + tb + sb);
-    std::vector<char> host(static_cast<size_t>(bytes));
-    int32_t* nbr = reinterpret_cast<int32_t*>(host.data());
-    int32_t* fid = nbr + 6 * N;
-    T* tv = reinterpret_cast<T*>(host.data() + 2 * ib);
-    int8_t* sgn = reinterpret_cast<int8_t*>(host.data() + 2 * ib + tb);
+    // The device arrays hold the faces by the local index fc they have in
+    // their lowest cell, and by that cell within one fc: consecutive cells
+    // then find face fc at consecutive places (a wave's 64 FP64 values in 4
+    // cache lines; in the order of face_perm, where a cell's own faces lie
+    // side by side, in 12).
+    // per (new cell, fc): the face and the new neighbour, gathered once
+    struct Side { int32_t f, nb; };
+    std::vector<Side> side(size_t(6 * N));
+#pragma omp parallel for schedule(static)
     for (int64_t n = 0; n < N; ++n) {
         const int64_t i = m->cell_perm[n];
         for (int fc = 0; fc < 6; ++fc) {
             const int64_t f = c.cell_faces[6 * i + fc];
             const int64_t a = c.face_cells[2 * f], b = c.face_cells[2 * f + 1];
             const int64_t other = b < 0 ? -1 : (a == i ? b : a);
-            nbr[fc * N + n] = other < 0 ? -1 : int32_t(m->cell_iperm[other]);
-            fid[fc * N + n] = int32_t(face_iperm[f]);
-            sgn[fc * N + n] = g.out_sign[6 * i + fc];
+            side[size_t(6 * n + fc)] = {int32_t(f), other < 0 ? -1 : int32_t(m->cell_iperm[other])};
         }
     }
+    std::vector<int32_t> place(size_t(F), -1);  // of each of the caller's faces in the device arrays
+    m->face_dev.clear();
+    m->face_dev.reserve(F);
+    for (int fc = 0; fc < 6; ++fc)
+        for (int64_t n = 0; n < N; ++n) {
+            const Side sd = side[size_t(6 * n + fc)];
+            if (sd.nb >= 0 && sd.nb < n) continue;
+            if (place[size_t(sd.f)] >= 0) continue;
+            place[size_t(sd.f)] = int32_t(m->face_dev.size());
+            m->face_dev.push_back(sd.f);
+        }
+    for (int64_t f = 0; f < F; ++f)  // faces that their lowest cell does not list
+        if (place[size_t(f)] < 0) {
+            place[size_t(f)] = int32_t(m->face_dev.size());
+            m->face_dev.push_back(f);
+        }
+
+    const size_t ib = 6 * size_t(N) * sizeof(int32_t);
+    const size_t tb = (5 * size_t(F) + 7 * size_t(N)) * sizeof(T);
+    const int64_t bytes = int64_t(2 * ib + tb);
+    std::vector<char> host(static_cast<size_t>(bytes));
+    T* tv = reinterpret_cast<T*>(host.data());
+    int32_t* nbr = reinterpret_cast<int32_t*>(host.data() + tb);
+    int32_t* fid = nbr + 6 * N;
+#pragma omp parallel for schedule(static)
+    for (int64_t n = 0; n < N; ++n) {
+        const int64_t i = m->cell_perm[n];
+        for (int fc = 0; fc < 6; ++fc) {
+            const Side sd = side[size_t(6 * n + fc)];
+            nbr[fc * N + n] = sd.nb;
+            fid[fc * N + n] = place[size_t(sd.f)] | (g.out_sign[6 * i + fc] < 0 ? ~kFaceId : 0);
+        }
+    }
+#pragma omp parallel for schedule(static)
     for (int64_t n = 0; n < F; ++n) {
-        const int64_t f = m->face_perm[n];
-        tv[n] = g.fnx[f];
-        tv[F + n] = g.fny[f];
-        tv[2 * F + n] = g.fnz[f];
-        tv[3 * F + n] = g.farea[f];
+        const int64_t f = m->face_dev[n];
+        T* r = tv + 4 * n;
+        r[0] = g.fnx[f];
+        r[1] = g.fny[f];
+        r[2] = g.fnz[f];
+        r[3] = g.farea[f];
         tv[4 * F + n] = g.falpha[f];
     }
-    for (int64_t n = 0; n < N; ++n) tv[5 * F + n] = g.vol[m->cell_perm[n]];
     T* lv = tv + 5 * F + N;
-    for (int64_t n = 0; n < N; ++n)
-        for (int fc = 0; fc < 6; ++fc) lv[fc * N + n] = g.len[6 * m->cell_perm[n] + fc];
+#pragma omp parallel for schedule(static)
+    for (int64_t n = 0; n < N; ++n) {
+        const int64_t i = m->cell_perm[n];
+        tv[5 * F + n] = g.vol[i];
+        for (int fc = 0; fc < 6; ++fc) lv[fc * N + n] = g.len[6 * i + fc];
+    }
 
     hipStream_t s = nullptr;
     m->dev_block = pool_alloc(m->ctx, bytes, s);
@@ -357,15 +406,13 @@ template <class T> void create_unstructured(cfd_mesh_s* m, int reorder) {
     UnstructGeo<T>& u = ugeo_u<T>(m);
     u.N = N;
     u.F = F;
-    u.nbr = reinterpret_cast<const int32_t*>(d);
-    u.face = reinterpret_cast<const int32_t*>(d + ib);
-    const T* dt = reinterpret_cast<const T*>(d + 2 * ib);
-    for (int k = 0; k < 3; ++k) u.fn[k] = dt + k * F;
-    u.area = dt + 3 * F;
+    const T* dt = reinterpret_cast<const T*>(d);
+    u.rec = dt;
     u.alpha = dt + 4 * F;
     u.vol = dt + 5 * F;
     u.len = dt + 5 * F + N;
-    u.osign = reinterpret_cast<const int8_t*>(d + 2 * ib + tb);
+    u.nbr = reinterpret_cast<const int32_t*>(d + tb);
+    u.face = u.nbr + 6 * N;
 }
 
 // Reference-layout tables of an unstructured mesh (N x 6 column-major), cells
