@@ -23,7 +23,9 @@ wave_star_aux_k(UniformGeo<T> g, const T* __restrict__ p, const T* __restrict__ 
                 const T* __restrict__ w, T* __restrict__ po, T* __restrict__ uo, T* __restrict__ vo,
                 T* __restrict__ wo, T K, const T* __restrict__ Kf, T dt, star::Plan pl, star::SensorSet sens,
                 star::WaveAux<T> aux) {
-    star::wave_cells<T, W, PW, KF, MODE>(g, p, u, v, w, po, uo, vo, wo, K, Kf, dt, pl, &sens, &aux);
+    star::Place at;
+    if (star::place<W>(pl, at))
+        star::wave_cells<T, W, PW, KF, MODE>(g, p, u, v, w, po, uo, vo, wo, K, Kf, dt, pl, at, &sens, &aux);
 }
 
 star::SensorSet sensor_set(const cfd_mesh_s* m, const SensorList& l) {

@@ -2,12 +2,11 @@
 // meshes; no reference counterpart).
 //
 // One launch advances every case by one step: the grid is the concatenation of
-// all cases' march tiles (tile rows x 64 columns x `chunk` planes), each
-// workgroup finds its case by a binary search over the cases' first-tile
-// offsets (scalar loads of a small descriptor table) and runs the same tile
-// code as the single-mesh kernels, so every case's fields equal a plain
-// single-case run bit for bit.  A run of n steps is captured once into a HIP
-// graph (n kernel nodes, no memset nodes) and replayed with one launch.
+// all cases' workgroups, each finds its case by a binary search over the cases'
+// first-workgroup offsets (scalar loads of a small descriptor table) and runs
+// the same device code as the single-mesh kernels, so every case's fields equal
+// a plain single-case run bit for bit.  A run of n steps is captured once into
+// a HIP graph (n kernel nodes, no memset nodes) and replayed with one launch.
 #include <hip/hip_runtime.h>
 
 #include <map>
@@ -19,6 +18,7 @@
 #include "march.hpp"
 #include "row.hpp"
 #include "row2.hpp"
+#include "star_wave.hpp"
 
 namespace cfd {
 
@@ -28,43 +28,59 @@ struct BatchCaseDev {
     float dt;
     int kind;            // CFD_CASE_HEAT / CFD_CASE_WAVE
     int nzt, nyt;
-    int64_t tile0;       // first tile of the case in the batched grid
+    int64_t tile0;       // first tile of the case in the batched grid (row forms)
     float* a[4];
     float* b[4];
+    // star form: workgroups of 256 threads, `star_wg` of them (a multiple of
+    // 8) from star0; thread / plan.bx is (thread * star_div) >> 16
+    star::Plan plan;
+    int star0, star_wg, star_width;
+    uint32_t star_div;
 };
 
-template <int TYT, int R> union BatchLds {
-    MarchLds<float, TYT, R> w;
-    HeatLds<float, TYT, R> h;
-};
-
-template <int TYT, int R>
-__global__ void __launch_bounds__(64 * TYT) batch_step_k(const BatchCaseDev* __restrict__ cases, int ncases,
-                                                         int parity, int L) {
-    __shared__ BatchLds<TYT, R> lds;
-    const int64_t tile = blockIdx.x;
-    int lo = 0, hi = ncases - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (cases[mid].tile0 <= tile) lo = mid;
-        else hi = mid - 1;
-    }
-    const BatchCaseDev& cs = cases[lo];
-    const int64_t t = tile - cs.tile0;
-    const int64_t zt = t % cs.nzt;
-    const int64_t yt = (t / cs.nzt) % cs.nyt;
-    const int64_t xc = t / (int64_t(cs.nzt) * cs.nyt);
+// Form 0: the star form (star.hpp) of every case's step.  us/step against 2.5D
+// march tiles of 4 rows x 8 planes, which it replaced: 16 cases of sides 16 to
+// 128 (161 MiB of fields) 38.7 / 56.3, 12 cases up to 96 (22 MiB) 10.1 / 18.2,
+// 64 cases up to 128 (615 MiB) 181 / 252.
+template <int W, bool PW>
+__device__ __forceinline__ void batch_star_cells(const BatchCaseDev& cs, int parity, int tx, int ty) {
+    const star::Plan pl = cs.plan;
+    star::Place at;
+    if (!star::place_at<W>(pl, int(blockIdx.x) - cs.star0, cs.star_wg, tx, ty, at)) return;
     float* const* in = parity ? cs.b : cs.a;
     float* const* out = parity ? cs.a : cs.b;
     if (cs.kind == CFD_CASE_HEAT) {
-        if (cs.g.vol_pow2) heat_march_tile<float, TYT, R, true>(cs.g, in[0], out[0], cs.coef, cs.dt, L, zt, yt, xc, lds.h);
-        else heat_march_tile<float, TYT, R, false>(cs.g, in[0], out[0], cs.coef, cs.dt, L, zt, yt, xc, lds.h);
-    } else if (cs.g.vol_pow2) {
-        wave_march_tile<float, TYT, R, false, true>(cs.g, in[0], in[1], in[2], in[3], out[0], out[1], out[2],
-                                                       out[3], cs.coef, nullptr, cs.dt, L, zt, yt, xc, lds.w);
+        const star::Offsets<W> o = star::offsets<W>(pl, at);
+        const star::Star7<float, W> s = star::load7<float, W>(in[0], o);
+        float r[W];
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+            r[i] = cs.dt * (cs.coef * star::lapl_uniform<float, W, PW>(cs.g, s, 7, i)) + s.c(i);
+        star::store<float, W>(out[0] + o.x0, o.o0, r);
     } else {
-        wave_march_tile<float, TYT, R, false, false>(cs.g, in[0], in[1], in[2], in[3], out[0], out[1], out[2],
-                                                        out[3], cs.coef, nullptr, cs.dt, L, zt, yt, xc, lds.w);
+        star::wave_cells<float, W, PW, false, 0>(cs.g, in[0], in[1], in[2], in[3], out[0], out[1], out[2], out[3],
+                                                 cs.coef, nullptr, cs.dt, pl, at);
+    }
+}
+
+// A case whose rows are shorter than a vector (or whose planes are too large
+// for 32-bit offsets) takes one cell per thread.
+__global__ void __launch_bounds__(256) batch_star_k(const BatchCaseDev* __restrict__ cases, int ncases, int parity) {
+    constexpr int W = star::kWidth<float>;
+    int lo = 0, hi = ncases - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (cases[mid].star0 <= int(blockIdx.x)) lo = mid;
+        else hi = mid - 1;
+    }
+    const BatchCaseDev& cs = cases[lo];
+    const int t = int(threadIdx.x), ty = int((uint32_t(t) * cs.star_div) >> 16), tx = t - ty * cs.plan.bx;
+    if (cs.star_width == 1) {
+        if (cs.g.vol_pow2) batch_star_cells<1, true>(cs, parity, tx, ty);
+        else batch_star_cells<1, false>(cs, parity, tx, ty);
+    } else {
+        if (cs.g.vol_pow2) batch_star_cells<W, true>(cs, parity, tx, ty);
+        else batch_star_cells<W, false>(cs, parity, tx, ty);
     }
 }
 
@@ -190,7 +206,8 @@ struct cfd_batch_s {
     BatchCaseDev* dev = nullptr;
     int tile_rows = 4;
     int chunk = 8;
-    int form = 0;  // 0: 2.5D march tiles, 1: row form, 2: row form, two steps per launch
+    int form = 0;  // 0: star form, 1: row form, 2: row form, two steps per launch
+    int star_wg = 0;  // workgroups of the star form
     int64_t total_tiles = 0;
     // form 2: single-step row-form layout (4-row tiles) for the steps left after
     // the pairs of two-step launches
@@ -240,6 +257,21 @@ static int64_t layout_into(std::vector<BatchCaseDev>& cases, int form, int T, in
     return off;
 }
 
+// The star form's workgroups.
+static void star_layout(cfd_batch_s* b) {
+    int64_t wg = 0;
+    for (auto& c : b->host) {
+        c.star_width = star::vector_form<float>(c.g.Y, c.g.Z) ? star::kWidth<float> : 1;
+        c.plan = star::make_plan(c.g.X, c.g.Y, c.g.Z, c.star_width, 256);
+        c.star0 = int(wg);
+        c.star_wg = (c.plan.blocks + 7) / 8 * 8;
+        c.star_div = (65536 + uint32_t(c.plan.bx) - 1) / uint32_t(c.plan.bx);
+        wg += c.star_wg;
+        CFD_REQUIRE(wg < (int64_t(1) << 31), "batched grid too large");
+    }
+    b->star_wg = int(wg);
+}
+
 static void batch_layout(cfd_batch_s* b, hipStream_t s) {
     b->total_tiles = layout_into(b->host, b->form, b->tile_rows, b->chunk);
     const size_t bytes = b->host.size() * sizeof(BatchCaseDev);
@@ -273,12 +305,7 @@ static void batch_launch(const cfd_batch_s* b, int parity, hipStream_t s) {
         }
         return;
     }
-    switch (b->tile_rows) {
-        case 4: batch_step_k<4, 1><<<grid, dim3(64, 4), 0, s>>>(b->dev, n, parity, b->chunk); break;
-        case 8: batch_step_k<4, 2><<<grid, dim3(64, 4), 0, s>>>(b->dev, n, parity, b->chunk); break;
-        case 16: batch_step_k<4, 4><<<grid, dim3(64, 4), 0, s>>>(b->dev, n, parity, b->chunk); break;
-        default: throw Error(CFD_E_INVALID, "batch tile rows must be 4, 8 or 16");
-    }
+    batch_star_k<<<dim3(unsigned(b->star_wg)), 256, 0, s>>>(b->dev, n, parity);
 }
 
 // nsteps steps from state_a: in form 2, pairs of two-step launches (a -> b ->
@@ -337,6 +364,7 @@ int cfd_batch_create(cfd_ctx_t ctx, const cfd_batch_case* cases, int ncases, cfd
             }
             b->host.push_back(d);
         }
+        star_layout(b.get());
         b->dev = (BatchCaseDev*)pool_alloc(ctx, int64_t(ncases) * int64_t(sizeof(BatchCaseDev)), nullptr);
         try {
             batch_layout(b.get(), nullptr);
@@ -356,7 +384,7 @@ int cfd_batch_set_form(cfd_batch_t b, int form) {
     return guarded([&] {
         CFD_REQUIRE(b != nullptr, "null batch");
         CFD_REQUIRE(form >= 0 && form <= 2,
-                    "batch form must be 0 (march tiles), 1 (row form) or 2 (row form, two steps per launch)");
+                    "batch form must be 0 (star form), 1 (row form) or 2 (row form, two steps per launch)");
         if (form >= 1) {
             for (const auto& c : b->host) {
                 if (!wave_row_supported(c.g.Z))

@@ -1,6 +1,5 @@
 // 2.5D march tile of the fused acoustic step on a uniform mesh (see
-// wave_march.hip), shared by the single-mesh kernel and the batched ensemble
-// kernel.
+// wave_march.hip) and the step's elementary operations, which every form shares.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -70,8 +69,7 @@ template <class T, int TYT, int R> struct MarchLds {
 };
 
 // One (zt, yt, xc) tile of the fused step: columns [yt*TY, +TY) x [zt*64, +64),
-// planes [xc*L, +L).  Called by the single-mesh kernel below and by the
-// batched ensemble kernel.
+// planes [xc*L, +L).
 // NT: stream the outputs past the L2 (non-temporal stores), leaving its
 // capacity to the halo rows that neighbouring tiles read again.
 template <class T, int TYT, int R, bool NT = false, bool PW = false>
@@ -275,126 +273,6 @@ __device__ inline void wave_march_tile(const UniformGeo<T>& g, const T* __restri
             Pp1[r] = Pp2[r];
             Um1[r] = U0[r];
             U0[r] = Up1[r];
-        }
-    }
-}
-
-// LDS plane of one heat march tile (halo 1 in y and z, double-buffered)
-template <class T, int TYT, int R> struct HeatLds {
-    static constexpr int TY = TYT * R;
-    static constexpr int TZ = 64;
-    static constexpr int PZ = TZ + 2;
-    static constexpr int PS = (TY + 2) * PZ;
-    T s[2][PS];
-};
-
-// One (zt, yt, xc) tile of the heat step dt * (alpha * lapl(T)) + T on a
-// uniform mesh, marching along x with T(x-1), T(x), T(x+1) in registers and the
-// plane's y/z neighbours in LDS.  The arithmetic is heat_star_k's
-// (Grad2Var with neighbour = self on the walls), so the two agree bit for bit.
-template <class T, int TYT, int R, bool PW = false>
-__device__ inline void heat_march_tile(const UniformGeo<T>& g, const T* __restrict__ Tin, T* __restrict__ Tout,
-                                       T alpha, T dt, int L, int64_t zt, int64_t yt, int64_t xc,
-                                       HeatLds<T, TYT, R>& lds) {
-    static_assert(TYT >= 2, "two halo-row threads are needed");
-    using H = HeatLds<T, TYT, R>;
-    constexpr int TY = H::TY;
-    constexpr int TZ = H::TZ;
-    constexpr int PZ = H::PZ;
-    const int64_t X = g.X, Y = g.Y, Z = g.Z, SX = Y * Z;
-    const VolDiv<T, PW> Vd{g.vol, g.inv_vol};
-    const int lz = threadIdx.x, ly = threadIdx.y;
-    const int64_t z = zt * TZ + lz;
-    const int64_t y0 = yt * TY;
-    const int64_t x0 = xc * L;
-    const int64_t x1 = (x0 + L < X) ? x0 + L : X;
-    if (x0 >= X) return;  // uniform across the workgroup
-    const int64_t zc = clamp_halo(z, Z);
-
-    int64_t col[R];
-    bool valid[R];
-    int own[R];
-    int64_t zh_col[R];  // z-halo column of lanes 0 / 63 (-1: none)
-    int zh_lds[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int row = r * TYT + ly;
-        const int64_t y = y0 + row;
-        valid[r] = z < Z && y < Y;
-        col[r] = valid[r] ? y * Z + z : 0;
-        own[r] = (row + 1) * PZ + (lz + 1);
-        zh_col[r] = -1;
-        zh_lds[r] = -1;
-        if (y < Y && (lz == 0 || lz == TZ - 1)) {
-            const int c = lz == 0 ? -1 : TZ;
-            const int64_t gz = clamp_halo(zt * TZ + c, Z);
-            if (gz >= 0) {
-                zh_col[r] = y * Z + gz;
-                zh_lds[r] = (row + 1) * PZ + (c + 1);
-            }
-        }
-    }
-    // y-halo rows -1 (ly 0) and TY (ly 1), neighbour = self at the walls
-    int64_t yh_col = -1;
-    int yh_lds = -1;
-    if ((ly == 0 || ly == 1) && zc >= 0 && z < Z) {
-        const int hr = ly == 0 ? -1 : TY;
-        const int64_t gy = clamp_halo(y0 + hr, Y);
-        if (gy >= 0) {
-            yh_col = gy * Z + z;
-            yh_lds = (hr + 1) * PZ + (lz + 1);
-        }
-    }
-    T Tm1[R], T0[R], Tp1[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        Tm1[r] = T0[r] = Tp1[r] = T(0);
-        if (valid[r]) {
-            T0[r] = Tin[x0 * SX + col[r]];
-            if (x0 >= 1) Tm1[r] = Tin[(x0 - 1) * SX + col[r]];
-            if (x0 + 1 < X) Tp1[r] = Tin[(x0 + 1) * SX + col[r]];
-        }
-    }
-    int b = 0;
-    for (int64_t x = x0; x < x1; ++x, b ^= 1) {
-        const int64_t base = x * SX;
-        T* P = lds.s[b];
-        T nxt[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            nxt[r] = T(0);
-            if (valid[r] && x + 2 < X) nxt[r] = Tin[base + 2 * SX + col[r]];
-            if (valid[r]) P[own[r]] = T0[r];
-            if (zh_lds[r] >= 0) P[zh_lds[r]] = Tin[base + zh_col[r]];
-        }
-        if (yh_lds >= 0) P[yh_lds] = Tin[base + yh_col];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (valid[r]) {
-                const int row = r * TYT + ly;
-                const int64_t y = y0 + row;
-                const T pc = T0[r];
-                // walls: the neighbour is the cell itself (reference rule); the
-                // LDS slots read here are all written this plane
-                const bool lo_w[3] = {x == 0, y == 0, z == 0};
-                const bool hi_w[3] = {x == X - 1, y == Y - 1, z == Z - 1};
-                const T nb_lo[3] = {lo_w[0] ? pc : Tm1[r], lo_w[1] ? pc : P[own[r] - PZ], lo_w[2] ? pc : P[own[r] - 1]};
-                const T nb_hi[3] = {hi_w[0] ? pc : Tp1[r], hi_w[1] ? pc : P[own[r] + PZ], hi_w[2] ? pc : P[own[r] + 1]};
-                T Lp = T(0);
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const T al_lo = lo_w[a] ? g.alpha_b[a] : g.alpha[a];
-                    const T al_hi = hi_w[a] ? g.alpha_b[a] : g.alpha[a];
-                    const T s_lo = (-pc + nb_lo[a]) * al_lo;
-                    const T s_hi = (-pc + nb_hi[a]) * al_hi;
-                    Lp = Lp + Vd(s_lo * g.area[a] + s_hi * g.area[a]);
-                }
-                Tout[base + col[r]] = dt * (alpha * Lp) + pc;
-            }
-            Tm1[r] = T0[r];
-            T0[r] = Tp1[r];
-            Tp1[r] = nxt[r];
         }
     }
 }

@@ -31,18 +31,12 @@ namespace {
 template <class T, int GEO> struct GeoArg { using type = UniformGeo<T>; };
 template <class T> struct GeoArg<T, 2> { using type = LatticeGeo<T>; };
 
-template <class T, int W> __device__ inline T face_nb(const star::Star7<T, W>& s, int a, bool upper, int i) {
-    if (a == 0) return upper ? s.xp[i] : s.xm[i];
-    if (a == 1) return upper ? s.yp[i] : s.ym[i];
-    return upper ? s.r[i + 2] : s.r[i];
-}
-
 // whether the lower / upper face of cell i along axis a is on the wall
 struct AtWall {
     bool lo[3], hi[3];
 };
-template <int W> __device__ inline AtWall at_wall(const star::Plan& pl, int x, int y, int z0, int i) {
-    return {{x == 0, y == 0, z0 + i == 0}, {x == pl.X - 1, y == pl.Y - 1, z0 + i == pl.Z - 1}};
+__device__ inline AtWall at_wall(const star::Plan& pl, const star::Place& q, int i) {
+    return {{q.x == 0, q.y == 0, q.z0 + i == 0}, {q.x == pl.X - 1, q.y == pl.Y - 1, q.z0 + i == pl.Z - 1}};
 }
 
 // interpolated face values of cell i, zero on the walls normal to wall_axis
@@ -51,8 +45,8 @@ __device__ inline star::Faces<T> lin_faces(const star::Star7<T, W>& s, const AtW
     star::Faces<T> f;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        f.lo[a] = mlin(s.c(i), face_nb(s, a, false, i));
-        f.hi[a] = mlin(s.c(i), face_nb(s, a, true, i));
+        f.lo[a] = mlin(s.c(i), star::face_nb(s, a, false, i));
+        f.hi[a] = mlin(s.c(i), star::face_nb(s, a, true, i));
         if (wall_axis == a) {
             if (w.lo[a]) f.lo[a] = T(0);
             if (w.hi[a]) f.hi[a] = T(0);
@@ -65,29 +59,22 @@ __device__ inline star::Faces<T> lin_faces(const star::Star7<T, W>& s, const AtW
 template <class T, int W, int GEO>
 __device__ inline T lapl_cell(const typename GeoArg<T, GEO>::type& g, const star::LatticeCells<T, W>& lc,
                               const star::Star7<T, W>& s, int mask, int i) {
-    const T pc = s.c(i);
-    T res = T(0);
-    if constexpr (GEO == 2) {
+    if constexpr (GEO != 2) {
+        return star::lapl_uniform<T, W, GEO == 0>(g, s, mask, i);
+    } else {
+        const T pc = s.c(i);
+        T res = T(0);
         star::Faces<T> f;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            f.lo[a] = (-pc + face_nb(s, a, false, i)) * (a == 0 ? lc.ax[0] : a == 1 ? lc.ay[0] : lc.az[i]);
-            f.hi[a] = (-pc + face_nb(s, a, true, i)) * (a == 0 ? lc.ax[1] : a == 1 ? lc.ay[1] : lc.az[i + 1]);
+            f.lo[a] = (-pc + star::face_nb(s, a, false, i)) * (a == 0 ? lc.ax[0] : a == 1 ? lc.ay[0] : lc.az[i]);
+            f.hi[a] = (-pc + star::face_nb(s, a, true, i)) * (a == 0 ? lc.ax[1] : a == 1 ? lc.ay[1] : lc.az[i + 1]);
         }
 #pragma unroll
         for (int a = 0; a < 3; ++a)
             if (mask & (1 << a)) res = res + star::lattice_gauss<T, W, false>(lc, f, a, i);
-    } else {
-        const VolDiv<T, GEO == 0> Vd{g.vol, g.inv_vol};
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            if (!(mask & (1 << a))) continue;
-            const T s_lo = (-pc + face_nb(s, a, false, i)) * g.alpha[a];
-            const T s_hi = (-pc + face_nb(s, a, true, i)) * g.alpha[a];
-            res = res + Vd(s_lo * g.area[a] + s_hi * g.area[a]);
-        }
+        return res;
     }
-    return res;
 }
 
 }  // namespace
@@ -95,16 +82,16 @@ __device__ inline T lapl_cell(const typename GeoArg<T, GEO>::type& g, const star
 template <class T, int W, int GEO>
 __global__ void __launch_bounds__(256) grad_star_k(typename GeoArg<T, GEO>::type g, const T* __restrict__ phi,
                                                    T* __restrict__ out, int mask, int wall_axis, star::Plan pl) {
-    int x, y, z0;
-    if (!star::place<W>(pl, x, y, z0)) return;
-    const star::Offsets<W> o = star::offsets<W>(pl, x, y, z0);
+    star::Place q;
+    if (!star::place<W>(pl, q)) return;
+    const star::Offsets<W> o = star::offsets<W>(pl, q);
     const star::Star7<T, W> s = star::load7<T, W>(phi, o);
     star::LatticeCells<T, W> lc;
-    if constexpr (GEO == 2) lc = star::load_lattice<T, W, false>(g, o, x, y, z0);
+    if constexpr (GEO == 2) lc = star::load_lattice<T, W, false>(g, o, q);
     T r[W];
 #pragma unroll
     for (int i = 0; i < W; ++i) {
-        const star::Faces<T> f = lin_faces(s, at_wall<W>(pl, x, y, z0, i), wall_axis, i);
+        const star::Faces<T> f = lin_faces(s, at_wall(pl, q, i), wall_axis, i);
         T res = T(0);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -124,12 +111,12 @@ __global__ void __launch_bounds__(256) grad_star_k(typename GeoArg<T, GEO>::type
 template <class T, int W, int GEO>
 __global__ void __launch_bounds__(256) lapl_star_k(typename GeoArg<T, GEO>::type g, const T* __restrict__ phi,
                                                    T* __restrict__ out, int mask, star::Plan pl) {
-    int x, y, z0;
-    if (!star::place<W>(pl, x, y, z0)) return;
-    const star::Offsets<W> o = star::offsets<W>(pl, x, y, z0);
+    star::Place q;
+    if (!star::place<W>(pl, q)) return;
+    const star::Offsets<W> o = star::offsets<W>(pl, q);
     const star::Star7<T, W> s = star::load7<T, W>(phi, o);
     star::LatticeCells<T, W> lc;
-    if constexpr (GEO == 2) lc = star::load_lattice<T, W, true>(g, o, x, y, z0);
+    if constexpr (GEO == 2) lc = star::load_lattice<T, W, true>(g, o, q);
     T r[W];
 #pragma unroll
     for (int i = 0; i < W; ++i) r[i] = lapl_cell<T, W, GEO>(g, lc, s, mask, i);
@@ -141,12 +128,12 @@ template <class T, int W, int GEO, bool AF>
 __global__ void __launch_bounds__(256) heat_star_k(typename GeoArg<T, GEO>::type g, const T* __restrict__ Tin,
                                                    T* __restrict__ Tout, T alpha, const T* __restrict__ alpha_f, T dt,
                                                    star::Plan pl) {
-    int x, y, z0;
-    if (!star::place<W>(pl, x, y, z0)) return;
-    const star::Offsets<W> o = star::offsets<W>(pl, x, y, z0);
+    star::Place q;
+    if (!star::place<W>(pl, q)) return;
+    const star::Offsets<W> o = star::offsets<W>(pl, q);
     const star::Star7<T, W> s = star::load7<T, W>(Tin, o);
     star::LatticeCells<T, W> lc;
-    if constexpr (GEO == 2) lc = star::load_lattice<T, W, true>(g, o, x, y, z0);
+    if constexpr (GEO == 2) lc = star::load_lattice<T, W, true>(g, o, q);
     T af[W];
     if constexpr (AF) star::load<T, W>(alpha_f + o.x0, o.o0, af);
     T r[W];
@@ -169,24 +156,24 @@ __global__ void __launch_bounds__(256) wave_vel_lattice_k(LatticeGeo<T> g, const
                                                           const T* __restrict__ w, T* __restrict__ uo,
                                                           T* __restrict__ vo, T* __restrict__ wo, T dt,
                                                           star::Plan pl) {
-    int x, y, z0;
-    if (!star::place<W>(pl, x, y, z0)) return;
-    const star::Offsets<W> o = star::offsets<W>(pl, x, y, z0);
+    star::Place q;
+    if (!star::place<W>(pl, q)) return;
+    const star::Offsets<W> o = star::offsets<W>(pl, q);
     const star::Star7<T, W> s = star::load7<T, W>(p, o);
-    const star::LatticeCells<T, W> lc = star::load_lattice<T, W, false>(g, o, x, y, z0);
-    T q[3][W];
-    star::load<T, W>(u + o.x0, o.o0, q[0]);
-    star::load<T, W>(v + o.x0, o.o0, q[1]);
-    star::load<T, W>(w + o.x0, o.o0, q[2]);
+    const star::LatticeCells<T, W> lc = star::load_lattice<T, W, false>(g, o, q);
+    T n[3][W];
+    star::load<T, W>(u + o.x0, o.o0, n[0]);
+    star::load<T, W>(v + o.x0, o.o0, n[1]);
+    star::load<T, W>(w + o.x0, o.o0, n[2]);
 #pragma unroll
     for (int i = 0; i < W; ++i) {
         const star::Faces<T> f = lin_faces(s, AtWall{}, -1, i);
 #pragma unroll
-        for (int a = 0; a < 3; ++a) q[a][i] = dt * (-star::lattice_gauss<T, W, true>(lc, f, a, i)) + q[a][i];
+        for (int a = 0; a < 3; ++a) n[a][i] = dt * (-star::lattice_gauss<T, W, true>(lc, f, a, i)) + n[a][i];
     }
-    star::store<T, W>(uo + o.x0, o.o0, q[0]);
-    star::store<T, W>(vo + o.x0, o.o0, q[1]);
-    star::store<T, W>(wo + o.x0, o.o0, q[2]);
+    star::store<T, W>(uo + o.x0, o.o0, n[0]);
+    star::store<T, W>(vo + o.x0, o.o0, n[1]);
+    star::store<T, W>(wo + o.x0, o.o0, n[2]);
 }
 
 template <class T, int W, bool KF>
@@ -194,17 +181,17 @@ __global__ void __launch_bounds__(256) wave_p_lattice_k(LatticeGeo<T> g, const T
                                                         const T* __restrict__ v, const T* __restrict__ w,
                                                         const T* __restrict__ p, T* __restrict__ po, T K,
                                                         const T* __restrict__ Kf, T dt, star::Plan pl) {
-    int x, y, z0;
-    if (!star::place<W>(pl, x, y, z0)) return;
-    const star::Offsets<W> o = star::offsets<W>(pl, x, y, z0);
+    star::Place q;
+    if (!star::place<W>(pl, q)) return;
+    const star::Offsets<W> o = star::offsets<W>(pl, q);
     const star::Star7<T, W> s[3] = {star::load7<T, W>(u, o), star::load7<T, W>(v, o), star::load7<T, W>(w, o)};
-    const star::LatticeCells<T, W> lc = star::load_lattice<T, W, false>(g, o, x, y, z0);
+    const star::LatticeCells<T, W> lc = star::load_lattice<T, W, false>(g, o, q);
     T pc[W], kf[W];
     star::load<T, W>(p + o.x0, o.o0, pc);
     if constexpr (KF) star::load<T, W>(Kf + o.x0, o.o0, kf);
 #pragma unroll
     for (int i = 0; i < W; ++i) {
-        const AtWall wl = at_wall<W>(pl, x, y, z0, i);
+        const AtWall wl = at_wall(pl, q, i);
         T S = T(0);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
+#include "march.hpp"
 
 namespace cfd {
 
@@ -69,13 +70,14 @@ struct Plan {
     int blocks;  // workgroups with work, before the padding
 };
 
-inline Plan make_plan(int64_t X, int64_t Y, int64_t Z, int W) {
+inline Plan make_plan(int64_t X, int64_t Y, int64_t Z, int W, int threads = 0) {
     Plan p{};
     p.X = int(X); p.Y = int(Y); p.Z = int(Z);
     const int units = int((Z + W - 1) / W);
-    // 256 threads, fewer on meshes that would not give each CU a workgroup
-    const int64_t all = X * Y * units;
-    const int threads = all >= 256 * 256 ? 256 : all >= 128 * 256 ? 128 : 64;
+    if (!threads) {  // 256 threads, fewer on meshes that would not give each CU a workgroup
+        const int64_t all = X * Y * units;
+        threads = all >= 256 * 256 ? 256 : all >= 128 * 256 ? 128 : 64;
+    }
     p.nzb = (units + threads - 1) / threads;
     p.bx = (units + p.nzb - 1) / p.nzb;
     p.by = threads / p.bx;
@@ -96,20 +98,28 @@ template <class T> inline bool vector_form(int64_t Y, int64_t Z) {
     return Z >= kWidth<T> && Y * Z * int64_t(sizeof(T)) < (int64_t(1) << 32);
 }
 
-// The thread's place: plane x (uniform), row y, first cell z0; false without
-// work.  The first *skip of its cells belong to the unit before as well.
-template <int W> __device__ inline bool place(const Plan& p, int& x, int& y, int& z0, int* skip = nullptr) {
-    const int lin = int((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+// A thread's place: plane x (uniform), row y, first cell z0.  The first `skip`
+// of its cells belong to the unit before as well.
+struct Place {
+    int x, y, z0, skip;
+};
+// The place of thread (tx, ty) of block `b` of a grid of `padded` blocks (a
+// multiple of 8, as plan_grid's); false without work.
+template <int W> __device__ inline bool place_at(const Plan& p, int b, int padded, int tx, int ty, Place& q) {
+    const int lin = (b % 8) * (padded / 8) + b / 8;
     if (lin >= p.blocks) return false;
     const int row = p.nzb == 1 ? lin : lin / p.nzb;
     const int zb = p.nzb == 1 ? 0 : lin - row * p.nzb;
-    x = row / p.nyb;
-    y = (row - x * p.nyb) * p.by + int(threadIdx.y);
-    const int zi = zb * p.bx + int(threadIdx.x);
-    if (y >= p.Y || zi * W >= p.Z) return false;
-    z0 = min(zi * W, p.Z - W);
-    if (skip) *skip = zi * W - z0;
+    q.x = row / p.nyb;
+    q.y = (row - q.x * p.nyb) * p.by + ty;
+    const int zi = zb * p.bx + tx;
+    if (ty >= p.by || q.y >= p.Y || zi * W >= p.Z) return false;
+    q.z0 = min(zi * W, p.Z - W);
+    q.skip = zi * W - q.z0;
     return true;
+}
+template <int W> __device__ inline bool place(const Plan& p, Place& q) {
+    return place_at<W>(p, int(blockIdx.x), int(gridDim.x), int(threadIdx.x), int(threadIdx.y), q);
 }
 
 // Element offsets of a thread's cells and of their six neighbours, clamped to
@@ -118,8 +128,9 @@ template <int W> struct Offsets {
     int64_t x0, xm1, xp1;           // planes
     Off<W> o0, ym1, yp1, zm1, zp1;  // within a plane: the W cells, rows y-1 and y+1, cells z0-1 and z0+W
 };
-template <int W> __device__ inline Offsets<W> offsets(const Plan& p, int x, int y, int z0) {
+template <int W> __device__ inline Offsets<W> offsets(const Plan& p, const Place& q) {
     using O = Off<W>;
+    const int x = q.x, y = q.y, z0 = q.z0;
     Offsets<W> o;
     const int64_t SX = int64_t(p.Y) * p.Z;
     o.x0 = int64_t(x) * SX;
@@ -157,6 +168,31 @@ template <class T, int W> __device__ inline Star7<T, W> load7(const T* __restric
     return s;
 }
 
+// Value across the lower or upper face of cell i along axis a
+template <class T, int W> __device__ inline T face_nb(const Star7<T, W>& s, int a, bool upper, int i) {
+    if (a == 0) return upper ? s.xp[i] : s.xm[i];
+    if (a == 1) return upper ? s.yp[i] : s.ym[i];
+    return upper ? s.r[i + 2] : s.r[i];
+}
+
+// Laplacian of cell i of a uniform mesh over the selected axes, from 0 in the
+// order x, y, z (a wall's neighbour is the cell itself, so its difference is an
+// exact zero whatever the wall's alpha_d)
+template <class T, int W, bool PW>
+__device__ inline T lapl_uniform(const UniformGeo<T>& g, const Star7<T, W>& s, int mask, int i) {
+    const VolDiv<T, PW> Vd{g.vol, g.inv_vol};
+    const T pc = s.c(i);
+    T res = T(0);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        if (!(mask & (1 << a))) continue;
+        const T s_lo = (-pc + face_nb(s, a, false, i)) * g.alpha[a];
+        const T s_hi = (-pc + face_nb(s, a, true, i)) * g.alpha[a];
+        res = res + Vd(s_lo * g.area[a] + s_hi * g.area[a]);
+    }
+    return res;
+}
+
 // Geometry of a thread's cells on an axis-aligned lattice (LatticeGeo).
 template <class T, int W> struct LatticeCells {
     T wx, wy, wz[W];
@@ -165,7 +201,8 @@ template <class T, int W> struct LatticeCells {
     __device__ T area(int a, int i) const { return a == 0 ? wy * wz[i] : a == 1 ? wx * wz[i] : wx * wy; }
 };
 template <class T, int W, bool ALPHA>
-__device__ inline LatticeCells<T, W> load_lattice(const LatticeGeo<T>& g, const Offsets<W>& o, int x, int y, int z0) {
+__device__ inline LatticeCells<T, W> load_lattice(const LatticeGeo<T>& g, const Offsets<W>& o, const Place& q) {
+    const int x = q.x, y = q.y, z0 = q.z0;
     LatticeCells<T, W> c;
     load<T, W>(g.vol + o.x0, o.o0, c.V);
     c.wx = g.w[0][x];

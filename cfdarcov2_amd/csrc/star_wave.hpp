@@ -47,18 +47,17 @@ template <class T> struct WaveAux {
 // (lam_p, lam_u, lam_v, lam_w) and q = (dt K) lam_p,
 //   mu_a = lam_a - G_a(q),  nu_p = dt (Dx mu_x + Dy mu_y + Dz mu_z) + lam_p.
 template <class T, int W, bool PW, bool KF, int MODE>
-__device__ inline void wave_cells(const UniformGeo<T>& g, const T* __restrict__ p, const T* __restrict__ u,
+__device__ __forceinline__ void wave_cells(const UniformGeo<T>& g, const T* __restrict__ p, const T* __restrict__ u,
                                   const T* __restrict__ v, const T* __restrict__ w, T* __restrict__ po,
                                   T* __restrict__ uo, T* __restrict__ vo, T* __restrict__ wo, T K,
-                                  const T* __restrict__ Kf, T dt, const Plan& pl, const SensorSet* sens = nullptr,
+                                  const T* __restrict__ Kf, T dt, const Plan& pl, const Place& at, const SensorSet* sens = nullptr,
                                   const WaveAux<T>* aux = nullptr) {
     constexpr bool ADJ = MODE >= 2;
-    int x, y, z0, skip;
-    if (!place<W>(pl, x, y, z0, &skip)) return;
+    const int x = at.x, y = at.y, z0 = at.z0;
     const int X = pl.X, Y = pl.Y, Z = pl.Z;
     const T Ax = g.area[0], Ay = g.area[1], Az = g.area[2];
     const VolDiv<T, PW> Vd{g.vol, g.inv_vol};
-    const Offsets<W> o = offsets<W>(pl, x, y, z0);
+    const Offsets<W> o = offsets<W>(pl, at);
     using O = Off<W>;
     const int64_t SX = int64_t(Y) * Z;
     const int64_t x0 = o.x0, xm1 = o.xm1, xp1 = o.xp1;
@@ -192,12 +191,12 @@ __device__ inline void wave_cells(const UniformGeo<T>& g, const T* __restrict__ 
     if constexpr (MODE == 3) {
         // gK is updated in place, so the cells a row's last unit shares with
         // the unit before are left to that one
-        if (skip == 0) {
+        if (at.skip == 0) {
             store<T, W>(aux->gK + x0, o0, gk);
         } else {
 #pragma unroll
             for (int i = 1; i < W; ++i)
-                if (i >= skip) aux->gK[x0 + int64_t(o0) + i] = gk[i];
+                if (i >= at.skip) aux->gK[x0 + int64_t(o0) + i] = gk[i];
         }
     }
 }

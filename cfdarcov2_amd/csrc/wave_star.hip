@@ -18,7 +18,9 @@ __global__ void __launch_bounds__(256)
 wave_star_k(UniformGeo<T> g, const T* __restrict__ p, const T* __restrict__ u, const T* __restrict__ v,
             const T* __restrict__ w, T* __restrict__ po, T* __restrict__ uo, T* __restrict__ vo, T* __restrict__ wo,
             T K, const T* __restrict__ Kf, T dt, star::Plan pl) {
-    star::wave_cells<T, W, PW, KF, 0>(g, p, u, v, w, po, uo, vo, wo, K, Kf, dt, pl);
+    star::Place at;
+    if (star::place<W>(pl, at))
+        star::wave_cells<T, W, PW, KF, 0>(g, p, u, v, w, po, uo, vo, wo, K, Kf, dt, pl, at);
 }
 
 template <class T, int W, bool PW>

@@ -167,3 +167,42 @@ def test_adjoint_star(hip_ctx, n, every, dtype):
             err = (a.cpu().double() - b).norm() / max(float(b.norm()), 1e-30)
             assert err < (2.5e-5 if dtype == np.float32 else 5e-14), (field, float(err))
     gm.close()
+
+
+def test_batch_star_mixed_extents(hip_ctx):
+    """One batch of cases of any extents (rows shorter than a vector, not a
+    multiple of it, volumes that are no power of two): each equals its
+    single-case run."""
+    import ctypes
+
+    from cfdarcov2_amd import capi
+    rng = np.random.default_rng(2)
+    meshes, states, keep = [], [], []
+    for k, n in enumerate(EXTENTS + [(20, 12, 33), (16, 16, 16)]):
+        d = (0.125, 0.375, 0.25) if k % 3 == 0 else (0.125,) * 3
+        m = capi.HexMesh(hip_ctx, *n, *d, dtype="f32")
+        assert m.info().uniform == 1
+        heat = k % 2 == 0
+        a = [torch.from_numpy(rng.standard_normal(m.N).astype(np.float32)).cuda() for _ in range(1 if heat else 4)]
+        meshes.append(m)
+        states.append((heat, a, [torch.empty_like(t) for t in a], [t.clone() for t in a]))
+    arr = (capi.BatchCase * len(meshes))()
+    for c, m, (heat, a, b, _) in zip(arr, meshes, states):
+        c.mesh, c.kind, c.coef, c.dt = m.h, 0 if heat else 1, 1e-3 if heat else -0.8, 0.02
+        for f, (x, y) in enumerate(zip(a, b)):
+            c.state_a[f], c.state_b[f] = x.data_ptr(), y.data_ptr()
+    h = ctypes.c_void_p()
+    capi.check(hip_ctx.lib.cfd_batch_create(hip_ctx.h, arr, len(meshes), ctypes.byref(h)))
+    for graph in (0, 1):
+        for _, a, _, a0 in states:
+            for x, y in zip(a, a0):
+                x.copy_(y)
+        for _ in range(2):
+            capi.check(hip_ctx.lib.cfd_batch_run(h, 4, graph, capi._stream_ptr()))
+        torch.cuda.synchronize()
+        for k, (m, (heat, a, _, a0)) in enumerate(zip(meshes, states)):
+            A, B = [t.clone() for t in a0], [torch.empty_like(t) for t in a0]
+            ref = [m.heat_run(A[0], B[0], 1e-3, 0.02, 8)] if heat else m.wave_run(A, B, -0.8, 0.02, 8)
+            for g, r in zip(a, ref):
+                assert torch.equal(g, r), (k, graph)
+    capi.check(hip_ctx.lib.cfd_batch_destroy(h))
