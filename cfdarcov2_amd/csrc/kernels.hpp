@@ -54,13 +54,15 @@ void launch_wave_march(const cfd_mesh_s* m, void* const a[4], void* const b[4], 
 
 // Star forms (star.hpp; any extents and alignment): the acoustic step on
 // uniform meshes (wave_star.hip); one acoustic step on an axis-aligned lattice,
-// and the gradient, Laplacian and heat step on both (ops_star.hip)
+// the gradient, Laplacian and heat step on both and the stabilisation on
+// uniform meshes (ops_star.hip)
 template <class T>
 void launch_wave_lattice(const cfd_mesh_s* m, void* const* in, void* const* out, double K, const void* Kf, double dt,
                          hipStream_t s);
 template <class T>
 void launch_grad_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s);
 template <class T> void launch_lapl_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s);
+template <class T> void launch_stab_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s);
 template <class T>
 void launch_heat_star(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
                       hipStream_t s);

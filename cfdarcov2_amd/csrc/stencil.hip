@@ -70,27 +70,6 @@ template <class T> __device__ inline int64_t face_hi(const GeneralGeo<T>& g, con
 __device__ inline int fc_axis(int fc) { return 2 - (fc >> 1); }
 __device__ inline int axis_family(int a) { return 2 - a; }  // family 0 = z-faces, 1 = y, 2 = x
 
-// ---------------------------------------------------------------------------
-// uniform-mesh building blocks
-// ---------------------------------------------------------------------------
-
-// x / V on a uniform mesh.  For a power-of-two volume the quotient equals the
-// product with the exact reciprocal bit for bit (both are the correctly
-// rounded value of the same real number), which is one instruction instead of
-// a division sequence; the branch is uniform across the launch.
-template <class T> __device__ inline T udiv(const UniformGeo<T>& g, T x) {
-    return g.vol_pow2 ? x * g.inv_vol : x / g.vol;
-}
-
-// Green-Gauss component along axis a from the two face values on that axis:
-// acc = (f_lo * -1) * A + (f_hi * +1) * A, then / V (gauss_grad_cu_k order,
-// include/custom_cuda_functions.hpp:277-295; the other four faces add zeros).
-template <class T> __device__ inline T gg_pair_u(const UniformGeo<T>& g, T f_lo, T f_hi, T A) {
-    const T t_lo = (-f_lo) * A;
-    const T t_hi = f_hi * A;
-    return udiv(g, t_lo + t_hi);
-}
-
 // Linear face interpolation, (phi_c + phi_nb) * 0.5 (grad_utils.hpp:23-36).
 template <class T> __device__ inline T lin(T c, T nb) { return (c + nb) * T(0.5); }
 
@@ -98,115 +77,6 @@ template <class T> __device__ inline T lin(T c, T nb) { return (c + nb) * T(0.5)
 // GradVar / Grad2Var / StabVar operator kernels (the gradient and Laplacian of
 // uniform meshes and axis-aligned lattices: ops_star.hip)
 // ---------------------------------------------------------------------------
-
-// One axis d of StabVar on a uniform mesh (src/fvm3d.cpp:909-936), added to
-// res.  Second stage: upwind face values phi + (len * g_d) * n_out_d, jump
-// against the neighbour's opposite face (self's opposite face on the
-// boundary), 0.5 * jump, Gauss with axis normals for component d.  The first
-// stage's gradient components it reads (own and the two axis neighbours') are
-// recomputed here from phi at five points on the axis: pc at the cell, pl / ph
-// at its lower / upper neighbour, pll / plh at the lower neighbour's own lower
-// / upper neighbour, phl / phh likewise for the upper one (self on walls).
-template <class T>
-__device__ inline T stab_axis_u(const UniformGeo<T>& g, T res, int d, T pc, T pl, T ph, T pll, T plh, T phl,
-                                T phh) {
-    const T L = g.len[d];
-    const T gc = gg_pair_u(g, lin(pc, pl), lin(pc, ph), g.area[d]);
-    const T glo = gg_pair_u(g, lin(pl, pll), lin(pl, plh), g.area[d]);
-    const T ghi = gg_pair_u(g, lin(ph, phl), lin(ph, phh), g.area[d]);
-    const T own_lo = pc + (L * gc) * T(-1);
-    const T col_lo = pl + (L * glo) * T(1);
-    const T own_hi = pc + (L * gc) * T(1);
-    const T col_hi = ph + (L * ghi) * T(-1);
-    const T f_lo = T(0.5) * (own_lo - col_lo);
-    const T f_hi = T(0.5) * (own_hi - col_hi);
-    return res + udiv(g, f_lo * g.area[d] + f_hi * g.area[d]);
-}
-
-// The five points of one axis from a fetch function P(offset) (offset in
-// cells along the axis, -2..2), coordinate k on an axis of n cells.
-template <class T, class F>
-__device__ inline T stab_axis_at(const UniformGeo<T>& g, T res, int d, int64_t k, int64_t n, T pc, F P) {
-    const bool wl = k == 0, wh = k == n - 1;
-    const T pl = wl ? pc : P(-1);
-    const T ph = wh ? pc : P(1);
-    const T pll = wl ? pc : (k == 1 ? pl : P(-2));
-    const T plh = wl ? ph : pc;
-    const T phh = wh ? pc : (k == n - 2 ? ph : P(2));
-    const T phl = wh ? pl : pc;
-    return stab_axis_u(g, res, d, pc, pl, ph, pll, plh, phl, phh);
-}
-
-// StabVar on a uniform mesh in one pass, as a march along x: a workgroup
-// holds TY rows of 64 z-cells and walks `L` planes.  Each thread keeps its
-// column's values at x-2 .. x+2 in registers; the plane x goes to LDS with
-// two halo rows and columns on each side, so the y and z points come from
-// there; the halo values of the next plane are loaded into registers while
-// the current one is computed.  Every value passed to the arithmetic is the
-// one the cell-indexed rule picks (self on walls), so the result is the
-// per-cell evaluation's.
-template <class T, int TY>
-__global__ void __launch_bounds__(64 * TY) stab_march_uniform_k(UniformGeo<T> g, const T* __restrict__ phi,
-                                                                T* __restrict__ out, int mask, int L, int nzt,
-                                                                int nyt) {
-    static_assert(TY >= 4, "halo rows come from two distinct leading and trailing rows");
-    __shared__ T sh[TY + 4][64 + 4];
-    const int64_t X = g.X, Y = g.Y, Z = g.Z, SX = Y * Z;
-    const int64_t lin_ = blockIdx.x;
-    const int64_t zt = lin_ % nzt, yt = (lin_ / nzt) % nyt, xc = lin_ / (int64_t(nzt) * nyt);
-    const int lz = threadIdx.x, ly = threadIdx.y;
-    const int64_t z = zt * 64 + lz, y = yt * TY + ly;
-    const bool valid = z < Z && y < Y;
-    const int64_t col = valid ? y * Z + z : 0;
-    const int64_t x0 = xc * L, x1 = (x0 + L < X) ? x0 + L : X;
-    // halo rows (threads of the first / last two rows) and columns (lanes
-    // 0, 1, 62, 63) of this thread, -1 where outside the mesh
-    int64_t hy = -1, hz = -1;
-    int hy_row = 0, hz_col = 0;
-    if (z < Z) {
-        int64_t yy = -1;
-        if (ly < 2) { yy = yt * TY - 2 + ly; hy_row = ly; }
-        else if (ly >= TY - 2) { yy = yt * TY + TY + (ly - (TY - 2)); hy_row = ly + 4; }
-        if (yy >= 0 && yy < Y) hy = yy * Z + z;
-    }
-    if (y < Y) {
-        int64_t zz = -1;
-        if (lz < 2) { zz = zt * 64 - 2 + lz; hz_col = lz; }
-        else if (lz >= 62) { zz = zt * 64 + 64 + (lz - 62); hz_col = lz + 4; }
-        if (zz >= 0 && zz < Z) hz = y * Z + zz;
-    }
-    T w[5] = {T(0), T(0), T(0), T(0), T(0)};  // column values at x-2 .. x+2
-    if (valid)
-        for (int k = 0; k < 5; ++k) {
-            const int64_t xx = x0 - 2 + k;
-            if (xx >= 0 && xx < X) w[k] = phi[xx * SX + col];
-        }
-    // halo values of plane x (x0 < x1 <= X whenever the block has planes)
-    T hyv = (hy >= 0 && x0 < x1) ? phi[x0 * SX + hy] : T(0);
-    T hzv = (hz >= 0 && x0 < x1) ? phi[x0 * SX + hz] : T(0);
-    for (int64_t x = x0; x < x1; ++x) {
-        const int64_t pb = x * SX;
-        if (valid) sh[ly + 2][lz + 2] = w[2];
-        if (hy >= 0) sh[hy_row][lz + 2] = hyv;
-        if (hz >= 0) sh[ly + 2][hz_col] = hzv;
-        if (x + 1 < x1) {
-            if (hy >= 0) hyv = phi[pb + SX + hy];
-            if (hz >= 0) hzv = phi[pb + SX + hz];
-        }
-        __syncthreads();
-        if (valid) {
-            const T pc = w[2];
-            T res = T(0);
-            if (mask & 1) res = stab_axis_at(g, res, 0, x, X, pc, [&](int o) { return w[2 + o]; });
-            if (mask & 2) res = stab_axis_at(g, res, 1, y, Y, pc, [&](int o) { return sh[ly + 2 + o][lz + 2]; });
-            if (mask & 4) res = stab_axis_at(g, res, 2, z, Z, pc, [&](int o) { return sh[ly + 2][lz + 2 + o]; });
-            out[pb + col] = res;
-            w[0] = w[1]; w[1] = w[2]; w[2] = w[3]; w[3] = w[4];
-            w[4] = (x + 3 < X) ? phi[(x + 3) * SX + col] : T(0);
-        }
-        __syncthreads();
-    }
-}
 
 // --- general (per-face geometry) forms -------------------------------------
 
@@ -443,21 +313,7 @@ template <class T> void launch_lapl(const cfd_mesh_s* m, const void* phi, void* 
 template <class T>
 void launch_stab(const cfd_mesh_s* m, const void* phi, void* out, int mask, void* scratch3, hipStream_t s) {
     if (m->uniform) {
-        const auto& g = ugeo<T>(m);
-#ifndef CFD_STAB_TY
-#define CFD_STAB_TY 4
-#endif
-#ifndef CFD_STAB_PLANES
-#define CFD_STAB_PLANES 8
-#endif
-        // workgroup rows and x-planes per workgroup (build-time tunables)
-        constexpr int TY = CFD_STAB_TY;
-        const int L = CFD_STAB_PLANES;
-        const int nzt = int((g.Z + 63) / 64), nyt = int((g.Y + TY - 1) / TY);
-        const int64_t nwg = int64_t(nzt) * nyt * ((g.X + L - 1) / L);
-        CFD_REQUIRE(nwg < (int64_t(1) << 31), "stabilisation grid too large");
-        stab_march_uniform_k<T, TY><<<dim3(unsigned(nwg)), dim3(64, TY), 0, s>>>(g, (const T*)phi, (T*)out, mask,
-                                                                                 L, nzt, nyt);
+        launch_stab_star<T>(m, phi, out, mask, s);
     } else {
         CFD_REQUIRE(scratch3 != nullptr, "stabilisation on a general mesh needs 3N scratch entries");
         T* gx = (T*)scratch3;

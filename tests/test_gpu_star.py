@@ -74,6 +74,7 @@ def test_operators_and_heat_star(hip_ctx, oracle_lib, n, kind, dtype):
             for wall in (-1, 0, 1, 2):
                 assert np.array_equal(gm.grad(t, mask, wall, out=out).cpu().numpy(), om.grad(phi, mask, wall)), (mask, wall)
             assert np.array_equal(gm.lapl(t, mask, out=out).cpu().numpy(), om.lapl(phi, mask)), mask
+            assert np.array_equal(gm.stab(t, mask, out=out).cpu().numpy(), om.stab(phi, mask)), mask
         for a in (None, af):
             A, B = _view(phi, dtype, shift), _view(phi, dtype, shift)
             got = gm.heat_run(A, B, 2e-3, 0.5, 5, alpha_field=None if a is None else _view(a, dtype, shift))
