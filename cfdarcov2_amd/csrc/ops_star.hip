@@ -11,7 +11,7 @@
 // general form (GEO 2): heat step 64^3 FP64 2.8 us against 3.5 (the launch and
 // one memory round trip), decimal 100^3 FP64 6.8 against 38.4 us (the general
 // form moves 144 bytes per cell, this one 24); gradient, Laplacian and
-// stabilisation of 200^3 FP32 together 94 against 151 us; acoustic step on a
+// stabilisation of 200^3 FP32 together 68 against 151 us; acoustic step on a
 // decimal 120x100x80 FP32 lattice 14.3 against 49.0 us.
 //
 // The arithmetic is the reference's (src/fvm3d.cpp:825-829,902-906 and
@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(256) heat_star_k(typename GeoArg<T, GEO>::type
 // (at a wall the cell's own at its opposite face, i.e. the neighbour is the
 // cell itself), 0.5 * jump, Gauss sum.  Along z the gradients of W + 2 cells
 // serve all W cells.  Bound by its arithmetic, 108 operations per cell: 200^3
-// FP32 @STAB@ us against 48 for a march along x with the plane in LDS.
+// FP32 23 us against 48 for a march along x with the plane in LDS.
 template <class T, int W, bool PW>
 __global__ void __launch_bounds__(256) stab_star_k(UniformGeo<T> g, const T* __restrict__ phi, T* __restrict__ out,
                                                    int mask, star::Plan pl) {
