@@ -52,13 +52,10 @@ template <class T>
 void launch_wave_march(const cfd_mesh_s* m, void* const a[4], void* const b[4], double K, const void* Kf, double dt,
                        int64_t nsteps, int variant, int ty, int L, int remap, hipStream_t s);
 
-// Star forms (star.hpp; any extents and alignment): the acoustic step on
-// uniform meshes (wave_star.hip); one acoustic step on an axis-aligned lattice,
-// the gradient, Laplacian and heat step on both and the stabilisation on
-// uniform meshes (ops_star.hip)
-template <class T>
-void launch_wave_lattice(const cfd_mesh_s* m, void* const* in, void* const* out, double K, const void* Kf, double dt,
-                         hipStream_t s);
+// Star forms (star.hpp; any extents and alignment): operators and the heat step
+// on uniform meshes (ops_star.hip), the same and the acoustic step on meshes
+// with face geometry (ops_faces.hip), and the acoustic step on uniform ones
+// (wave_star.hip)
 template <class T>
 void launch_grad_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s);
 template <class T> void launch_lapl_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s);
@@ -66,6 +63,17 @@ template <class T> void launch_stab_star(const cfd_mesh_s* m, const void* phi, v
 template <class T>
 void launch_heat_star(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
                       hipStream_t s);
+template <class T>
+void launch_grad_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s);
+template <class T> void launch_lapl_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s);
+template <class T>
+void launch_stab_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, void* scratch3, hipStream_t s);
+template <class T>
+void launch_heat_faces(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
+                       hipStream_t s);
+template <class T>
+void launch_wave_faces(const cfd_mesh_s* m, void* const* in, void* const* out, double K, const void* Kf, double dt,
+                       hipStream_t s);
 template <class T>
 void launch_wave_star(const UniformGeo<T>& g, void* const* in, void* const* out, double K, const void* Kf, double dt,
                       hipStream_t s);

@@ -1,12 +1,13 @@
-// Stencil kernels of the explicit finite-volume step on the structured hex
-// mesh: Green-Gauss gradient, Laplacian, stabilisation, and the fused heat and
-// acoustic steps.  Three geometry forms:
+// Operators and explicit steps on the structured hex mesh: Green-Gauss
+// gradient, Laplacian, stabilisation, heat and acoustic steps, and the heat
+// step's adjoint.  Three geometry forms:
 //   uniform  - exactly uniform meshes; geometry is a handful of constants and
-//              neighbours are implicit, so only state crosses HBM;
+//              neighbours are implicit, so only state crosses HBM
+//              (ops_star.hip, wave_*.hip, heat_row.hip, heat_multi.hip);
 //   lattice  - axis-aligned faces (any spacing): widths and alpha_d per cell
-//              layer, volume per cell (ops_star.hip);
+//              layer, volume per cell (ops_faces.hip);
 //   general  - per-face SoA geometry (face families z, y, x) for perturbed
-//              meshes; neighbours are still implicit (structured topology).
+//              meshes; neighbours are still implicit (ops_faces.hip).
 // All arithmetic follows the reference operation order (see the oracle and
 // src/fvm3d.cpp / include/grad_utils.hpp cited per kernel) and the library is
 // built with -ffp-contract=off, so FP64 results are bit-identical to a CPU
@@ -55,222 +56,6 @@ template <class G> __device__ inline bool at_hi(const G& g, const Cell& c, int a
     return a == 0 ? c.x == g.X - 1 : a == 1 ? c.y == g.Y - 1 : c.z == g.Z - 1;
 }
 
-// Face-family index of the lower / upper face of cell c on axis a.
-template <class T> __device__ inline int64_t face_lo(const GeneralGeo<T>& g, const Cell& c, int a) {
-    if (a == 2) return c.x * g.Y * (g.Z + 1) + c.y * (g.Z + 1) + c.z;
-    if (a == 1) return c.x * (g.Y + 1) * g.Z + c.y * g.Z + c.z;
-    return c.x * g.Y * g.Z + c.y * g.Z + c.z;
-}
-template <class T> __device__ inline int64_t face_hi(const GeneralGeo<T>& g, const Cell& c, int a) {
-    if (a == 2) return face_lo(g, c, a) + 1;
-    if (a == 1) return face_lo(g, c, a) + g.Z;
-    return face_lo(g, c, a) + g.Y * g.Z;
-}
-// local face fc -> axis: fc 0,1 z; 2,3 y; 4,5 x
-__device__ inline int fc_axis(int fc) { return 2 - (fc >> 1); }
-__device__ inline int axis_family(int a) { return 2 - a; }  // family 0 = z-faces, 1 = y, 2 = x
-
-// Linear face interpolation, (phi_c + phi_nb) * 0.5 (grad_utils.hpp:23-36).
-template <class T> __device__ inline T lin(T c, T nb) { return (c + nb) * T(0.5); }
-
-// ---------------------------------------------------------------------------
-// GradVar / Grad2Var / StabVar operator kernels (the gradient and Laplacian of
-// uniform meshes and axis-aligned lattices: ops_star.hip)
-// ---------------------------------------------------------------------------
-
-// --- general (per-face geometry) forms -------------------------------------
-
-// value of face fc's stored axis normal component d and the outward sign
-template <class T>
-__device__ inline void face_geo(const GeneralGeo<T>& g, const Cell& c, int fc, int64_t& f, int& fam) {
-    const int a = fc_axis(fc);
-    fam = axis_family(a);
-    f = (fc & 1) ? face_hi(g, c, a) : face_lo(g, c, a);
-}
-template <class G> __device__ inline int64_t nb_of(const G& g, const Cell& c, int fc) {
-    const int a = fc_axis(fc);
-    return (fc & 1) ? nb_hi(g, c, a) : nb_lo(g, c, a);
-}
-template <class G> __device__ inline bool is_bnd_face(const G& g, const Cell& c, int fc) {
-    const int a = fc_axis(fc);
-    return (fc & 1) ? at_hi(g, c, a) : at_lo(g, c, a);
-}
-
-// Gauss sum of six face values for component d, fc = 0..5 from 0, outward
-// (use_alt=false in the reference's inverted flag) or axis normals.
-template <class T>
-__device__ inline T gauss_general(const GeneralGeo<T>& g, const Cell& c, const T fv[6], int d, bool axis_normals) {
-    T acc = T(0);
-    for (int fc = 0; fc < 6; ++fc) {
-        int64_t f; int fam;
-        face_geo(g, c, fc, f, fam);
-        T n = g.fn[fam][d][f];
-        if (!axis_normals && !(fc & 1)) n = -n;
-        T t = fv[fc] * n;
-        t = t * g.farea[fam][f];
-        acc = acc + t;
-    }
-    return acc / g.vol[c.id];
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) grad_general_k(GeneralGeo<T> g, const T* __restrict__ phi,
-                                                      T* __restrict__ out, int mask, int wall_axis) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = phi[c.id];
-    T fv[6];
-    for (int fc = 0; fc < 6; ++fc) {
-        fv[fc] = lin(pc, phi[nb_of(g, c, fc)]);
-        if (wall_axis == fc_axis(fc) && is_bnd_face(g, c, fc)) fv[fc] = T(0);
-    }
-    T res = T(0);
-    for (int d = 0; d < 3; ++d)
-        if (mask & (1 << d)) res = res + gauss_general(g, c, fv, d, false);
-    out[c.id] = res;
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) lapl_general_k(GeneralGeo<T> g, const T* __restrict__ phi,
-                                                      T* __restrict__ out, int mask) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = phi[c.id];
-    T fv[6];
-    for (int fc = 0; fc < 6; ++fc) {
-        int64_t f; int fam;
-        face_geo(g, c, fc, f, fam);
-        fv[fc] = (-pc + phi[nb_of(g, c, fc)]) * g.falpha[fam][f];
-    }
-    T res = T(0);
-    for (int d = 0; d < 3; ++d)
-        if (mask & (1 << d)) res = res + gauss_general(g, c, fv, d, true);
-    out[c.id] = res;
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) grad3_general_k(GeneralGeo<T> g, const T* __restrict__ phi,
-                                                       T* __restrict__ gx, T* __restrict__ gy, T* __restrict__ gz) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = phi[c.id];
-    T fv[6];
-    for (int fc = 0; fc < 6; ++fc) fv[fc] = lin(pc, phi[nb_of(g, c, fc)]);
-    gx[c.id] = gauss_general(g, c, fv, 0, false);
-    gy[c.id] = gauss_general(g, c, fv, 1, false);
-    gz[c.id] = gauss_general(g, c, fv, 2, false);
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) stab_general_k(GeneralGeo<T> g, const T* __restrict__ phi,
-                                                      const T* __restrict__ gx, const T* __restrict__ gy,
-                                                      const T* __restrict__ gz, T* __restrict__ out, int mask) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T* gs[3] = {gx, gy, gz};
-    const int64_t N = g.X * g.Y * g.Z;
-    T res = T(0);
-    for (int d = 0; d < 3; ++d) {
-        if (!(mask & (1 << d))) continue;
-        T fv[6];
-        for (int fc = 0; fc < 6; ++fc) {
-            int64_t f; int fam;
-            face_geo(g, c, fc, f, fam);
-            const T n = g.fn[fam][d][f];
-            const int ofc = fc ^ 1;
-            const int64_t nb = nb_of(g, c, fc);
-            // outward normal of (cell, fc) = (fc odd ? +n : -n); the neighbour
-            // sees the same face as its opposite local face.  On a boundary the
-            // neighbour is the cell itself and the opposite face is its own.
-            const T n_own = (fc & 1) ? n : -n;
-            T n_col;
-            if (nb == c.id) {
-                int64_t f2; int fam2;
-                face_geo(g, c, ofc, f2, fam2);
-                const T n2 = g.fn[fam2][d][f2];
-                n_col = (ofc & 1) ? n2 : -n2;
-            } else {
-                n_col = (ofc & 1) ? n : -n;
-            }
-            const T own = phi[c.id] + (g.len[int64_t(fc) * N + c.id] * gs[d][c.id]) * n_own;
-            const T col = phi[nb] + (g.len[int64_t(ofc) * N + nb] * gs[d][nb]) * n_col;
-            fv[fc] = T(0.5) * (own - col);
-        }
-        res = res + gauss_general(g, c, fv, d, true);
-    }
-    out[c.id] = res;
-}
-
-// ---------------------------------------------------------------------------
-// Fused heat step: T' = dt * (alpha * lapl(T)) + T   (DtVar::extract order,
-// src/fvm3d.cpp:690-692, with lapl = ((0 + L_x) + L_y) + L_z).
-// ---------------------------------------------------------------------------
-template <class T>
-__global__ void __launch_bounds__(256) heat_general_k(GeneralGeo<T> g, const T* __restrict__ Tin,
-                                                      T* __restrict__ Tout, T alpha, const T* __restrict__ alpha_f,
-                                                      T dt) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = Tin[c.id];
-    T fv[6];
-    for (int fc = 0; fc < 6; ++fc) {
-        int64_t f; int fam;
-        face_geo(g, c, fc, f, fam);
-        fv[fc] = (-pc + Tin[nb_of(g, c, fc)]) * g.falpha[fam][f];
-    }
-    T L = T(0);
-    for (int d = 0; d < 3; ++d) L = L + gauss_general(g, c, fv, d, true);
-    const T k = alpha_f ? alpha_f[c.id] : alpha;
-    Tout[c.id] = dt * (k * L) + pc;
-}
-
-// ---------------------------------------------------------------------------
-// Fused acoustic step.  Uniform meshes: wave_star.hip, wave_row.hip,
-// wave_row2.hip, wave_march.hip.
-// ---------------------------------------------------------------------------
-
-// General-mesh acoustic step.  Skewed face normals make every gradient
-// component depend on all six faces, so the step runs as two launches: the
-// three velocity equations (reading p), then the pressure equation (reading the
-// new velocities) - the same sequential semantics as the uniform kernel.
-template <class T>
-__global__ void __launch_bounds__(256) wave_vel_general_k(GeneralGeo<T> g, const T* __restrict__ p,
-                                                          const T* __restrict__ u, const T* __restrict__ v,
-                                                          const T* __restrict__ w, T* __restrict__ uo,
-                                                          T* __restrict__ vo, T* __restrict__ wo, T dt) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T pc = p[c.id];
-    T fv[6];
-    for (int fc = 0; fc < 6; ++fc) fv[fc] = lin(pc, p[nb_of(g, c, fc)]);
-    uo[c.id] = dt * (-gauss_general(g, c, fv, 0, false)) + u[c.id];
-    vo[c.id] = dt * (-gauss_general(g, c, fv, 1, false)) + v[c.id];
-    wo[c.id] = dt * (-gauss_general(g, c, fv, 2, false)) + w[c.id];
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) wave_p_general_k(GeneralGeo<T> g, const T* __restrict__ uo,
-                                                        const T* __restrict__ vo, const T* __restrict__ wo,
-                                                        const T* __restrict__ p, T* __restrict__ po, T K,
-                                                        const T* __restrict__ Kf, T dt) {
-    const Cell c = cell_of_thread(g);
-    if (!c.valid) return;
-    const T* vel[3] = {uo, vo, wo};
-    T S = T(0);
-    for (int a = 0; a < 3; ++a) {
-        const T qc = vel[a][c.id];
-        T fv[6];
-        for (int fc = 0; fc < 6; ++fc) {
-            fv[fc] = lin(qc, vel[a][nb_of(g, c, fc)]);
-            if (fc_axis(fc) == a && is_bnd_face(g, c, fc)) fv[fc] = T(0);
-        }
-        const T G = gauss_general(g, c, fv, a, false);
-        S = (a == 0) ? G : S + G;
-    }
-    const T k = Kf ? Kf[c.id] : K;
-    po[c.id] = dt * (k * S) + p[c.id];
-}
-
 // ---------------------------------------------------------------------------
 // launch helpers
 // ---------------------------------------------------------------------------
@@ -282,49 +67,28 @@ static const dim3 kBlock(64, 4, 1);
 template <class T> const UniformGeo<T>& ugeo(const cfd_mesh_s* m);
 template <> const UniformGeo<float>& ugeo<float>(const cfd_mesh_s* m) { return m->ug32; }
 template <> const UniformGeo<double>& ugeo<double>(const cfd_mesh_s* m) { return m->ug64; }
-template <class T> const GeneralGeo<T>& ggeo(const cfd_mesh_s* m);
-template <> const GeneralGeo<float>& ggeo<float>(const cfd_mesh_s* m) { return m->gg32; }
-template <> const GeneralGeo<double>& ggeo<double>(const cfd_mesh_s* m) { return m->gg64; }
-
 inline void check_launch() { CFD_HIP(hipGetLastError()); }
 
 template <class T> void launch_grad(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s) {
-    if (m->uniform || m->lattice) {
-        launch_grad_star<T>(m, phi, out, mask, wall, s);
-    } else {
-        const auto& g = ggeo<T>(m);
-        grad_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, (T*)out, mask, wall);
-    }
-    check_launch();
+    if (m->uniform) launch_grad_star<T>(m, phi, out, mask, wall, s);
+    else launch_grad_faces<T>(m, phi, out, mask, wall, s);
 }
 
 template <class T> void launch_lapl(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s) {
-    if (m->uniform || m->lattice) {
-        launch_lapl_star<T>(m, phi, out, mask, s);
-    } else {
-        const auto& g = ggeo<T>(m);
-        lapl_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, (T*)out, mask);
-    }
-    check_launch();
+    if (m->uniform) launch_lapl_star<T>(m, phi, out, mask, s);
+    else launch_lapl_faces<T>(m, phi, out, mask, s);
 }
 
-// scratch3 (3N entries, the first stage's gradients) is needed by the
-// general form only: uniform meshes run the one-pass kernel
+// scratch3 (3N entries, the first stage's gradients) is needed by meshes with
+// face geometry only: uniform meshes run the one-pass kernel
 template <class T>
 void launch_stab(const cfd_mesh_s* m, const void* phi, void* out, int mask, void* scratch3, hipStream_t s) {
     if (m->uniform) {
         launch_stab_star<T>(m, phi, out, mask, s);
     } else {
         CFD_REQUIRE(scratch3 != nullptr, "stabilisation on a general mesh needs 3N scratch entries");
-        T* gx = (T*)scratch3;
-        T* gy = gx + m->N;
-        T* gz = gy + m->N;
-        const auto& g = ggeo<T>(m);
-        grad3_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, gx, gy, gz);
-        check_launch();
-        stab_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, (const T*)phi, gx, gy, gz, (T*)out, mask);
+        launch_stab_faces<T>(m, phi, out, mask, scratch3, s);
     }
-    check_launch();
 }
 
 template <class T>
@@ -360,13 +124,8 @@ void launch_heat(const cfd_mesh_s* m, void* Ta, void* Tb, double alpha, const vo
     for (int64_t k = k0; k < nsteps; ++k) {
         const T* in = (const T*)((k & 1) ? Tb : Ta);
         T* out = (T*)((k & 1) ? Ta : Tb);
-        if (m->uniform || m->lattice) {
-            launch_heat_star<T>(m, in, out, alpha, af, dt, s);
-        } else {
-            const auto& g = ggeo<T>(m);
-            heat_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(g, in, out, T(alpha), (const T*)af, T(dt));
-        }
-        check_launch();
+        if (m->uniform) launch_heat_star<T>(m, in, out, alpha, af, dt, s);
+        else launch_heat_faces<T>(m, in, out, alpha, af, dt, s);
     }
 }
 
@@ -374,23 +133,8 @@ template <class T>
 void launch_wave(const cfd_mesh_s* m, void* const a[4], void* const b[4], double K, const void* Kf, double dt,
                  int64_t nsteps, hipStream_t s) {
     if (!m->uniform) {
-        const auto& g = ggeo<T>(m);
-        for (int64_t k = 0; k < nsteps; ++k) {
-            void* const* in = (k & 1) ? b : a;
-            void* const* out = (k & 1) ? a : b;
-            if (m->lattice) {
-                launch_wave_lattice<T>(m, in, out, K, Kf, dt, s);
-                continue;
-            }
-            wave_vel_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(
-                g, (const T*)in[0], (const T*)in[1], (const T*)in[2], (const T*)in[3], (T*)out[1], (T*)out[2],
-                (T*)out[3], T(dt));
-            check_launch();
-            wave_p_general_k<T><<<grid_for(g, kBlock), kBlock, 0, s>>>(
-                g, (const T*)out[1], (const T*)out[2], (const T*)out[3], (const T*)in[0], (T*)out[0], T(K),
-                (const T*)Kf, T(dt));
-            check_launch();
-        }
+        for (int64_t k = 0; k < nsteps; ++k)
+            launch_wave_faces<T>(m, (k & 1) ? b : a, (k & 1) ? a : b, K, Kf, dt, s);
         return;
     }
     launch_wave_march<T>(m, a, b, K, Kf, dt, nsteps, m->wave_variant, m->wave_ty, m->wave_L, m->wave_remap, s);

@@ -44,26 +44,28 @@ def test_wave_star(hip_ctx, oracle_lib, n, shift, dtype):
 
 
 def _mesh(hip_ctx, oracle_lib, n, kind, dtype):
-    """(star mesh, the same mesh in general form, oracle) of a uniform, decimal or graded lattice."""
+    """(star mesh, the same mesh in general form, oracle) of a uniform, decimal or graded lattice or a skewed mesh."""
     from cfdarcov2_amd import capi
     off, d = None, (0.125, 0.25, 0.5) if kind == "dyadic" else (0.1, 0.3, 0.7)
     if kind == "graded":  # vertex layers moved along their own axis
         g = np.meshgrid(*[0.05 * s * (np.arange(k + 1) % 3) for k, s in zip(n, d)], indexing="ij")
         off = np.stack([a.ravel() for a in g], axis=1)
+    elif kind == "skewed":
+        off = np.random.default_rng(8).uniform(-0.02, 0.02, ((n[0] + 1) * (n[1] + 1) * (n[2] + 1), 3))
     gm = capi.HexMesh(hip_ctx, *n, *d, dtype=dtype, vertex_offsets=off)
     gg = capi.HexMesh(hip_ctx, *n, *d, dtype=dtype, vertex_offsets=off, force_general=True)
     assert gg.info().uniform == 0
     if kind == "dyadic":
         assert gm.info().uniform == 1
-    elif min(n) > 3:  # (one or two layers can be exactly uniform) the lattice's tables are there
+    elif kind != "skewed" and min(n) > 3:  # (one or two layers can be exactly uniform) the lattice's tables are there
         assert gm.info().uniform == 0 and gm.info().device_bytes > gg.info().device_bytes
     return gm, gg, oracle_lib.OracleMesh(*n, *d, dtype=dtype, perturb=off)
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("kind", ["dyadic", "decimal", "graded"])
+@pytest.mark.parametrize("kind", ["dyadic", "decimal", "graded", "skewed"])
 @pytest.mark.parametrize("n", EXTENTS, ids=lambda n: "x".join(map(str, n)))
-def test_operators_and_heat_star(hip_ctx, oracle_lib, n, kind, dtype):
+def test_operators_and_steps_star(hip_ctx, oracle_lib, n, kind, dtype):
     gm, gg, om = _mesh(hip_ctx, oracle_lib, n, kind, dtype)
     rng = np.random.default_rng(5)
     phi = rng.standard_normal(om.N).astype(dtype)
@@ -79,6 +81,12 @@ def test_operators_and_heat_star(hip_ctx, oracle_lib, n, kind, dtype):
             A, B = _view(phi, dtype, shift), _view(phi, dtype, shift)
             got = gm.heat_run(A, B, 2e-3, 0.5, 5, alpha_field=None if a is None else _view(a, dtype, shift))
             assert np.array_equal(got.cpu().numpy(), om.heat_run(phi, 2e-3, 0.5, 5, alpha_field=a)), a is None
+        f = [phi, *(rng.standard_normal(om.N).astype(dtype) for _ in range(3))]
+        for k in (None, -af):
+            A, B = [[_view(a, dtype, shift) for a in f] for _ in range(2)]
+            got = gm.wave_run(A, B, -1.0, 0.02, 3, K_field=None if k is None else _view(k, dtype, shift))
+            for g, r in zip(got, om.wave_run(*f, -1.0, 0.02, 3, K_field=k)):
+                assert np.array_equal(g.cpu().numpy(), r), k is None
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
