@@ -72,7 +72,8 @@ void launch_wave_star_aux(const cfd_mesh_s* m, int mode, const void* const in[4]
             else with_mode(w, std::false_type{}, std::false_type{});
         }
     };
-    if (star::vector_form<T>(g.Y, g.Z)) with_geo(std::integral_constant<int, star::kWidth<T>>{});
+    if (star::vector_form<T>(g.Y, g.Z) && !star::narrow<T>(g.X * g.Y * g.Z))
+        with_geo(std::integral_constant<int, star::kWidth<T>>{});
     else with_geo(std::integral_constant<int, 1>{});
 }
 

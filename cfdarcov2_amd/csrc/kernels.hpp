@@ -63,6 +63,10 @@ template <class T> void launch_stab_star(const cfd_mesh_s* m, const void* phi, v
 template <class T>
 void launch_heat_star(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
                       hipStream_t s);
+constexpr int64_t kHeat2Cells = int64_t(1) << 18;  // the largest mesh that takes two heat steps per launch
+template <class T>
+void launch_heat2_star(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
+                       hipStream_t s);
 template <class T>
 void launch_grad_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s);
 template <class T> void launch_lapl_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s);

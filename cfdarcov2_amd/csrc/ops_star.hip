@@ -4,7 +4,7 @@
 // memory; PW: the cell volume is a power of two.
 //
 // Measured against one cell per thread with 64-bit indices: heat step 64^3
-// FP64 2.8 us against 3.5 (the launch and one memory round trip); gradient,
+// FP64 2.8 us against 3.5 (2.6 as one of two per launch); gradient,
 // Laplacian and stabilisation of 200^3 FP32 together 68 against 151 us.
 //
 // The arithmetic is the reference's (src/fvm3d.cpp:825-829,902-906 and
@@ -102,6 +102,95 @@ __global__ void __launch_bounds__(256) heat_star_k(UniformGeo<T> g, const T* __r
     star::store<T, W>(Tout + o.x0, o.o0, r);
 }
 
+// Two heat steps in one launch: a thread recomputes the first step's values of
+// its cells' neighbours (W + 2 cells of its row and W of each adjacent one)
+// from the rows up to two cells away, each with its own operation sequence, so
+// the bits are those of two launches. us per step against
+// one step per launch: 16^3 FP32 1.4 / 2.2, 48^3 1.7 / 2.5, 64^3 2.1 / 2.6,
+// 16^3 FP64 1.6 / 2.3, 64^3 2.65 / 2.85.  Bound by the launch (2 us) and by
+// one wavefront's serial work, so only for meshes that a launch outlasts: the
+// redundant steps make 80^3 (3.3 / 3.2 FP32, 4.5 / 3.8 FP64) slower.
+template <class T, int W, bool PW, bool AF>
+__global__ void __launch_bounds__(256) heat2_star_k(UniformGeo<T> g, const T* __restrict__ Tin,
+                                                    T* __restrict__ Tout, T alpha, const T* __restrict__ alpha_f,
+                                                    T dt, star::Plan pl) {
+    using star::load;
+    using star::load1;
+    using O = star::Off<W>;
+    star::Place q;
+    if (!star::place<W>(pl, q)) return;
+    const star::Offsets<W> o = star::offsets<W>(pl, q);
+    const VolDiv<T, PW> Vd{g.vol, g.inv_vol};
+    const int64_t SX = int64_t(pl.Y) * pl.Z;
+    const O uz = O(pl.Z), zl = O(o.o0 - o.zm1), zh = O(o.zp1 - o.o0);
+    // W values of a row with one cell on each side
+    auto wide = [&](const T* f, O off, T(&r)[W + 2]) {
+        T c[W];
+        load<T, W>(f, off, c);
+        r[0] = load1(f, O(off - zl));
+        r[W + 1] = load1(f, O(off + zh));
+#pragma unroll
+        for (int i = 0; i < W; ++i) r[i + 1] = c[i];
+    };
+    const T *const f0 = Tin + o.x0, *const fl = Tin + o.xm1, *const fh = Tin + o.xp1;
+    T c[W + 2], xl[W + 2], xh[W + 2], yl[W + 2], yh[W + 2];
+    T xl2[W], xh2[W], yl2[W], yh2[W], ll[W], lh[W], hl[W], hh[W];
+    wide(f0, o.o0, c);
+    wide(fl, o.o0, xl);
+    wide(fh, o.o0, xh);
+    wide(f0, o.ym1, yl);
+    wide(f0, o.yp1, yh);
+    const T zl2 = load1(f0, q.z0 >= 2 ? o.zm1 - 1 : o.zm1);
+    const T zh2 = load1(f0, q.z0 + W + 1 < pl.Z ? o.zp1 + 1 : o.zp1);
+    load<T, W>(q.x >= 2 ? fl - SX : fl, o.o0, xl2);
+    load<T, W>(q.x + 2 < pl.X ? fh + SX : fh, o.o0, xh2);
+    load<T, W>(f0, q.y >= 2 ? o.ym1 - uz : o.ym1, yl2);
+    load<T, W>(f0, q.y + 2 < pl.Y ? o.yp1 + uz : o.yp1, yh2);
+    load<T, W>(fl, o.ym1, ll);  // rows (x-1, y-1), (x-1, y+1), (x+1, y-1), (x+1, y+1)
+    load<T, W>(fl, o.yp1, lh);
+    load<T, W>(fh, o.ym1, hl);
+    load<T, W>(fh, o.yp1, hh);
+    T kc[W + 2], kxl[W], kxh[W], kyl[W], kyh[W];
+    if constexpr (AF) {
+        wide(alpha_f + o.x0, o.o0, kc);
+        load<T, W>(alpha_f + o.xm1, o.o0, kxl);
+        load<T, W>(alpha_f + o.xp1, o.o0, kxh);
+        load<T, W>(alpha_f + o.x0, o.ym1, kyl);
+        load<T, W>(alpha_f + o.x0, o.yp1, kyh);
+    }
+    auto step = [&](T pc, T a0, T a1, T b0, T b1, T d0, T d1, T k) {
+        const T lo[3] = {a0, b0, d0}, hi[3] = {a1, b1, d1};
+        T L = T(0);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const T s_lo = (-pc + lo[a]) * g.alpha[a];
+            const T s_hi = (-pc + hi[a]) * g.alpha[a];
+            L = L + Vd(s_lo * g.area[a] + s_hi * g.area[a]);
+        }
+        return dt * (k * L) + pc;
+    };
+    const bool wxl = q.x == 0, wxh = q.x == pl.X - 1, wyl = q.y == 0, wyh = q.y == pl.Y - 1;
+    T n[W + 2];  // the row after the first step
+#pragma unroll
+    for (int j = 0; j < W + 2; ++j)
+        n[j] = step(c[j], xl[j], xh[j], yl[j], yh[j], j ? c[j - 1] : zl2, j < W + 1 ? c[j + 1] : zh2,
+                    AF ? kc[j] : alpha);
+    if (q.z0 == 0) n[0] = n[1];
+    if (q.z0 + W == pl.Z) n[W + 1] = n[W];
+    T r[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        const int j = i + 1;
+        const T a0 = step(xl[j], xl2[i], c[j], ll[i], lh[i], xl[j - 1], xl[j + 1], AF ? kxl[i] : alpha);
+        const T a1 = step(xh[j], c[j], xh2[i], hl[i], hh[i], xh[j - 1], xh[j + 1], AF ? kxh[i] : alpha);
+        const T b0 = step(yl[j], ll[i], hl[i], yl2[i], c[j], yl[j - 1], yl[j + 1], AF ? kyl[i] : alpha);
+        const T b1 = step(yh[j], lh[i], hh[i], c[j], yh2[i], yh[j - 1], yh[j + 1], AF ? kyh[i] : alpha);
+        r[i] = step(n[j], wxl ? n[j] : a0, wxh ? n[j] : a1, wyl ? n[j] : b0, wyh ? n[j] : b1, n[j - 1], n[j + 1],
+                    AF ? kc[j] : alpha);
+    }
+    star::store<T, W>(Tout + o.x0, o.o0, r);
+}
+
 // StabVar on a uniform mesh (src/fvm3d.cpp:909-936) in one pass.  Per selected
 // axis: the Green-Gauss gradient of the cell and of its two neighbours on the
 // axis from phi at up to two cells away, the upwind face values
@@ -189,13 +278,13 @@ template <class T> const UniformGeo<T>& ug(const cfd_mesh_s* m) {
 
 // Calls f(plan, vector width, whether the volume is a power of two, geometry),
 // the two in the middle as integral constants.
-template <class T, class F> void with_star(const cfd_mesh_s* m, F f) {
+template <class T, class F> void with_star(const cfd_mesh_s* m, F f, bool narrow = false) {
     auto with_width = [&](auto w) {
         const star::Plan pl = star::make_plan(m->X, m->Y, m->Z, w());
         if (ug<T>(m).vol_pow2) f(pl, w, std::true_type{}, ug<T>(m));
         else f(pl, w, std::false_type{}, ug<T>(m));
     };
-    if (star::vector_form<T>(m->Y, m->Z)) with_width(std::integral_constant<int, star::kWidth<T>>{});
+    if (star::vector_form<T>(m->Y, m->Z) && !narrow) with_width(std::integral_constant<int, star::kWidth<T>>{});
     else with_width(std::integral_constant<int, 1>{});
     CFD_HIP(hipGetLastError());
 }
@@ -236,12 +325,29 @@ void launch_heat_star(const cfd_mesh_s* m, const void* in, void* out, double alp
     });
 }
 
+template <class T>
+void launch_heat2_star(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
+                       hipStream_t s) {
+    static_assert(kHeat2Cells <= int64_t(1) << 18, "two-step meshes are narrow in FP32");
+    with_star<T>(m, [&](const star::Plan& pl, auto w, auto pw, const auto& g) {
+        constexpr int W = decltype(w)::value;
+        constexpr bool PW = decltype(pw)::value;
+        if constexpr (sizeof(T) == 8 || W == 1) {  // FP32 is narrow wherever two steps are taken
+            auto* kern = af ? heat2_star_k<T, W, PW, true> : heat2_star_k<T, W, PW, false>;
+            kern<<<star::plan_grid(pl), star::plan_block(pl), 0, s>>>(g, (const T*)in, (T*)out, T(alpha),
+                                                                    (const T*)af, T(dt), pl);
+        }
+    }, star::narrow<T>(m->N));
+}
+
 #define CFD_INSTANTIATE(T)                                                                                         \
     template void launch_grad_star<T>(const cfd_mesh_s*, const void*, void*, int, int, hipStream_t);              \
     template void launch_lapl_star<T>(const cfd_mesh_s*, const void*, void*, int, hipStream_t);                   \
     template void launch_stab_star<T>(const cfd_mesh_s*, const void*, void*, int, hipStream_t);                   \
     template void launch_heat_star<T>(const cfd_mesh_s*, const void*, void*, double, const void*, double,         \
-                                      hipStream_t);
+                                      hipStream_t);                                                                \
+    template void launch_heat2_star<T>(const cfd_mesh_s*, const void*, void*, double, const void*, double,        \
+                                       hipStream_t);
 CFD_INSTANTIATE(float)
 CFD_INSTANTIATE(double)
 

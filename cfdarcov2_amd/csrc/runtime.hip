@@ -255,9 +255,12 @@ template <class T> static void create_mesh(cfd_mesh_s* m, const cfd_hex_desc& d)
         u.vol_pow2 = (u.vol > T(0) && std::frexp(u.vol, &ex) == T(0.5)) ? 1 : 0;
         u.inv_vol = T(1) / u.vol;
         m->uniform = true;
-        // two heat steps per launch on large meshes (256^3: 1.5-1.7x the
-        // per-thread kernel); small ones stay on the per-thread kernel
-        if (d.nx * d.ny * d.nz >= (int64_t(1) << 23) && heat_row_supported(d.nz, 12)) {
+        // Heat step.  The star form while both states fit the last-level cache
+        // (us/step, star / two steps per pass in row form: FP32 256^3 24 / 26,
+        // 512x256x256 43 / 47; FP64 256^3 44 / 45); beyond, its single steps
+        // cross memory and the row form's pairs halve that (FP32 1024x256x256
+        // 124 / 89; FP64 384x256x256 115 / 67).
+        if (2 * d.nx * d.ny * d.nz * int64_t(sizeof(T)) > kLastLevelCacheBytes && heat_row_supported(d.nz, 12)) {
             m->heat_variant = 1;
             m->heat_nw = 12;
             m->heat_L = 16;
@@ -265,7 +268,7 @@ template <class T> static void create_mesh(cfd_mesh_s* m, const cfd_hex_desc& d)
         // Acoustic step.  While both states (8 fields) fit the last-level
         // cache the star form is the fastest measured at every size and
         // extent (us/step, star / best row form / best march tiles; FP32
-        // 48^3: 4.0 / 5.2 / 6.5, 128^3: 14.5 / 14.3 / 20.2, 200^3: 42.7 /
+        // 48^3: 3.3 / 5.2 / 6.5, 128^3: 14.5 / 14.3 / 20.2, 200^3: 42.7 /
         // 48.6 / 63.7; FP64 128^3: 23.0 / 26.5 / 28.3); its re-read rows cost
         // it beyond (FP32 256^3: 155 / 71 / 140; FP64 200^3: 149 / 106 / 154).
         if (8 * d.nx * d.ny * d.nz * int64_t(sizeof(T)) <= kLastLevelCacheBytes) {

@@ -98,6 +98,16 @@ template <class T> inline bool vector_form(int64_t Y, int64_t Z) {
     return Z >= kWidth<T> && Y * Z * int64_t(sizeof(T)) < (int64_t(1) << 32);
 }
 
+// Whether a step of a mesh of this size is better with one cell per thread: a
+// launch then lasts about as long as one wavefront's chain of operations, and
+// the chain of W cells is longer than the chip needs to be filled (acoustic
+// step, us with one cell per thread / with vectors: FP32 16^3 2.4 / 2.9, 48^3
+// 2.8 / 3.3, 80^3 5.3 / 5.9, 100^3 8.6 / 8.0; FP64 16^3 2.4 / 3.0, 48^3 3.93 /
+// 3.98, 56^3 5.5 / 4.7).
+template <class T> inline bool narrow(int64_t cells) {
+    return cells <= (sizeof(T) == 4 ? int64_t(1) << 19 : int64_t(1) << 17);
+}
+
 // A thread's place: plane x (uniform), row y, first cell z0.  The first `skip`
 // of its cells belong to the unit before as well.
 struct Place {

@@ -121,6 +121,14 @@ void launch_heat(const cfd_mesh_s* m, void* Ta, void* Tb, double alpha, const vo
             launch_heat_row2<T>(g, Tb, Ta, alpha, dt, m->heat_nw, m->heat_L, s);
         }
     }
+    // meshes that a launch outlasts (heat2_star_k): two steps per launch, in
+    // pairs for the same reason
+    if (m->uniform && m->heat_variant == 0 && m->N <= kHeat2Cells) {
+        for (; k0 + 4 <= nsteps; k0 += 4) {
+            launch_heat2_star<T>(m, Ta, Tb, alpha, af, dt, s);
+            launch_heat2_star<T>(m, Tb, Ta, alpha, af, dt, s);
+        }
+    }
     for (int64_t k = k0; k < nsteps; ++k) {
         const T* in = (const T*)((k & 1) ? Tb : Ta);
         T* out = (T*)((k & 1) ? Ta : Tb);

@@ -2,7 +2,7 @@
 // star.hpp for the form and star_wave.hpp for the step.
 //
 // Bound by its arithmetic (104 operations per cell against the march's 59) and
-// the launch: 48^3 FP32 4.0 us/step, 128^3 FP32 14.5 (4.6 TB/s), 90x77x123
+// the launch: 48^3 FP32 2.8 us/step in a captured graph (3.3 launched one by one), 128^3 FP32 14.5 (4.6 TB/s), 90x77x123
 // FP64 12.0 us/step against 167 for the 16-row march tile, whose 30 workgroups
 // left most of the chip idle.
 #include <hip/hip_runtime.h>
@@ -38,7 +38,7 @@ template <class T>
 void launch_wave_star(const UniformGeo<T>& g, void* const* in, void* const* out, double K, const void* Kf, double dt,
                       hipStream_t s) {
     constexpr int W = star::kWidth<T>;
-    if (star::vector_form<T>(g.Y, g.Z)) {
+    if (star::vector_form<T>(g.Y, g.Z) && !star::narrow<T>(g.X * g.Y * g.Z)) {
         if (g.vol_pow2) launch_star<T, W, true>(g, in, out, K, Kf, dt, s);
         else launch_star<T, W, false>(g, in, out, K, Kf, dt, s);
     } else {

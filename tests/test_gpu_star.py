@@ -12,6 +12,8 @@ torch = pytest.importorskip("torch")
 # z extents around the vector widths (4 in FP32, 2 in FP64) and the workgroup's
 # units; x and y extents where a cell's two neighbours on each side are walls
 EXTENTS = [(1, 1, 1), (2, 1, 2), (3, 2, 3), (1, 3, 4), (5, 4, 5), (4, 5, 7), (2, 3, 130), (3, 2, 1030), (6, 67, 9)]
+# above the sizes that take one cell per thread: FP64, and both
+VECTOR = [(24, 90, 67), (40, 121, 131)]
 
 
 def _view(a, dtype, shift):
@@ -23,7 +25,7 @@ def _view(a, dtype, shift):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("n", EXTENTS, ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("n", EXTENTS + VECTOR, ids=lambda n: "x".join(map(str, n)))
 def test_wave_star(hip_ctx, oracle_lib, n, shift, dtype):
     from cfdarcov2_amd import capi
     d = (0.125, 0.25, 0.5) if shift else (0.125, 0.125, 0.125)
@@ -64,7 +66,7 @@ def _mesh(hip_ctx, oracle_lib, n, kind, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("kind", ["dyadic", "decimal", "graded", "skewed"])
-@pytest.mark.parametrize("n", EXTENTS, ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("n", EXTENTS + VECTOR[:1], ids=lambda n: "x".join(map(str, n)))
 def test_operators_and_steps_star(hip_ctx, oracle_lib, n, kind, dtype):
     gm, gg, om = _mesh(hip_ctx, oracle_lib, n, kind, dtype)
     rng = np.random.default_rng(5)
@@ -142,7 +144,7 @@ def test_perturbed_mesh_is_no_lattice(hip_ctx):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("every", [1, 2, 3, 9])
-@pytest.mark.parametrize("n", EXTENTS[1:] + [(600, 2, 5)], ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("n", EXTENTS[1:] + [(600, 2, 5), VECTOR[1]], ids=lambda n: "x".join(map(str, n)))
 def test_adjoint_star(hip_ctx, n, every, dtype):
     """Traces and gradients (K field and constant K, checkpoint segments of
     one to all steps, sensors in the first and last cells) against autograd
