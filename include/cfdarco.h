@@ -429,16 +429,17 @@ int cfd_mesh_geometry(cfd_mesh_t mesh, cfd_geometry* out);
 int cfd_mesh_set_wave_shape(cfd_mesh_t mesh, int variant, int tile_rows, int chunk, int xcd_remap);
 
 /* Kernel form of the heat step (cfd_heat_run) on exactly uniform meshes (no
- * counterpart in the reference): variant 0 = one thread per cell, one step per
- * launch; variant 1 = two steps per launch in row form (z extent a multiple of
+ * counterpart in the reference): variant 0 = star form (16 bytes of z-cells or
+ * one cell per thread), one step per launch, or two up to 2^18 cells (in pairs
+ * of launches); variant 1 = two steps per launch in row form (z extent a multiple of
  * 4 and at most 256, else CFD_E_UNSUPPORTED), `waves` (8, 12 or 16) waves per
  * workgroup and `chunk` x-planes per tile; runs go in pairs of launches, and
  * the remaining steps and runs with a diffusivity field take variant 0;
  * variant 2 = up to `chunk` (2 or 4) steps per launch in LDS boxes of `waves`
  * (4 or 8) x `waves` x min(Z, 64 - 2 chunk) output cells, each workgroup
- * computing its box widened by `chunk` cells for the steps in between; the
- * form for small meshes whose single step lasts about a launch.  All give bit-identical results.  Variant 1 pays on large meshes (it needs
- * enough tiles to fill the GPU): meshes of at least 2^23 cells that allow it
+ * computing its box widened by `chunk` cells for the steps in between,
+ * kept for comparison.  All give bit-identical results.  Meshes whose two
+ * states exceed the last-level cache (256 MiB) and whose z extent allows it
  * start on variant 1 (12 waves, 16 planes), others on variant 0;
  * cfdarcov2_amd/autotune.py:tune_heat times both. */
 int cfd_mesh_set_heat_shape(cfd_mesh_t mesh, int variant, int waves, int chunk);
