@@ -380,9 +380,13 @@ template <class T, class F> void with_faces(const cfd_mesh_s* m, F f) {
         if (m->lattice) f(pl, grid, block, w, std::integral_constant<int, 2>{}, lg<T>(m));
         else f(pl, grid, block, w, std::integral_constant<int, 3>{}, gg<T>(m));
     };
-    // (a plane's y- and z-faces are one row or column more than its cells, and
-    // their offsets are 32-bit in the vector form too)
-    if (m->Z >= star::kWidth<T> && star::vector_form<T>(m->Y + 1, m->Z + 1))
+    // One cell per thread on small meshes, by the uniform meshes' line (us per
+    // acoustic step with vectors / one cell: perturbed FP32 16^3 6.9 / 5.0, 64^3
+    // 10.6 / 8.8, lattice FP32 48^3 6.1 / 5.2, 80^3 9.7 / 9.0, 100^3 13.0 / 14.5;
+    // lattice FP64 32^3 5.4 / 4.8, 48^3 6.5 / 6.6, 64^3 7.7 / 9.5).
+    // (A plane's y- and z-faces are one row or column more than its cells, and
+    // their offsets are 32-bit in the vector form too.)
+    if (m->Z >= star::kWidth<T> && star::vector_form<T>(m->Y + 1, m->Z + 1) && !star::narrow<T>(m->N))
         with_width(std::integral_constant<int, star::kWidth<T>>{});
     else with_width(std::integral_constant<int, 1>{});
     CFD_HIP(hipGetLastError());

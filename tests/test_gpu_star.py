@@ -66,7 +66,7 @@ def _mesh(hip_ctx, oracle_lib, n, kind, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("kind", ["dyadic", "decimal", "graded", "skewed"])
-@pytest.mark.parametrize("n", EXTENTS + VECTOR[:1], ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("n", EXTENTS + VECTOR, ids=lambda n: "x".join(map(str, n)))
 def test_operators_and_steps_star(hip_ctx, oracle_lib, n, kind, dtype):
     gm, gg, om = _mesh(hip_ctx, oracle_lib, n, kind, dtype)
     rng = np.random.default_rng(5)
@@ -93,7 +93,7 @@ def test_operators_and_steps_star(hip_ctx, oracle_lib, n, kind, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("kind", ["decimal", "graded"])
-@pytest.mark.parametrize("n", EXTENTS, ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("n", EXTENTS + VECTOR, ids=lambda n: "x".join(map(str, n)))
 def test_lattice_equals_general_form(hip_ctx, oracle_lib, n, kind, dtype):
     """Every operator and step on a lattice against the general form of the
     same mesh, with infinities, NaN and values near the ends of the range
