@@ -255,7 +255,7 @@ def suite_sod(ctx, cpu=True, verbose=False):
     rec = {"workload": "Sod 512x64x64 perturbed (20% dx), FP32, Rusanov, CFL 0.3, 500 steps",
            "mcups": N * cfg.steps / wall / 1e6, "kernel_us_per_step": ev * 1e3 / cfg.steps,
            "gbs_algorithmic": gbs, "roofline_frac": gbs / HBM_PEAK_GBS, "nonfinite": int(bad),
-           "kernel": "euler_march_k" if shape["variant"] == 1 else "euler_step_k",
+           "kernel": "euler_step_k" if shape["variant"] == 0 else "euler_tile_k",  # rows of 64 cells fit every tile
            "kernel_shape": {k: shape[k] for k in ("variant", "tile_rows", "chunk")}}
     m.close()
     if cpu:

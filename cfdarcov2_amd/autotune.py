@@ -93,13 +93,26 @@ def tune_wave(mesh, steps: int = 20, candidates=None, use_cache: bool = True, ve
     return dict(best, table=table)
 
 
-EULER_CANDIDATES = [(0, 4, 16)] + [(1, ty, L) for ty in (2, 4, 8) for L in (8, 16, 32, 64)]
+# the tile by the mesh's size (which takes chunks of 1 to 32 planes) and set ones
+EULER_CANDIDATES = [(-1, 4, 16), (0, 4, 16)] + [(1, ty, L) for ty in (2, 4, 8) for L in (1, 2, 4, 8, 16, 32, 64)]
+
+
+def _best(table, key, automatic=-1):
+    """The fastest row of `table`; the row whose `key` is `automatic` unless a
+    set shape beats it by more than 3%, about what two timings of one shape
+    differ by: the automatic form also suits the calls that were not timed."""
+    best = min(table, key=lambda r: r["ms_per_step"])
+    for r in table:
+        if r[key] == automatic and r["ms_per_step"] <= 1.03 * best["ms_per_step"]:
+            return r
+    return best
 
 
 def tune_euler(mesh, U, gamma=1.4, cfl=0.3, steps=10, candidates=None, verbose=False) -> dict:
     """Pick the fastest Rusanov-step shape for `mesh` from runs on a copy of
     the state U (list of five device fields); the caller's fields are not
-    touched.  Returns the best shape and the table."""
+    touched.  Returns the best shape (variant -1: the size's own tile, see
+    _best) and the table."""
     import torch
 
     from .capi import CfdError
@@ -127,7 +140,7 @@ def tune_euler(mesh, U, gamma=1.4, cfl=0.3, steps=10, candidates=None, verbose=F
         table.append({"variant": variant, "tile_rows": ty, "chunk": L, "ms_per_step": ms})
         if verbose:
             print(f"  euler shape variant={variant} ty={ty} L={L}: {ms * 1e3:.1f} us/step", flush=True)
-    best = min(table, key=lambda r: r["ms_per_step"])
+    best = _best(table, "variant")
     mesh.set_euler_shape(best["variant"], best["tile_rows"], best["chunk"])
     del A, B
     return dict(best, table=table)

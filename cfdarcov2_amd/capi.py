@@ -380,6 +380,8 @@ class HexMesh:
         return T_a if nsteps % 2 == 0 else T_b
 
     def set_euler_shape(self, variant=1, tile_rows=4, chunk=16):
+        """Kernel form of euler_run: 0 = one thread per cell, 1 = march with this
+        tile, -1 = march with a tile by the mesh's size (the initial form)."""
         check(self.lib.cfd_mesh_set_euler_shape(self.h, int(variant), int(tile_rows), int(chunk)))
 
     def autotune(self, kind="wave", steps=10):

@@ -219,7 +219,7 @@ struct cfd_mesh_s {
     int hg_shape[3] = {-1, 0, 0};
     // Euler stepper: variant 0 = one thread per cell, 1 = march with
     // `euler_ty` x 64 cells x `euler_L` planes per workgroup, -1 = variant 1
-    // with a tile by the mesh's size
+    // with a tile by the mesh's size (euler_tile_shape)
     int euler_variant = -1;
     int euler_ty = 4;
     int euler_L = 16;

@@ -272,8 +272,9 @@ int cfd_euler_run(cfd_mesh_t mesh, void* const state_a[5], void* const state_b[5
  * with 64 * tile_rows (2, 4 or 8; 2 or 4 in FP64) cells of a plane per
  * workgroup, each cell's primitives computed once per plane and shared through
  * LDS: consecutive cells where two rows fit the tile (nz <= 32 * tile_rows),
- * tile_rows y-rows x 64 z-cells elsewhere.  Until a shape is set the tile
- * follows the mesh's size.  All give bit-identical results. */
+ * tile_rows y-rows x 64 z-cells elsewhere; -1 = variant 1 with the tile and the
+ * chunk by the mesh's size (tile_rows and chunk are checked and have no effect):
+ * the form of a mesh until a shape is set.  All give bit-identical results. */
 int cfd_mesh_set_euler_shape(cfd_mesh_t mesh, int variant, int tile_rows, int chunk);
 
 /* ---- adjoint of the fused acoustic step (uniform meshes; no reference
