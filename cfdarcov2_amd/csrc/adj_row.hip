@@ -111,16 +111,19 @@ template <class T> int adj_row_tile_rows(const cfd_mesh_s* m) { return m->adj_ty
 
 // Whether a run takes the row form: it was set, or no form was set and both
 // states (8 fields) exceed the last-level cache (without the K gradient) or
-// half of it (with it: the recomputed segment's fields want room too), and the
-// fields are aligned (16-byte rows in FP32, 32-byte in FP64).  Measured
+// reach half of it (with it: the recomputed segment's fields want room too),
+// and the fields are aligned (16-byte rows in FP32, 32-byte in FP64).  Measured
 // us/step, star / row form (4 rows, 8 planes): transposed step 128^3 FP32
-// 15.7 / 17.0, 160^3 FP64 51.8 / 67.7, 192^3 FP64 135 / 101; with the K
-// gradient 160^3 FP32 72.9 / 83.0, 128^3 FP64 73.4 / 70.0, 192^3 FP32 137 / 125.
+// 16.6 / 18.0, 256x256x128 FP32 45.8 / 48.7, 160^3 FP64 43.9 / 66.8, 192x192x128
+// FP64 84.7 / 71.6; with the K gradient, below half 128x160x128 FP32 41.0 /
+// 48.0 and 160x160x64 FP64 56.4 / 63.5, at half 256x256x64 FP32 73.0 / 67.2 and
+// 128^3 FP64 73.0 / 71.4, at all of it 256x256x128 FP32 171 / 137.
 template <class T>
 bool adj_row_usable(const cfd_mesh_s* m, const void* const* fields, int n, bool grad_K) {
     if (!m->uniform || !wave_row_supported(m->Z)) return false;
-    const int64_t room = grad_K ? kLastLevelCacheBytes / 2 - 1 : kLastLevelCacheBytes;
-    if (m->adj_form == 0 || (m->adj_form < 0 && 8 * m->N * int64_t(sizeof(T)) <= room)) return false;
+    const int64_t states = 8 * m->N * int64_t(sizeof(T));
+    const bool small = grad_K ? 2 * states < kLastLevelCacheBytes : states <= kLastLevelCacheBytes;
+    if (m->adj_form == 0 || (m->adj_form < 0 && small)) return false;
     for (int i = 0; i < n; ++i)
         if (fields[i] && !aligned4(fields[i], sizeof(T))) return false;
     return true;
