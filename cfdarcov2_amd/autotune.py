@@ -189,14 +189,16 @@ def tune_heat(mesh, alpha, dt, steps=100, candidates=None, verbose=False) -> dic
     return dict(best, table=table)
 
 
-ADJOINT_CANDIDATES = [(0, 4, 8)] + [(1, ty, L) for ty in (4, 8) for L in (2, 4, 8, 16, 32)]
+ADJOINT_CANDIDATES = [(-1, 4, 8), (0, 4, 8)] + [(1, ty, L) for ty in (4, 8) for L in (2, 4, 8, 16, 32)]
 
 
 def tune_adjoint(problem, steps=40, candidates=None, verbose=False, repeats=3) -> dict:
     """Pick the fastest kernel shape of the transposed acoustic step for the
     problem's mesh (constant K, no K gradient: the dL/dp0 path), from runs on
     scratch fields (best of `repeats` timed runs per shape, the shapes being
-    a few per cent apart); forms the mesh does not allow are skipped."""
+    a few per cent apart); forms the mesh does not allow are skipped.  The form
+    by size (-1), which differs with the K gradient, is kept unless a set shape
+    is clearly faster (_best)."""
     import torch
 
     from . import adjoint
@@ -224,6 +226,6 @@ def tune_adjoint(problem, steps=40, candidates=None, verbose=False, repeats=3) -
         table.append({"form": form, "tile_rows": ty, "chunk": L, "ms_per_step": ms})
         if verbose:
             print(f"  adjoint shape form={form} ty={ty} L={L}: {ms * 1e3:.1f} us/step", flush=True)
-    best = min(table, key=lambda r: r["ms_per_step"])
+    best = _best(table, "form")
     mesh.set_adjoint_shape(best["form"], best["tile_rows"], best["chunk"])
     return dict(best, table=table)

@@ -404,7 +404,8 @@ class HexMesh:
         check(self.lib.cfd_mesh_set_heat_shape(self.h, int(variant), int(waves), int(chunk)))
 
     def set_adjoint_shape(self, form=1, tile_rows=4, chunk=8):
-        """Kernel form of wave_traces / wave_adjoint: 0 = star form, 1 = row form."""
+        """Kernel form of wave_traces / wave_adjoint: 0 = star form, 1 = row form,
+        -1 = by the size of the fields, per call (the initial form)."""
         check(self.lib.cfd_mesh_set_adjoint_shape(self.h, int(form), int(tile_rows), int(chunk)))
 
     def wave_run(self, state_a, state_b, K, dt, nsteps, K_field=None):

@@ -1186,7 +1186,7 @@ int cfd_mesh_set_adjoint_shape(cfd_mesh_t m, int form, int tile_rows, int chunk)
     return guarded([&] {
         CFD_REQUIRE(m != nullptr, "null mesh");
         require_lattice(m, "cfd_mesh_set_adjoint_shape");
-        CFD_REQUIRE(form == 0 || form == 1, "adjoint form must be 0 or 1");
+        CFD_REQUIRE(form >= -1 && form <= 1, "adjoint form must be -1, 0 or 1");
         CFD_REQUIRE(chunk >= 1 && chunk <= 65535, "adjoint chunk must be in [1, 65535]");
         if (form == 1 && !(m->uniform && wave_row_supported(m->Z)))
             throw Error(CFD_E_UNSUPPORTED,

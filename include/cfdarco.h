@@ -327,9 +327,10 @@ int cfd_heat_adjoint(cfd_mesh_t mesh, void* adj_a, void* adj_b, double alpha, co
  * step needs a constant K (runs with a K field take form 0 for the transposed
  * steps).  Both record the traces in the step itself, keep one divergence
  * field per recomputed step for the K gradient and give bit-identical traces
- * and gradients.  Until a form is set, a run takes form 0 while both states (8
- * fields) fit 256 MiB (with the K gradient: half of that) and form 1 (4 waves,
- * 8 planes) beyond, where the mesh allows it. */
+ * and gradients.  Until a form is set, and again with form -1 (tile_rows and
+ * chunk then apply where it comes to form 1), a run takes form 0 while both
+ * states (8 fields) fit 256 MiB (with the K gradient: are below half of that)
+ * and form 1 (4 waves, 8 planes) beyond, where the mesh allows it. */
 int cfd_mesh_set_adjoint_shape(cfd_mesh_t mesh, int form, int tile_rows, int chunk);
 
 /* ---- batched ensemble (FP32 uniform meshes; no reference counterpart) -----

@@ -48,3 +48,31 @@ def test_euler_tuner_times_the_automatic_tile(hip_ctx, dtype):
     with pytest.raises(capi.CfdError):
         gm.set_euler_shape(-2, 4, 16)
     gm.close()
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_adjoint_tuner_times_the_form_by_size(hip_ctx, dtype):
+    """The form by size is among the candidates, and -1 returns a mesh to it:
+    the K gradient's path, which the tuner does not time, stays free to differ."""
+    torch = pytest.importorskip("torch")
+    from cfdarcov2_amd import adjoint, capi
+    n = (16, 12, 32)
+    gm = capi.HexMesh(hip_ctx, *n, 1 / 32, 1 / 32, 1 / 32, dtype=dtype)
+    pr = adjoint.WaveProblem(gm, np.array([0, 7, gm.N - 1]), 0.01, 6, K=-0.8)
+    p0 = torch.from_numpy(np.random.default_rng(0).standard_normal(gm.N).astype(dtype)).cuda()
+
+    def run():
+        tr, _, ck = adjoint.forward_traces(pr, p0)
+        return [tr, *adjoint.adjoint(pr, tr, None, ck, want_K=True)]
+
+    ref = run()
+    best = autotune.tune_adjoint(pr, steps=4)
+    auto = [r for r in best["table"] if r["form"] == -1]
+    assert len(auto) == 1 and best["ms_per_step"] <= auto[0]["ms_per_step"]
+    for shape in ((best["form"], best["tile_rows"], best["chunk"]), (1, 4, 2), (-1, 4, 8)):
+        gm.set_adjoint_shape(*shape)
+        assert all(torch.equal(a, b) for a, b in zip(run(), ref)), shape
+    with pytest.raises(capi.CfdError):
+        gm.set_adjoint_shape(-2, 4, 8)
+    gm.close()
