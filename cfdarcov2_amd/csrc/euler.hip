@@ -929,16 +929,39 @@ template <class T> static const FvAxis<T>* fv_axis(cfd_mesh_s* m, hipStream_t s)
     return &fa;
 }
 
+// The geometry that the mesh's shape reads, built where it is not there yet:
+// the axis-aligned form where it exists and the tiles take the mesh, else the
+// face arrays.
+template <class T> struct EulerGeometry {
+    const FvAxis<T>* axis = nullptr;
+    const FvGeo<T>* faces = nullptr;
+};
+template <class T> static EulerGeometry<T> euler_geometry(cfd_mesh_s* m, hipStream_t s) {
+    EulerGeometry<T> g;
+    const int rows = m->euler_variant < 0 ? (sizeof(T) == 4 ? 8 : 4) : m->euler_ty;
+    if (m->euler_variant != 0 && euler_tile_supported(m, rows)) g.axis = fv_axis<T>(m, s);
+    if (!g.axis) g.faces = &fv_geometry<T>(m, s);
+    return g;
+}
+
+// Builds what a newly set shape reads on a mesh that has run already, so that
+// its next run can be captured in a graph like any further run.
+template <class T> void euler_shape_changed(cfd_mesh_s* m) {
+    if (m->fv_block || m->fv_axis == 1) euler_geometry<T>(m, nullptr);
+}
+template void euler_shape_changed<float>(cfd_mesh_s*);
+template void euler_shape_changed<double>(cfd_mesh_s*);
+
 template <class T>
 void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamma, double cfl, int64_t nsteps,
                   void* dt_hist, hipStream_t s) {
     int ty = m->euler_ty, L = m->euler_L;
     const bool march = m->euler_variant != 0, chosen = m->euler_variant < 0;
-    const FvAxis<T>* axis = nullptr;
-    if (march && euler_tile_supported(m, chosen ? (sizeof(T) == 4 ? 8 : 4) : ty)) axis = fv_axis<T>(m, s);
+    const EulerGeometry<T> geo = euler_geometry<T>(m, s);
+    const FvAxis<T>* const axis = geo.axis;
+    const FvGeo<T>* const faces = geo.faces;
     if (chosen) euler_tile_shape(m, axis != nullptr, ty, L);
     const bool tile = march && euler_tile_supported(m, ty);
-    const FvGeo<T>* faces = axis ? nullptr : &fv_geometry<T>(m, s);
     Bits<T>* slots = (Bits<T>*)pool_alloc(m->ctx, 3 * kDtSet * sizeof(Bits<T>), s);
     try {
         const dim3 block(64, 4, 1);

@@ -112,6 +112,7 @@ template <class T>
 void launch_heat_multi(const UniformGeo<T>& g, const void* in, void* out, double alpha, double dt, int B, int K,
                        int ns, hipStream_t s);
 
+template <class T> void euler_shape_changed(cfd_mesh_s* m);
 template <class T>
 void launch_euler(cfd_mesh_s* m, void* const a[5], void* const b[5], double gamma, double cfl, int64_t nsteps,
                   void* dt_hist, hipStream_t s);

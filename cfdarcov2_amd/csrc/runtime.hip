@@ -1084,6 +1084,11 @@ int cfd_mesh_set_euler_shape(cfd_mesh_t m, int variant, int tile_rows, int chunk
         m->euler_variant = variant;
         m->euler_ty = tile_rows;
         m->euler_L = chunk;
+        try {
+            DISPATCH(m, euler_shape_changed, m);
+        } catch (const Error& e) {
+            if (e.code != CFD_E_NOMEM) throw;  // no room for it now: the run that needs it reports that
+        }
     });
 }
 

@@ -219,3 +219,38 @@ def test_euler_axis_aligned_equals_face_arrays(hip_ctx, kind):
                 gm.close()
             for k, (x, y) in enumerate(zip(*res)):
                 assert np.array_equal(x, y, equal_nan=True), (special, field, k)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["decimal", "dyadic"])
+@pytest.mark.parametrize("first,then", [((-1, 4, 16), (0, 4, 16)), ((1, 4, 2), (1, 2, 2)), ((0, 4, 16), (-1, 4, 16))],
+                         ids=["auto-cell", "tile-march", "cell-auto"])
+def test_euler_capture_after_a_change_of_shape(hip_ctx, first, then, kind, dtype):
+    """A mesh that has run once can change its shape (and with it the geometry
+    the kernels read) and have the next run captured: every replay, with eager
+    work and synchronisations between, equals the eager run."""
+    from cfdarcov2_amd import capi
+    n, d = (6, 5, 100), (0.125,) * 3 if kind == "dyadic" else (0.1, 0.07, 0.09)
+    gm = capi.HexMesh(hip_ctx, *n, *d, dtype=dtype)
+    rng = np.random.default_rng(3)
+    U0 = [1.0 + 0.3 * rng.random(gm.N), *(0.2 * rng.standard_normal((3, gm.N))), 3.0 + rng.random(gm.N)]
+    U0 = [torch.from_numpy(u.astype(dtype)).cuda() for u in U0]
+    A, B = [u.clone() for u in U0], [torch.empty_like(u) for u in U0]
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        gm.set_euler_shape(*first)
+        ref = [t.clone() for t in gm.euler_run(A, B, 1.4, 0.3, 4)]
+        gm.set_euler_shape(*then)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            gm.euler_run(A, B, 1.4, 0.3, 4)
+        for _ in range(3):
+            for a, u in zip(A, U0):
+                a.copy_(u)
+            graph.replay()
+            torch.randn(1 << 18, device="cuda").sum().item()
+            assert all(torch.equal(a, r) for a, r in zip(A, ref))
+    torch.cuda.synchronize()
+    del graph
+    gm.close()
