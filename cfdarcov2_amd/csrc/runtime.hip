@@ -228,8 +228,9 @@ template <class T> static bool upload_lattice(cfd_mesh_s* m, const HexGeometry<T
     const int64_t bytes = off[6] * int64_t(sizeof(T));
     try {
         m->lat_block = pool_alloc(m->ctx, bytes, s);
-    } catch (const Error&) {
-        return false;  // at the pool's limit the mesh does without the tables
+    } catch (const Error& e) {
+        if (e.code != CFD_E_NOMEM) throw;
+        return false;  // without room for them in the pool the mesh does without the tables
     }
     m->device_bytes += bytes;
     CFD_HIP(hipMemcpyAsync(m->lat_block, host.data(), size_t(bytes), hipMemcpyHostToDevice, s));

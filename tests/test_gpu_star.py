@@ -142,6 +142,32 @@ def test_perturbed_mesh_is_no_lattice(hip_ctx):
     assert gm.info().device_bytes == gg.info().device_bytes
 
 
+def test_lattice_without_room_for_its_tables(hip_ctx):
+    """A pool limit that holds the face arrays and no more: the mesh is made
+    without the tables, as before they existed, and gives the same results."""
+    from cfdarcov2_amd import capi
+    n, d = (7, 6, 9), (0.1, 0.3, 0.7)
+    ctx = capi.Context(0)
+    gm = capi.HexMesh(ctx, *n, *d, dtype="f64")
+    gg = capi.HexMesh(ctx, *n, *d, dtype="f64", force_general=True)
+    faces, both = gg.info().device_bytes, gm.info().device_bytes
+    assert both > faces
+    gg.close()
+    ctx.pool_set_limit(both + faces)
+    gl = capi.HexMesh(ctx, *n, *d, dtype="f64")
+    assert gl.info().device_bytes == faces
+    phi = torch.from_numpy(np.random.default_rng(1).standard_normal(gm.N)).cuda()
+    for op in ("grad", "lapl"):
+        assert torch.equal(getattr(gm, op)(phi), getattr(gl, op)(phi))
+    ctx.pool_set_limit(both + 2 * faces - 1)
+    with pytest.raises(capi.CfdError):
+        capi.HexMesh(ctx, *n, *d, dtype="f64")
+    torch.cuda.synchronize()
+    gl.close()
+    gm.close()
+    ctx.close()
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("every", [1, 2, 3, 9])
 @pytest.mark.parametrize("n", EXTENTS[1:] + [(600, 2, 5), VECTOR[1]], ids=lambda n: "x".join(map(str, n)))
