@@ -1,8 +1,9 @@
 // Batched ensemble of independent heat and acoustic cases (FP32, uniform
 // meshes; no reference counterpart).
 //
-// One launch advances every case by one step: the grid is the concatenation of
-// all cases' workgroups, each finds its case by a binary search over the cases'
+// One launch advances every case by one step (two in form 0 where large acoustic
+// cases take the march tiles): the grid is the concatenation of all cases'
+// workgroups, each finds its case by a binary search over the cases'
 // first-workgroup offsets (scalar loads of a small descriptor table) and runs
 // the same device code as the single-mesh kernels, so every case's fields equal
 // a plain single-case run bit for bit.  A run of n steps is captured once into
@@ -28,7 +29,8 @@ struct BatchCaseDev {
     float dt;
     int kind;            // CFD_CASE_HEAT / CFD_CASE_WAVE
     int nzt, nyt;
-    int64_t tile0;       // first tile of the case in the batched grid (row forms)
+    int march;           // form 0: the case takes march tiles
+    int64_t tile0;       // first tile of the case in the batched grid (row forms, march tiles)
     float* a[4];
     float* b[4];
     // star form: workgroups of 256 threads, `star_wg` of them (a multiple of
@@ -82,6 +84,43 @@ __global__ void __launch_bounds__(256) batch_star_k(const BatchCaseDev* __restri
         if (cs.g.vol_pow2) batch_star_cells<W, true>(cs, parity, tx, ty);
         else batch_star_cells<W, false>(cs, parity, tx, ty);
     }
+}
+
+// Form 0 of acoustic cases whose own states exceed the last-level cache: 2.5D
+// march tiles, which read each plane once from memory where the star form reads
+// neighbouring rows again, unless their columns of 64 z-cells would idle more
+// than an eighth of the lanes.  us/step, march (4 rows, 8 planes) / star: one
+// 256^3 case 136 / 159, 300^3 253 / 260, three of 224^3 287 / 306; with idle
+// lanes 208^3 95 / 80, 260^3 175 / 167; within the cache three of 200^3 199 / 112.
+static bool takes_march(const BatchCaseDev& c) {
+    const int64_t columns = (c.g.Z + 63) / 64 * 64;
+    return c.kind == CFD_CASE_WAVE && 8 * c.g.Z >= 7 * columns &&
+           8 * c.g.X * c.g.Y * c.g.Z * int64_t(sizeof(float)) > kLastLevelCacheBytes;
+}
+template <int TYT, int R>
+__global__ void __launch_bounds__(64 * TYT) batch_march_k(const BatchCaseDev* __restrict__ cases, int ncases,
+                                                          int parity, int L) {
+    __shared__ MarchLds<float, TYT, R> lds;
+    const int64_t tile = blockIdx.x;
+    int lo = 0, hi = ncases - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (cases[mid].tile0 <= tile) lo = mid;
+        else hi = mid - 1;
+    }
+    const BatchCaseDev& cs = cases[lo];
+    const int64_t t = tile - cs.tile0;
+    const int64_t zt = t % cs.nzt;
+    const int64_t yt = (t / cs.nzt) % cs.nyt;
+    const int64_t xc = t / (int64_t(cs.nzt) * cs.nyt);
+    float* const* in = parity ? cs.b : cs.a;
+    float* const* out = parity ? cs.a : cs.b;
+    if (cs.g.vol_pow2)
+        wave_march_tile<float, TYT, R, false, true>(cs.g, in[0], in[1], in[2], in[3], out[0], out[1], out[2], out[3],
+                                                    cs.coef, nullptr, cs.dt, L, zt, yt, xc, lds);
+    else
+        wave_march_tile<float, TYT, R, false, false>(cs.g, in[0], in[1], in[2], in[3], out[0], out[1], out[2], out[3],
+                                                     cs.coef, nullptr, cs.dt, L, zt, yt, xc, lds);
 }
 
 // Row form of the batched step (form 1): every case's z extent is a multiple
@@ -206,7 +245,7 @@ struct cfd_batch_s {
     BatchCaseDev* dev = nullptr;
     int tile_rows = 4;
     int chunk = 8;
-    int form = 0;  // 0: star form, 1: row form, 2: row form, two steps per launch
+    int form = 0;  // 0: star form and march tiles, 1: row form, 2: row form, two steps per launch
     int star_wg = 0;  // workgroups of the star form
     int64_t total_tiles = 0;
     // form 2: single-step row-form layout (4-row tiles) for the steps left after
@@ -245,6 +284,10 @@ static void check_form2(const std::vector<BatchCaseDev>& cases, int T) {
 static int64_t layout_into(std::vector<BatchCaseDev>& cases, int form, int T, int L) {
     int64_t off = 0;
     for (auto& c : cases) {
+        if (form == 0 && !c.march) {  // no tiles: the search passes over it
+            c.tile0 = off;
+            continue;
+        }
         c.nzt = form >= 1 ? 1 : int((c.g.Z + 63) / 64);  // a row-form tile spans the z row
         const int64_t rows = tile_rows_of(c, form, T);
         CFD_REQUIRE(rows >= 1, "batch tile without output rows");
@@ -257,10 +300,15 @@ static int64_t layout_into(std::vector<BatchCaseDev>& cases, int form, int T, in
     return off;
 }
 
-// The star form's workgroups.
+// The star form's workgroups (none for a case that takes march tiles).
 static void star_layout(cfd_batch_s* b) {
     int64_t wg = 0;
     for (auto& c : b->host) {
+        c.march = takes_march(c);
+        if (c.march) {
+            c.star0 = int(wg);
+            continue;
+        }
         c.star_width = star::vector_form<float>(c.g.Y, c.g.Z) ? star::kWidth<float> : 1;
         c.plan = star::make_plan(c.g.X, c.g.Y, c.g.Z, c.star_width, 256);
         c.star0 = int(wg);
@@ -305,7 +353,15 @@ static void batch_launch(const cfd_batch_s* b, int parity, hipStream_t s) {
         }
         return;
     }
-    batch_star_k<<<dim3(unsigned(b->star_wg)), 256, 0, s>>>(b->dev, n, parity);
+    if (b->star_wg) batch_star_k<<<dim3(unsigned(b->star_wg)), 256, 0, s>>>(b->dev, n, parity);
+    if (b->total_tiles) {
+        switch (b->tile_rows) {
+            case 4: batch_march_k<4, 1><<<grid, dim3(64, 4), 0, s>>>(b->dev, n, parity, b->chunk); break;
+            case 8: batch_march_k<4, 2><<<grid, dim3(64, 4), 0, s>>>(b->dev, n, parity, b->chunk); break;
+            case 16: batch_march_k<4, 4><<<grid, dim3(64, 4), 0, s>>>(b->dev, n, parity, b->chunk); break;
+            default: throw Error(CFD_E_INVALID, "batch tile rows must be 4, 8 or 16");
+        }
+    }
 }
 
 // nsteps steps from state_a: in form 2, pairs of two-step launches (a -> b ->

@@ -73,8 +73,9 @@ class Ensemble:
     def configure(self, tile_rows=4, chunk=8, group_bytes=0, form=0):
         """Pack cases into groups of at most `group_bytes` of fields (0: one
         group), largest first, and set the tile form (0: star form, which takes
-        any extents and no shape, 1:
-        row form, 2: row form with two steps per launch) and shape."""
+        any extents and no shape, with march tiles of this shape for large
+        acoustic cases, 1: row form, 2: row form with two steps per
+        launch) and shape."""
         self._destroy_groups()
         order = sorted(range(len(self.cases)), key=lambda i: -self.cases[i].nbytes)
         packs, cur, cur_b = [], [], 0

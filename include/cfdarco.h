@@ -353,7 +353,8 @@ typedef struct cfd_batch_case {
 } cfd_batch_case;
 int cfd_batch_create(cfd_ctx_t ctx, const cfd_batch_case* cases, int ncases, cfd_batch_t* out);
 /* Tile form: 0 = star form (any extents; the default; tile_rows 4, 8 or 16 and
- * chunk are taken and have no effect on it), 1 = row form (256/Z z rows per wave, tile_rows
+ * chunk are taken and shape the march tiles of 64 z-columns that acoustic cases
+ * with more than 256 MiB of fields take where z fills 7/8 of the columns), 1 = row form (256/Z z rows per wave, tile_rows
  * 4 or 8 output waves + 2 halo waves per workgroup; every case's z extent a
  * multiple of 4 and at most 256 and its fields 16-byte aligned, else
  * CFD_E_UNSUPPORTED), 2 = row form with two steps per launch (tile_rows = 8, 10

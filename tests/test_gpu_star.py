@@ -243,3 +243,40 @@ def test_batch_star_mixed_extents(hip_ctx):
             for g, r in zip(a, ref):
                 assert torch.equal(g, r), (k, graph)
     capi.check(hip_ctx.lib.cfd_batch_destroy(h))
+
+
+def test_batch_with_a_case_beyond_the_cache(hip_ctx):
+    """Form 0 of a batch whose acoustic case exceeds the last-level cache (march
+    tiles, at each of their shapes) between cases that do not (star form), in
+    every order of the descriptors: each equals its single-case run."""
+    import ctypes
+    import itertools
+
+    from cfdarcov2_amd import capi
+    rng = np.random.default_rng(4)
+    cases = []
+    for n, heat in (((191, 187, 250), False), ((9, 7, 33), False), ((16, 12, 20), True)):
+        m = capi.HexMesh(hip_ctx, *n, 0.125, 0.125, 0.125, dtype="f32")
+        a0 = [torch.from_numpy(rng.standard_normal(m.N, dtype=np.float32)).cuda() for _ in range(1 if heat else 4)]
+        a, b = [t.clone() for t in a0], [torch.empty_like(t) for t in a0]
+        ref = [m.heat_run(a[0], b[0], 1e-3, 0.02, 4)] if heat else m.wave_run(a, b, -0.8, 0.02, 4)
+        cases.append((m, heat, a0, a, b, [t.clone() for t in ref]))
+    assert 8 * 4 * cases[0][0].N > 256 << 20
+    shapes = itertools.cycle([(4, 8), (8, 5), (16, 32)])
+    for order in itertools.permutations(range(3)):
+        arr = (capi.BatchCase * 3)()
+        for c, i in zip(arr, order):
+            m, heat, a0, a, b, _ = cases[i]
+            c.mesh, c.kind, c.coef, c.dt = m.h, 0 if heat else 1, 1e-3 if heat else -0.8, 0.02
+            for f in range(len(a0)):
+                a[f].copy_(a0[f])
+                c.state_a[f], c.state_b[f] = a[f].data_ptr(), b[f].data_ptr()
+        h = ctypes.c_void_p()
+        capi.check(hip_ctx.lib.cfd_batch_create(hip_ctx.h, arr, 3, ctypes.byref(h)))
+        shape = next(shapes)
+        capi.check(hip_ctx.lib.cfd_batch_set_shape(h, *shape))
+        capi.check(hip_ctx.lib.cfd_batch_run(h, 4, order[0] % 2, capi._stream_ptr()))
+        for i in order:
+            for g, r in zip(cases[i][3], cases[i][5]):
+                assert torch.equal(g, r), (order, shape, i)
+        capi.check(hip_ctx.lib.cfd_batch_destroy(h))
