@@ -248,6 +248,9 @@ struct cfd_batch_s {
     int form = 0;  // 0: star form and march tiles, 1: row form, 2: row form, two steps per launch
     int star_wg = 0;  // workgroups of the star form
     int64_t total_tiles = 0;
+    bool march = false;  // a case takes march tiles in form 0
+    // whether the tile shape is part of the launches: not where every case takes the star form
+    bool shaped() const { return form != 0 || march; }
     // form 2: single-step row-form layout (4-row tiles) for the steps left after
     // the pairs of two-step launches
     std::vector<BatchCaseDev> host1;
@@ -306,6 +309,7 @@ static void star_layout(cfd_batch_s* b) {
     for (auto& c : b->host) {
         c.march = takes_march(c);
         if (c.march) {
+            b->march = true;
             c.star0 = int(wg);
             continue;
         }
@@ -483,7 +487,7 @@ int cfd_batch_set_shape(cfd_batch_t b, int tile_rows, int chunk) {
         if (tile_rows != b->tile_rows || chunk != b->chunk) {
             b->tile_rows = tile_rows;
             b->chunk = chunk;
-            b->dirty = true;
+            if (b->shaped()) b->dirty = true;
         }
     });
 }
@@ -509,7 +513,8 @@ int cfd_batch_run(cfd_batch_t b, int64_t nsteps, int use_graph, void* stream) {
         // a replay starts from state_a again, so the state must end there
         CFD_REQUIRE(nsteps % 2 == 0, "cfd_batch_run: graph runs need an even step count");
         if (nsteps == 0) return;
-        const auto key = std::make_tuple(nsteps, b->tile_rows * 4 + b->form, b->chunk);
+        const auto key = b->shaped() ? std::make_tuple(nsteps, b->tile_rows * 4 + b->form, b->chunk)
+                                     : std::make_tuple(nsteps, 0, 0);
         auto it = b->graphs.find(key);
         if (it == b->graphs.end()) {
             hipGraph_t graph = nullptr;

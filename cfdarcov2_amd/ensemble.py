@@ -150,16 +150,24 @@ def time_gpu(fn, reps=1):
     return best
 
 
+def tune_candidates(specs):
+    """The (tile_rows, chunk, group_bytes, form) that autotune times.  Form 0
+    has a shape only where an acoustic case is beyond 256 MiB of fields."""
+    shaped = any(sp.kind == "wave" and 32 * sp.n ** 3 > 256 << 20 for sp in specs)
+    shapes = [(ty, L) for ty in (4, 8, 16) for L in (8, 16, 32)] if shaped else [(4, 8)]
+    candidates = [(ty, L, gb, 0) for ty, L in shapes for gb in (0, 96 << 20, 192 << 20)]
+    candidates += [(ty, L, gb, 1) for ty in (4, 8) for L in (4, 8, 16, 32)
+                   for gb in (0, 96 << 20, 192 << 20)]
+    candidates += [(nw, L, gb, 2) for nw in (8, 10, 12) for L in (8, 16, 32)
+                   for gb in (0, 192 << 20)]
+    return candidates
+
+
 def autotune(ens: Ensemble, steps=20, candidates=None, verbose=False):
-    """Pick (tile_rows, chunk, group_bytes) by timing graph runs of `steps`
+    """Pick (tile_rows, chunk, group_bytes, form) by timing graph runs of `steps`
     steps; leaves the ensemble configured with the winner and its state reset."""
     if candidates is None:
-        candidates = [(ty, L, gb, 0) for ty in (4, 8, 16) for L in (8, 16, 32)
-                      for gb in (0, 96 << 20, 192 << 20)]
-        candidates += [(ty, L, gb, 1) for ty in (4, 8) for L in (4, 8, 16, 32)
-                       for gb in (0, 96 << 20, 192 << 20)]
-        candidates += [(nw, L, gb, 2) for nw in (8, 10, 12) for L in (8, 16, 32)
-                       for gb in (0, 192 << 20)]
+        candidates = tune_candidates([c.spec for c in ens.cases])
     results = []
     for cand in candidates:
         ty, L, gb = cand[:3]

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-# (tile_rows, chunk, group_bytes, form): 2.5D march tiles, single-step row
+# (tile_rows, chunk, group_bytes, form): star form, single-step row
 # tiles, two-step row tiles in one group and in cache-sized groups
 SHAPES = [(8, 16, 0, 0), (8, 16, 0, 1), (12, 16, 0, 2), (10, 16, 192 << 20, 2)]
 

@@ -15,6 +15,17 @@ def test_best_keeps_the_automatic_form_within_noise():
     assert autotune._best(rows(1.05, 3.0, 1.0)[1:], "variant")["variant"] == 1
 
 
+def test_batch_candidates_hold_no_launch_twice():
+    """Form 0 is timed once per group size, unless a case takes its tiles."""
+    from types import SimpleNamespace as S
+
+    from cfdarcov2_amd.ensemble import tune_candidates
+    small = [S(kind="wave", n=128), S(kind="heat", n=300)]
+    form0 = [c for c in tune_candidates(small) if c[3] == 0]
+    assert len(form0) == len({c[2] for c in form0}) == 3
+    assert len([c for c in tune_candidates(small + [S(kind="wave", n=256)]) if c[3] == 0]) == 27
+
+
 def _euler_state(torch, N, dtype):
     rng = np.random.default_rng(2)
     U = np.stack([1.0 + 0.3 * rng.random(N), *(0.1 * rng.standard_normal((3, N))), 3.0 + rng.random(N)])
