@@ -179,7 +179,7 @@ ROW_CASES = [((20, 18, 64), (4, 8)), ((13, 11, 256), (8, 3)), ((9, 30, 32), (4, 
 def test_row_form_equals_per_thread_form(hip_ctx, dtype, n, shape):
     """The row-form forward (traces recorded in the fused step) and transposed
     step (trace gradients added in the step, K gradient from one divergence
-    field per recomputed step) against the per-thread kernels, bit for bit:
+    field per recomputed step) against the star form, bit for bit:
     traces, checkpoints, dL/dp0 and dL/dK, constant K, with sensors on the
     walls, the corners and chunk borders, an uneven last checkpoint segment
     and an odd step count."""
@@ -198,7 +198,7 @@ def test_row_form_equals_per_thread_form(hip_ctx, dtype, n, shape):
     if dtype == np.float64:
         shape = (4, shape[1])  # FP64 row tiles have 4 output waves (the 8-row builds spill)
     for form in (0, 1):
-        print(f"\n[case] adjoint row vs per-thread n={n} shape={shape} dtype={dtype.__name__} form={form}", flush=True)
+        print(f"\n[case] adjoint row vs star n={n} shape={shape} dtype={dtype.__name__} form={form}", flush=True)
         pr = _problem(hip_ctx, n, d, dt, steps, sens, every=4, dtype=dtype, K=K)
         pr.mesh.set_adjoint_shape(form, *shape)
         tr, final, ck = adjoint.forward_traces(pr, p0, checkpoints=True)
@@ -220,8 +220,9 @@ def test_row_form_equals_per_thread_form(hip_ctx, dtype, n, shape):
 
 def test_constant_K_gradient_equals_K_field_gradient(hip_ctx):
     """dL/dK at a constant K through the row form (constant-K transposed
-    steps) equals the gradient at the equal K field (per-thread transposed
-    steps with a K field), bit for bit."""
+    steps) equals the gradient at the equal K field (star-form transposed
+    steps with a K field after the row form's forward), bit for bit, and both
+    equal the star form throughout."""
     from cfdarcov2_amd import adjoint
     n, d = (24, 20, 32), (1 / 32,) * 3
     N = n[0] * n[1] * n[2]
@@ -231,15 +232,17 @@ def test_constant_K_gradient_equals_K_field_gradient(hip_ctx):
     pr = _problem(hip_ctx, n, d, 0.4 / 32, 16, sens, every=5, dtype=np.float64, K=K)
     p0 = torch.from_numpy(rng.standard_normal(N)).cuda()
     Kf = torch.full((N,), K, dtype=torch.float64, device="cuda")
-    print("\n[case] constant-K gradient vs K-field gradient", flush=True)
-    tr, _, ck = adjoint.forward_traces(pr, p0, checkpoints=True)
-    trf, _, ckf = adjoint.forward_traces(pr, p0, Kf, checkpoints=True)
-    assert torch.equal(tr, trf) and torch.equal(ck, ckf)
-    g = torch.from_numpy(rng.standard_normal(tuple(tr.shape))).cuda()
-    gp, gK = adjoint.adjoint(pr, g, None, ck, want_K=True)
-    gpf, gKf = adjoint.adjoint(pr, g, Kf, ckf, want_K=True)
-    torch.cuda.synchronize()
-    assert torch.equal(gp, gpf) and torch.equal(gK, gKf)
+    g = torch.from_numpy(rng.standard_normal((16, 20))).cuda()
+    ref = None
+    for form in (1, 0):
+        print(f"\n[case] constant-K gradient vs K-field gradient form={form}", flush=True)
+        pr.mesh.set_adjoint_shape(form, 4, 8)
+        for kf in (None, Kf):
+            tr, _, ck = adjoint.forward_traces(pr, p0, kf, checkpoints=True)
+            got = [tr, ck, *adjoint.adjoint(pr, g, kf, ck, want_K=True)]
+            torch.cuda.synchronize()
+            ref = ref or got
+            assert all(torch.equal(a, b) for a, b in zip(got, ref)), (form, kf is None)
 
 
 

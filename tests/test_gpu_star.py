@@ -131,12 +131,97 @@ def test_lattice_equals_general_form(hip_ctx, oracle_lib, n, kind, dtype):
                 assert same(g, r)
 
 
+def _uniform_ops(phi, h):
+    """Gradient, Laplacian and stabilisation of (X, Y, Z) values on a uniform
+    mesh of power-of-two spacings, in the scheme's operation order."""
+    T = phi.dtype.type
+    V = T(h[0] * h[1] * h[2])
+    lo = lambda f, a: np.concatenate([f.take([0], a), f.take(range(f.shape[a] - 1), a)], a)
+    hi = lambda f, a: np.concatenate([f.take(range(1, f.shape[a]), a), f.take([-1], a)], a)
+    grad, lapl, stab = (np.zeros_like(phi) for _ in range(3))
+    for a in range(3):
+        A, al, L = T(h[0] * h[1] * h[2] / h[a]), T(1 / h[a]), T(h[a] / 2)
+        g = (-((phi + lo(phi, a)) * T(0.5)) * A + (phi + hi(phi, a)) * T(0.5) * A) / V
+        grad = grad + g
+        lapl = lapl + ((-phi + lo(phi, a)) * al * A + (-phi + hi(phi, a)) * al * A) / V
+        f_lo = T(0.5) * ((phi + L * g * T(-1)) - (lo(phi, a) + L * lo(g, a)))
+        f_hi = T(0.5) * ((phi + L * g) - (hi(phi, a) + L * hi(g, a) * T(-1)))
+        stab = stab + (f_lo * A + f_hi * A) / V
+    return grad, lapl, stab
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [(3, 2, 3), (5, 4, 8), (16, 12, 32), (40, 121, 132)], ids=lambda n: "x".join(map(str, n)))
+def test_uniform_nonfinite(hip_ctx, n, dtype):
+    """Infinities, NaN and values near the ends of the range on a uniform mesh:
+    the operators against their definition, the acoustic step against the
+    march tiles, the heat step (one and two per launch) against the LDS boxes,
+    the adjoint against the row form: the same bits, NaN in the same places."""
+    from cfdarcov2_amd import adjoint, capi
+    h = (0.125, 0.25, 0.5)
+    gm = capi.HexMesh(hip_ctx, *n, *h, dtype=dtype)
+    assert gm.info().uniform == 1
+    N = gm.N
+    rng = np.random.default_rng(7)
+    special = np.array([np.inf, -np.inf, np.nan, np.finfo(dtype).max, -np.finfo(dtype).max,
+                        np.finfo(dtype).smallest_subnormal, -0.0], dtype=dtype)
+
+    def field():
+        f = rng.standard_normal(N).astype(dtype)
+        f[rng.integers(N, size=max(2, N // 60))] = rng.choice(special, size=max(2, N // 60))
+        return f
+
+    def same(a, b):
+        a, b = (x.cpu().numpy() if torch.is_tensor(x) else x for x in (a, b))
+        return np.array_equal(a, b, equal_nan=True)
+
+    phi = field()
+    with np.errstate(all="ignore"):
+        ref = [r.reshape(-1) for r in _uniform_ops(phi.reshape(n), h)]
+    t = _view(phi, dtype, 1)
+    for name, r in zip(("grad", "lapl", "stab"), ref):
+        assert same(getattr(gm, name)(t), r), name
+
+    def heat(shape, steps, af=None):
+        gm.set_heat_shape(*shape)
+        return gm.heat_run(_view(phi, dtype, 0), _view(phi, dtype, 0), 2e-3, 0.5, steps, alpha_field=af)
+
+    for steps in (1, 4, 6):
+        assert same(heat((0, 8, 16), steps), heat((2, 4, 2), steps)), steps
+    af = _view(np.abs(field()), dtype, 0)
+    x = [_view(phi, dtype, 0), _view(phi, dtype, 0)]
+    for k in range(4):  # single steps against two per launch, with an alpha field
+        x.reverse() if k else None
+        gm.heat_run(*x, 2e-3, 0.5, 1, alpha_field=af)
+    assert same(heat((0, 8, 16), 4, af), x[1])
+
+    f = [field() for _ in range(4)]
+    for kf in (None, _view(-np.abs(field()), dtype, 0)):
+        out = []
+        for shape in ((0, 4, 8, 0), (1, 4, 8, 0)):
+            gm.set_wave_shape(*shape)
+            out.append(gm.wave_run([_view(a, dtype, 0) for a in f], [_view(a, dtype, 0) for a in f], -1.0, 0.02, 3,
+                                   K_field=kf))
+        assert all(same(a, b) for a, b in zip(*out)), kf is None
+    if n[2] % 4 == 0:
+        pr = adjoint.WaveProblem(gm, np.array([0, N // 2, N - 1]), 0.02, 5, K=-1.0, every=2)
+        out, g = [], torch.from_numpy(rng.standard_normal((5, 3)).astype(dtype)).cuda()
+        g[2, 1] = float("inf")
+        for form in (0, 1):
+            gm.set_adjoint_shape(form, 4, 8)
+            tr, _, ck = adjoint.forward_traces(pr, _view(f[0], dtype, 0))
+            out.append([tr, *adjoint.adjoint(pr, g, None, ck, want_K=True)])
+        assert all(same(a, b) for a, b in zip(*out))
+    gm.close()
+
+
 def test_perturbed_mesh_is_no_lattice(hip_ctx):
-    """One vertex moved by one unit in the last place: the general form."""
+    """One vertex moved by one unit in the last place of its coordinate (0.9),
+    which reaches the face normals: the general form."""
     from cfdarcov2_amd import capi
     n, d = (5, 4, 6), (0.1, 0.3, 0.7)
     off = np.zeros(((n[0] + 1) * (n[1] + 1) * (n[2] + 1), 3))
-    off[2 * 5 * 7 + 2 * 7 + 3, 1] = 2.0 ** -40
+    off[2 * 5 * 7 + 3 * 7 + 3, 1] = np.spacing(3 * d[1])
     gm = capi.HexMesh(hip_ctx, *n, *d, dtype="f64", vertex_offsets=off)
     gg = capi.HexMesh(hip_ctx, *n, *d, dtype="f64", vertex_offsets=off, force_general=True)
     assert gm.info().device_bytes == gg.info().device_bytes
