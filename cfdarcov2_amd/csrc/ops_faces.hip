@@ -42,11 +42,11 @@ template <class T> struct FaceArg<T, 3> { using type = GeneralGeo<T>; };
 // axis of local face fc
 __device__ constexpr int axis_of(int fc) { return 2 - (fc >> 1); }
 
-template <class T, int W, int GEO> struct CellGeo;
+template <class T, int W, int GEO, class O> struct CellGeo;
 
-template <class T, int W> struct CellGeo<T, W, 2> {
+template <class T, int W, class O> struct CellGeo<T, W, 2, O> {
     star::LatticeCells<T, W> c;
-    __device__ CellGeo(const LatticeGeo<T>& g, const Plan&, const Place& q, const Offsets<W>& o)
+    __device__ CellGeo(const LatticeGeo<T>& g, const Plan&, const Place& q, const Offsets<W, O>& o)
         : c(star::load_lattice<T, W, true>(g, o, q)) {}
     __device__ void alphas(T (&al)[6][W]) const {
 #pragma unroll
@@ -73,13 +73,12 @@ template <class T, int W> struct CellGeo<T, W, 2> {
     }
 };
 
-template <class T, int W> struct CellGeo<T, W, 3> {
-    using O = star::Off<W>;
+template <class T, int W, class O> struct CellGeo<T, W, 3, O> {
     const GeneralGeo<T>& g;
     int64_t zb, yb, xb, SX;  // plane bases of the z-, y- and x-faces
     O zo, co, Z;             // the first cell's z-face, and its cell and lower y- and x-face, within a plane
     T A[6][W], V[W];
-    __device__ CellGeo(const GeneralGeo<T>& geo, const Plan& pl, const Place& q, const Offsets<W>& o) : g(geo) {
+    __device__ CellGeo(const GeneralGeo<T>& geo, const Plan& pl, const Place& q, const Offsets<W, O>& o) : g(geo) {
         SX = int64_t(pl.Y) * pl.Z;
         zb = int64_t(q.x) * pl.Y * (pl.Z + 1);
         yb = int64_t(q.x) * (pl.Y + 1) * pl.Z;
@@ -147,8 +146,8 @@ __device__ inline void lin_faces(const Star7<T, W>& s, const Plan& pl, const Pla
 }
 
 // Laplacian over the selected axes, from 0 in the order x, y, z
-template <class T, int W, int GEO>
-__device__ inline void lapl_of(const CellGeo<T, W, GEO>& c, const Star7<T, W>& s, int mask, T (&res)[W]) {
+template <class T, int W, int GEO, class O>
+__device__ inline void lapl_of(const CellGeo<T, W, GEO, O>& c, const Star7<T, W>& s, int mask, T (&res)[W]) {
     T fv[6][W], n[6][W], r[W];
     c.alphas(fv);
 #pragma unroll
@@ -172,14 +171,14 @@ __device__ inline void lapl_of(const CellGeo<T, W, GEO>& c, const Star7<T, W>& s
 #define CFD_STAR_HEAD                                 \
     Place q;                                          \
     if (!star::place<W>(pl, q)) return;               \
-    const Offsets<W> o = star::offsets<W>(pl, q);
+    const Offsets<W, O> o = star::offsets<W, O>(pl, q);
 
-template <class T, int W, int GEO>
+template <class T, int W, int GEO, class O>
 __global__ void __launch_bounds__(256) fgrad_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ phi,
                                                T* __restrict__ out, int mask, int wall_axis, Plan pl) {
     CFD_STAR_HEAD
     const Star7<T, W> s = star::load7<T, W>(phi, o);
-    const CellGeo<T, W, GEO> c(g, pl, q, o);
+    const CellGeo<T, W, GEO, O> c(g, pl, q, o);
     T fv[6][W], n[6][W], r[W], res[W];
     lin_faces(s, pl, q, wall_axis, fv);
 #pragma unroll
@@ -195,25 +194,25 @@ __global__ void __launch_bounds__(256) fgrad_k(typename FaceArg<T, GEO>::type g,
     star::store<T, W>(out + o.x0, o.o0, res);
 }
 
-template <class T, int W, int GEO>
+template <class T, int W, int GEO, class O>
 __global__ void __launch_bounds__(256) flapl_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ phi,
                                                T* __restrict__ out, int mask, Plan pl) {
     CFD_STAR_HEAD
     const Star7<T, W> s = star::load7<T, W>(phi, o);
-    const CellGeo<T, W, GEO> c(g, pl, q, o);
+    const CellGeo<T, W, GEO, O> c(g, pl, q, o);
     T res[W];
     lapl_of(c, s, mask, res);
     star::store<T, W>(out + o.x0, o.o0, res);
 }
 
 // T' = dt * (alpha * lapl(T)) + T (DtVar::extract order, src/fvm3d.cpp:690-692)
-template <class T, int W, int GEO, bool AF>
+template <class T, int W, int GEO, class O, bool AF>
 __global__ void __launch_bounds__(256) fheat_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ Tin,
                                                T* __restrict__ Tout, T alpha, const T* __restrict__ alpha_f, T dt,
                                                Plan pl) {
     CFD_STAR_HEAD
     const Star7<T, W> s = star::load7<T, W>(Tin, o);
-    const CellGeo<T, W, GEO> c(g, pl, q, o);
+    const CellGeo<T, W, GEO, O> c(g, pl, q, o);
     T af[W], res[W];
     if constexpr (AF) star::load<T, W>(alpha_f + o.x0, o.o0, af);
     lapl_of(c, s, 7, res);
@@ -226,21 +225,22 @@ __global__ void __launch_bounds__(256) fheat_k(typename FaceArg<T, GEO>::type g,
 }
 
 // StabVar, first stage: the three gradient components
-template <class T, int W, int GEO>
+template <class T, int W, int GEO, class O>
 __global__ void __launch_bounds__(256) fgrad3_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ phi,
                                                 T* __restrict__ gx, T* __restrict__ gy, T* __restrict__ gz, Plan pl) {
     CFD_STAR_HEAD
     const Star7<T, W> s = star::load7<T, W>(phi, o);
-    const CellGeo<T, W, GEO> c(g, pl, q, o);
+    const CellGeo<T, W, GEO, O> c(g, pl, q, o);
     T* const out[3] = {gx, gy, gz};
-    T fv[6][W], n[6][W], r[W];
+    T fv[6][W], n[6][W], r[3][W];
     lin_faces(s, pl, q, -1, fv);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         c.normals(d, n);
-        c.template gauss<true>(fv, n, d, r);
-        star::store<T, W>(out[d] + o.x0, o.o0, r);
+        c.template gauss<true>(fv, n, d, r[d]);
     }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) star::store<T, W>(out[d] + o.x0, o.o0, r[d]);
 }
 
 // StabVar, second stage: per selected component d the upwind face value
@@ -248,7 +248,7 @@ __global__ void __launch_bounds__(256) fgrad3_k(typename FaceArg<T, GEO>::type g
 // (which it sees as its opposite local face; on a wall the neighbour is the
 // cell itself, at its own opposite face), 0.5 * jump, axis-normal Gauss sum.
 // len: six centre-to-face distances per cell, fc-major.
-template <class T, int W, int GEO>
+template <class T, int W, int GEO, class O>
 __global__ void __launch_bounds__(256) fstab_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ len,
                                                const T* __restrict__ phi, const T* __restrict__ gx,
                                                const T* __restrict__ gy, const T* __restrict__ gz,
@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(256) fstab_k(typename FaceArg<T, GEO>::type g,
     CFD_STAR_HEAD
     const int64_t N = int64_t(pl.X) * pl.Y * pl.Z;
     const Star7<T, W> s = star::load7<T, W>(phi, o);
-    const CellGeo<T, W, GEO> c(g, pl, q, o);
+    const CellGeo<T, W, GEO, O> c(g, pl, q, o);
     const T* const gd[3] = {gx, gy, gz};
     // own lengths, and the neighbours' at their opposite local faces (the
     // clamped neighbour of a wall cell is the cell itself, as its rule asks)
@@ -307,14 +307,14 @@ __global__ void __launch_bounds__(256) fstab_k(typename FaceArg<T, GEO>::type g,
 // one pass would recompute the neighbours' velocities from p, and these turn
 // NaN wherever any face value of that cell is not finite, which the
 // recomputation could not see without loading all its faces.
-template <class T, int W, int GEO>
+template <class T, int W, int GEO, class O>
 __global__ void __launch_bounds__(256) fwave_vel_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ p,
                                                    const T* __restrict__ u, const T* __restrict__ v,
                                                    const T* __restrict__ w, T* __restrict__ uo, T* __restrict__ vo,
                                                    T* __restrict__ wo, T dt, Plan pl) {
     CFD_STAR_HEAD
     const Star7<T, W> s = star::load7<T, W>(p, o);
-    const CellGeo<T, W, GEO> c(g, pl, q, o);
+    const CellGeo<T, W, GEO, O> c(g, pl, q, o);
     const T* const in[3] = {u, v, w};
     T* const out[3] = {uo, vo, wo};
     T fv[6][W], n[6][W], r[W], vel[3][W];
@@ -327,17 +327,19 @@ __global__ void __launch_bounds__(256) fwave_vel_k(typename FaceArg<T, GEO>::typ
         c.template gauss<true>(fv, n, d, r);
 #pragma unroll
         for (int i = 0; i < W; ++i) vel[d][i] = dt * (-r[i]) + vel[d][i];
-        star::store<T, W>(out[d] + o.x0, o.o0, vel[d]);
     }
+    // (after all loads: a store between them would keep the later ones back)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) star::store<T, W>(out[d] + o.x0, o.o0, vel[d]);
 }
 
-template <class T, int W, int GEO, bool KF>
+template <class T, int W, int GEO, class O, bool KF>
 __global__ void __launch_bounds__(256) fwave_p_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ u,
                                                  const T* __restrict__ v, const T* __restrict__ w,
                                                  const T* __restrict__ p, T* __restrict__ po, T K,
                                                  const T* __restrict__ Kf, T dt, Plan pl) {
     CFD_STAR_HEAD
-    const CellGeo<T, W, GEO> c(g, pl, q, o);
+    const CellGeo<T, W, GEO, O> c(g, pl, q, o);
     const T* const in[3] = {u, v, w};
     T pc[W], kf[W], S[W];
     star::load<T, W>(p + o.x0, o.o0, pc);
@@ -371,24 +373,36 @@ template <class T> const GeneralGeo<T>& gg(const cfd_mesh_s* m) {
     if constexpr (sizeof(T) == 4) return m->gg32; else return m->gg64;
 }
 
-// f(plan, grid, block, width, geometry kind, geometry), width and kind as
-// integral constants
+// f(plan, grid, block, width, geometry kind, offset, geometry): width and kind
+// as integral constants, the offset a value of its type
 template <class T, class F> void with_faces(const cfd_mesh_s* m, F f) {
-    auto with_width = [&](auto w) {
+    auto with_width = [&](auto w, auto off) {
         const Plan pl = star::make_plan(m->X, m->Y, m->Z, w());
         const dim3 grid = star::plan_grid(pl), block = star::plan_block(pl);
-        if (m->lattice) f(pl, grid, block, w, std::integral_constant<int, 2>{}, lg<T>(m));
-        else f(pl, grid, block, w, std::integral_constant<int, 3>{}, gg<T>(m));
+        if (m->lattice) f(pl, grid, block, w, std::integral_constant<int, 2>{}, off, lg<T>(m));
+        else f(pl, grid, block, w, std::integral_constant<int, 3>{}, off, gg<T>(m));
     };
     // One cell per thread on small meshes, by the uniform meshes' line (us per
     // acoustic step with vectors / one cell: perturbed FP32 16^3 6.9 / 5.0, 64^3
     // 10.6 / 8.8, lattice FP32 48^3 6.1 / 5.2, 80^3 9.7 / 9.0, 100^3 13.0 / 14.5;
     // lattice FP64 32^3 5.4 / 4.8, 48^3 6.5 / 6.6, 64^3 7.7 / 9.5).
-    // (A plane's y- and z-faces are one row or column more than its cells, and
-    // their offsets are 32-bit in the vector form too.)
-    if (m->Z >= star::kWidth<T> && star::vector_form<T>(m->Y + 1, m->Z + 1) && !star::narrow<T>(m->N))
-        with_width(std::integral_constant<int, star::kWidth<T>>{});
-    else with_width(std::integral_constant<int, 1>{});
+    // Its offsets: 32 bits in FP32 (us per acoustic step of perturbed meshes with
+    // 64 / 32: 48^3 6.30 / 5.87, 64^3 8.39 / 8.08), 64 in FP64, where 32 cost (48^3
+    // 9.08 / 9.57, 128^3 130 / 140) and 64 save registers.
+    // (A plane's y- and z-faces are one row or column more than its cells.)
+    const bool small = star::small_plane<T>(m->Y + 1, m->Z + 1);
+    if (m->Z >= star::kWidth<T> && small && !star::narrow<T>(m->N)) {
+        with_width(std::integral_constant<int, star::kWidth<T>>{}, uint32_t(0));
+    } else {
+        bool done = false;
+        if constexpr (sizeof(T) == 4) {
+            if (small) {
+                with_width(std::integral_constant<int, 1>{}, uint32_t(0));
+                done = true;
+            }
+        }
+        if (!done) with_width(std::integral_constant<int, 1>{}, uint64_t(0));
+    }
     CFD_HIP(hipGetLastError());
 }
 
@@ -396,15 +410,15 @@ template <class T, class F> void with_faces(const cfd_mesh_s* m, F f) {
 
 template <class T>
 void launch_grad_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, const auto& g) {
-        fgrad_k<T, decltype(w)::value, decltype(geo)::value>
+    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
+        fgrad_k<T, decltype(w)::value, decltype(geo)::value, decltype(off)>
             <<<gr, bl, 0, s>>>(g, (const T*)phi, (T*)out, mask, wall, pl);
     });
 }
 
 template <class T> void launch_lapl_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, const auto& g) {
-        flapl_k<T, decltype(w)::value, decltype(geo)::value><<<gr, bl, 0, s>>>(g, (const T*)phi, (T*)out, mask, pl);
+    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
+        flapl_k<T, decltype(w)::value, decltype(geo)::value, decltype(off)><<<gr, bl, 0, s>>>(g, (const T*)phi, (T*)out, mask, pl);
     });
 }
 
@@ -413,20 +427,22 @@ void launch_stab_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask
     T* gx = (T*)scratch3;
     T* gy = gx + m->N;
     T* gz = gy + m->N;
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, const auto& g) {
+    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
         constexpr int W = decltype(w)::value, GEO = decltype(geo)::value;
-        fgrad3_k<T, W, GEO><<<gr, bl, 0, s>>>(g, (const T*)phi, gx, gy, gz, pl);
+        using O = decltype(off);
+        fgrad3_k<T, W, GEO, O><<<gr, bl, 0, s>>>(g, (const T*)phi, gx, gy, gz, pl);
         CFD_HIP(hipGetLastError());
-        fstab_k<T, W, GEO><<<gr, bl, 0, s>>>(g, gg<T>(m).len, (const T*)phi, gx, gy, gz, (T*)out, mask, pl);
+        fstab_k<T, W, GEO, O><<<gr, bl, 0, s>>>(g, gg<T>(m).len, (const T*)phi, gx, gy, gz, (T*)out, mask, pl);
     });
 }
 
 template <class T>
 void launch_heat_faces(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
                        hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, const auto& g) {
+    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
         constexpr int W = decltype(w)::value, GEO = decltype(geo)::value;
-        auto* kern = af ? fheat_k<T, W, GEO, true> : fheat_k<T, W, GEO, false>;
+        using O = decltype(off);
+        auto* kern = af ? fheat_k<T, W, GEO, O, true> : fheat_k<T, W, GEO, O, false>;
         kern<<<gr, bl, 0, s>>>(g, (const T*)in, (T*)out, T(alpha), (const T*)af, T(dt), pl);
     });
 }
@@ -434,12 +450,13 @@ void launch_heat_faces(const cfd_mesh_s* m, const void* in, void* out, double al
 template <class T>
 void launch_wave_faces(const cfd_mesh_s* m, void* const* in, void* const* out, double K, const void* Kf, double dt,
                        hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, const auto& g) {
+    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
         constexpr int W = decltype(w)::value, GEO = decltype(geo)::value;
-        fwave_vel_k<T, W, GEO><<<gr, bl, 0, s>>>(g, (const T*)in[0], (const T*)in[1], (const T*)in[2],
+        using O = decltype(off);
+        fwave_vel_k<T, W, GEO, O><<<gr, bl, 0, s>>>(g, (const T*)in[0], (const T*)in[1], (const T*)in[2],
                                                  (const T*)in[3], (T*)out[1], (T*)out[2], (T*)out[3], T(dt), pl);
         CFD_HIP(hipGetLastError());
-        auto* kern = Kf ? fwave_p_k<T, W, GEO, true> : fwave_p_k<T, W, GEO, false>;
+        auto* kern = Kf ? fwave_p_k<T, W, GEO, O, true> : fwave_p_k<T, W, GEO, O, false>;
         kern<<<gr, bl, 0, s>>>(g, (const T*)out[1], (const T*)out[2], (const T*)out[3], (const T*)in[0], (T*)out[0],
                                T(K), (const T*)Kf, T(dt), pl);
     });

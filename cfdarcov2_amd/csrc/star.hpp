@@ -28,7 +28,8 @@ template <class T, int W> struct VecOf {
 
 // Offsets within a plane.  The vector form keeps them in 32 bits (planes below
 // 4 GiB), so an address is a base uniform over the workgroup plus one
-// register; rows shorter than a vector and larger planes take W = 1 with 64.
+// register; rows shorter than a vector and larger planes take W = 1 with 64
+// (or with 32, where a kernel's launch chooses the type O of its offsets).
 template <int W> struct OffOf { using type = uint32_t; };
 template <> struct OffOf<1> { using type = uint64_t; };
 template <int W> using Off = typename OffOf<W>::type;
@@ -37,18 +38,18 @@ template <class T, class O> __device__ inline T load1(const T* base, O off) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + O(off * O(sizeof(T))));
 }
 // W values at an element offset from a uniform pointer
-template <class T, int W> __device__ inline void load(const T* base, Off<W> off, T (&v)[W]) {
+template <class T, int W, class O> __device__ inline void load(const T* base, O off, T (&v)[W]) {
     if constexpr (W == 1) {
         v[0] = load1(base, off);
     } else {
         using V = typename VecOf<T, W>::type;
-        const V r = *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + Off<W>(off * Off<W>(sizeof(T))));
+        const V r = *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + O(off * O(sizeof(T))));
 #pragma unroll
         for (int i = 0; i < W; ++i) v[i] = r[i];
     }
 }
-template <class T, int W> __device__ inline void store(T* base, Off<W> off, const T (&v)[W]) {
-    char* const a = reinterpret_cast<char*>(base) + Off<W>(off * Off<W>(sizeof(T)));
+template <class T, int W, class O> __device__ inline void store(T* base, O off, const T (&v)[W]) {
+    char* const a = reinterpret_cast<char*>(base) + O(off * O(sizeof(T)));
     if constexpr (W == 1) {
         *reinterpret_cast<T*>(a) = v[0];
     } else {
@@ -94,9 +95,10 @@ inline dim3 plan_block(const Plan& p) { return dim3(unsigned(p.bx), unsigned(p.b
 
 // Whether rows and planes suit the vector form of T
 template <class T> constexpr int kWidth = 16 / int(sizeof(T));
-template <class T> inline bool vector_form(int64_t Y, int64_t Z) {
-    return Z >= kWidth<T> && Y * Z * int64_t(sizeof(T)) < (int64_t(1) << 32);
+template <class T> inline bool small_plane(int64_t Y, int64_t Z) {  // 32-bit offsets reach all of it
+    return Y * Z * int64_t(sizeof(T)) < (int64_t(1) << 32);
 }
+template <class T> inline bool vector_form(int64_t Y, int64_t Z) { return Z >= kWidth<T> && small_plane<T>(Y, Z); }
 
 // Whether a step of a mesh of this size is better with one cell per thread: a
 // launch then lasts about as long as one wavefront's chain of operations, and
@@ -134,14 +136,13 @@ template <int W> __device__ inline bool place(const Plan& p, Place& q) {
 
 // Element offsets of a thread's cells and of their six neighbours, clamped to
 // the mesh: a neighbour beyond a wall is the cell itself (the reference rule).
-template <int W> struct Offsets {
-    int64_t x0, xm1, xp1;           // planes
-    Off<W> o0, ym1, yp1, zm1, zp1;  // within a plane: the W cells, rows y-1 and y+1, cells z0-1 and z0+W
+template <int W, class O = Off<W>> struct Offsets {
+    int64_t x0, xm1, xp1;      // planes
+    O o0, ym1, yp1, zm1, zp1;  // within a plane: the W cells, rows y-1 and y+1, cells z0-1 and z0+W
 };
-template <int W> __device__ inline Offsets<W> offsets(const Plan& p, const Place& q) {
-    using O = Off<W>;
+template <int W, class O = Off<W>> __device__ inline Offsets<W, O> offsets(const Plan& p, const Place& q) {
     const int x = q.x, y = q.y, z0 = q.z0;
-    Offsets<W> o;
+    Offsets<W, O> o;
     const int64_t SX = int64_t(p.Y) * p.Z;
     o.x0 = int64_t(x) * SX;
     o.xm1 = x >= 1 ? o.x0 - SX : o.x0;
@@ -162,7 +163,8 @@ template <class T, int W> struct Star7 {
     T xm[W], xp[W], ym[W], yp[W], r[W + 2];
     __device__ T c(int i) const { return r[i + 1]; }
 };
-template <class T, int W> __device__ inline Star7<T, W> load7(const T* __restrict__ f, const Offsets<W>& o) {
+template <class T, int W, class O>
+__device__ inline Star7<T, W> load7(const T* __restrict__ f, const Offsets<W, O>& o) {
     Star7<T, W> s;
     T c[W];
     const T* const f0 = f + o.x0;
@@ -210,21 +212,21 @@ template <class T, int W> struct LatticeCells {
     T ax[2], ay[2], az[W + 1];  // alpha_d of the lower and upper faces (az: of the W + 1 z-faces)
     __device__ T area(int a, int i) const { return a == 0 ? wy * wz[i] : a == 1 ? wx * wz[i] : wx * wy; }
 };
-template <class T, int W, bool ALPHA>
-__device__ inline LatticeCells<T, W> load_lattice(const LatticeGeo<T>& g, const Offsets<W>& o, const Place& q) {
+template <class T, int W, bool ALPHA, class O>
+__device__ inline LatticeCells<T, W> load_lattice(const LatticeGeo<T>& g, const Offsets<W, O>& o, const Place& q) {
     const int x = q.x, y = q.y, z0 = q.z0;
     LatticeCells<T, W> c;
     load<T, W>(g.vol + o.x0, o.o0, c.V);
     c.wx = g.w[0][x];
     c.wy = g.w[1][y];
-    load<T, W>(g.w[2], Off<W>(z0), c.wz);
+    load<T, W>(g.w[2], O(z0), c.wz);
     if constexpr (ALPHA) {
         T lo[W];
         c.ax[0] = g.alpha[0][x];
         c.ax[1] = g.alpha[0][x + 1];
         c.ay[0] = g.alpha[1][y];
         c.ay[1] = g.alpha[1][y + 1];
-        load<T, W>(g.alpha[2], Off<W>(z0), lo);
+        load<T, W>(g.alpha[2], O(z0), lo);
 #pragma unroll
         for (int i = 0; i < W; ++i) c.az[i] = lo[i];
         c.az[W] = g.alpha[2][z0 + W];
