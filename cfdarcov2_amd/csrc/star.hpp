@@ -15,6 +15,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "march.hpp"
 
@@ -61,17 +63,41 @@ template <class T, int W, class O> __device__ inline void store(T* base, O off, 
     }
 }
 
+// Division of 0 <= k < 2^31 by a constant n >= 1: the product with the
+// reciprocal rounded up to 32 significant bits, exact for these k (the
+// hardware has no integer division, and a workgroup's first loads wait for it).
+struct Div {
+    uint32_t m, s;  // k / n = (k m) >> (32 + s); m = 0 for n = 1
+    __device__ int operator()(int k) const { return m ? int(__umulhi(uint32_t(k), m) >> s) : k; }
+};
+inline Div make_div(int64_t n) {
+    Div d{};
+    if (n == 1) return d;
+    while ((int64_t(2) << d.s) < n) ++d.s;
+    d.m = uint32_t(((uint64_t(1) << (32 + d.s)) + uint64_t(n) - 1) / uint64_t(n));
+    return d;
+}
+
 // Launch geometry: workgroups of bx units x by rows of one x-plane, nzb x nyb
 // of them per plane, X planes; the grid is padded to a multiple of 8 and each
-// XCD (round-robin dispatch) takes a contiguous run, so the planes that a
-// stencil shares are in its own L2.
+// XCD (round-robin dispatch) takes a contiguous run, so what neighbouring
+// workgroups share is in its own L2.
 struct Plan {
     int X, Y, Z;
     int bx, by, nzb, nyb;
     int blocks;  // workgroups with work, before the padding
+    int cut;     // the axis whose blocks the runs divide (outermost in the run)
+    Div d0, d1;  // by the number of innermost blocks, and of the next
 };
 
-inline Plan make_plan(int64_t X, int64_t Y, int64_t Z, int W, int threads = 0) {
+// The runs divide x.  Slabs of a few planes share most of what they read with
+// the next XCD's, so where y is at least four times as long the runs divide y
+// (us, cut in x / y: acoustic step FP64 64x256x256 61.3 / 43.0, 40x1000x40
+// 22.1 / 19.4, FP32 20x300x300 15.3 / 13.1; perturbed heat step FP64 40x1000x40
+// 45.6 / 35.0; at twice as long neither is better: 64x128x128 FP64 14.2 / 13.9,
+// perturbed 57.4 / 58.0).  z only on demand (long_z: its columns make a row's
+// halo, so only face arrays that leave the cache repay it).
+inline Plan make_plan(int64_t X, int64_t Y, int64_t Z, int W, int threads = 0, bool long_z = false) {
     Plan p{};
     p.X = int(X); p.Y = int(Y); p.Z = int(Z);
     const int units = int((Z + W - 1) / W);
@@ -79,15 +105,31 @@ inline Plan make_plan(int64_t X, int64_t Y, int64_t Z, int W, int threads = 0) {
         const int64_t all = X * Y * units;
         threads = all >= 256 * 256 ? 256 : all >= 128 * 256 ? 128 : 64;
     }
-    p.nzb = (units + threads - 1) / threads;
-    p.bx = (units + p.nzb - 1) / p.nzb;
-    p.by = threads / p.bx;
-    if (p.by < 1) p.by = 1;
-    if (p.by > Y) p.by = int(Y);
+    auto split = [&](int nzb) {
+        p.nzb = nzb;
+        p.bx = (units + nzb - 1) / nzb;
+        p.by = int(std::min<int64_t>(threads / p.bx, Y));
+        if (p.by < 1) p.by = 1;
+    };
+    const int columns = (units + threads - 1) / threads;
+    split(columns);
+    // A row just over half a workgroup would leave the rest of it idle: three
+    // times the columns then (FP64 z = 300, 150 units: stabilisation of 300^3 201
+    // us as 150 threads, 185 as 5 rows of 50; 160^3 one cell per thread, lattice
+    // heat step FP64 31.0 / 26.5).
+    if (threads == 256 && p.by == 1 && Y >= 4 && 3 * p.bx < 2 * threads) split(3 * columns);
+    if (long_z && units >= 64) {
+        split(std::max(8, (units + 63) / 64));
+        p.cut = 2;
+    } else {
+        p.cut = Y >= 4 * X ? 1 : 0;
+    }
     p.nyb = int((Y + p.by - 1) / p.by);
     const int64_t n = int64_t(p.nzb) * p.nyb * X;
     CFD_REQUIRE(n < (int64_t(1) << 31) - 8, "star grid too large");
     p.blocks = int(n);
+    p.d0 = make_div(p.cut == 2 ? p.nyb : p.nzb);
+    p.d1 = make_div(p.cut == 0 ? p.nyb : p.X);
     return p;
 }
 inline dim3 plan_grid(const Plan& p) { return dim3(unsigned((p.blocks + 7) / 8 * 8)); }
@@ -120,10 +162,13 @@ struct Place {
 template <int W> __device__ inline bool place_at(const Plan& p, int b, int padded, int tx, int ty, Place& q) {
     const int lin = (b % 8) * (padded / 8) + b / 8;
     if (lin >= p.blocks) return false;
-    const int row = p.nzb == 1 ? lin : lin / p.nzb;
-    const int zb = p.nzb == 1 ? 0 : lin - row * p.nzb;
-    q.x = row / p.nyb;
-    q.y = (row - q.x * p.nyb) * p.by + ty;
+    // blocks of the run's cut axis outermost: (x, y, z), (y, x, z) or (z, x, y)
+    const int n0 = p.cut == 2 ? p.nyb : p.nzb, n1 = p.cut == 0 ? p.nyb : p.X;
+    const int row = p.d0(lin), in = lin - row * n0;
+    const int out = p.d1(row), mid = row - out * n1;
+    const int zb = p.cut == 2 ? out : in;
+    q.x = p.cut == 0 ? out : mid;
+    q.y = (p.cut == 0 ? mid : p.cut == 1 ? out : in) * p.by + ty;
     const int zi = zb * p.bx + tx;
     if (ty >= p.by || q.y >= p.Y || zi * W >= p.Z) return false;
     q.z0 = min(zi * W, p.Z - W);

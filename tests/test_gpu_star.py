@@ -227,6 +227,48 @@ def test_perturbed_mesh_is_no_lattice(hip_ctx):
     assert gm.info().device_bytes == gg.info().device_bytes
 
 
+# launch geometries: runs that divide y, three columns where a row is just over
+# half a workgroup (in cells and in vectors), and the rows' ends of both
+PLANS = [(22, 20, 300), (22, 20, 150), (9, 40, 130), (6, 24, 67), (2, 512, 140), (3, 13, 1030)]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["dyadic", "decimal", "skewed"])
+@pytest.mark.parametrize("n", PLANS, ids=lambda n: "x".join(map(str, n)))
+def test_launch_geometries(hip_ctx, oracle_lib, n, kind, dtype):
+    _check_against_oracle(*_mesh(hip_ctx, oracle_lib, n, kind, dtype), dtype)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float64, (20, 21, 2400)), (np.float32, (24, 23, 3602))], ids=["f64", "f32"])
+def test_launch_geometry_of_long_perturbed_meshes(hip_ctx, oracle_lib, n, dtype):
+    """Runs of columns: face arrays beyond half the last-level cache, z at
+    least eight times as long as x and y."""
+    assert 34 * np.prod(n) * np.dtype(dtype).itemsize > 256 << 20
+    _check_against_oracle(*_mesh(hip_ctx, oracle_lib, n, "skewed", dtype), dtype)
+
+
+def _check_against_oracle(gm, gg, om, dtype):
+    """Every operator and step of the mesh against the oracle's."""
+    gg.close()
+    rng = np.random.default_rng(12)
+    f = [rng.standard_normal(om.N).astype(dtype) for _ in range(4)]
+    phi, (t, out) = f[0], (_view(f[0], dtype, 1), _view(f[0], dtype, 1))
+    for mask in (7, 1, 2, 4, 5):
+        assert np.array_equal(gm.grad(t, mask, mask % 3, out=out).cpu().numpy(), om.grad(phi, mask, mask % 3)), mask
+        assert np.array_equal(gm.lapl(t, mask, out=out).cpu().numpy(), om.lapl(phi, mask)), mask
+    assert np.array_equal(gm.stab(t, 7, out=out).cpu().numpy(), om.stab(phi, 7))
+    A, B = [[_view(a, dtype, 0) for a in f] for _ in range(2)]
+    for steps in (1, 4):
+        A[0].copy_(_view(phi, dtype, 0))
+        assert np.array_equal(gm.heat_run(A[0], B[0], 2e-3, 0.5, steps).cpu().numpy(), om.heat_run(phi, 2e-3, 0.5, steps))
+    A[0].copy_(_view(phi, dtype, 0))
+    if gm.info().uniform:
+        gm.set_wave_shape(0, 4, 8, 0)
+    for g, r in zip(gm.wave_run(A, B, -1.0, 0.02, 2), om.wave_run(*f, -1.0, 0.02, 2)):
+        assert np.array_equal(g.cpu().numpy(), r)
+    gm.close()
+
+
 def test_lattice_without_room_for_its_tables(hip_ctx):
     """A pool limit that holds the face arrays and no more: the mesh is made
     without the tables, as before they existed, and gives the same results."""
