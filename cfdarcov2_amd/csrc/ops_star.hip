@@ -48,13 +48,18 @@ __device__ inline star::Faces<T> lin_faces(const star::Star7<T, W>& s, const AtW
 
 }  // namespace
 
-template <class T, int W, bool PW>
+// SOME: an operator over some axes loads only their neighbours.  On fields that
+// stay in the last-level cache the other loads cost nothing (they bring lines
+// that other workgroups read: one-axis gradient 256^3 FP64 39.3 us with all, 48
+// with the axis' own), beyond it they cross memory (one-axis gradient FP64
+// 512x256x256 128 / 100, 300^3 118 / 94).
+template <class T, int W, bool PW, bool SOME>
 __global__ void __launch_bounds__(256) grad_star_k(UniformGeo<T> g, const T* __restrict__ phi,
                                                    T* __restrict__ out, int mask, int wall_axis, star::Plan pl) {
     star::Place q;
     if (!star::place<W>(pl, q)) return;
     const star::Offsets<W> o = star::offsets<W>(pl, q);
-    const star::Star7<T, W> s = star::load7<T, W>(phi, o);
+    const star::Star7<T, W> s = SOME ? star::load_axes<T, W>(phi, o, mask) : star::load7<T, W>(phi, o);
     const VolDiv<T, PW> Vd{g.vol, g.inv_vol};
     T r[W];
 #pragma unroll
@@ -69,13 +74,13 @@ __global__ void __launch_bounds__(256) grad_star_k(UniformGeo<T> g, const T* __r
     star::store<T, W>(out + o.x0, o.o0, r);
 }
 
-template <class T, int W, bool PW>
+template <class T, int W, bool PW, bool SOME>
 __global__ void __launch_bounds__(256) lapl_star_k(UniformGeo<T> g, const T* __restrict__ phi,
                                                    T* __restrict__ out, int mask, star::Plan pl) {
     star::Place q;
     if (!star::place<W>(pl, q)) return;
     const star::Offsets<W> o = star::offsets<W>(pl, q);
-    const star::Star7<T, W> s = star::load7<T, W>(phi, o);
+    const star::Star7<T, W> s = SOME ? star::load_axes<T, W>(phi, o, mask) : star::load7<T, W>(phi, o);
     T r[W];
 #pragma unroll
     for (int i = 0; i < W; ++i) r[i] = star::lapl_uniform<T, W, PW>(g, s, mask, i);
@@ -289,20 +294,29 @@ template <class T, class F> void with_star(const cfd_mesh_s* m, F f, bool narrow
     CFD_HIP(hipGetLastError());
 }
 
+// whether an operator over `mask` loads the neighbours of its axes only (see grad_star_k)
+template <class T> bool some_axes(const cfd_mesh_s* m, int mask) {
+    return mask != 7 && 2 * m->N * int64_t(sizeof(T)) > kLastLevelCacheBytes;
+}
+
 }  // namespace
 
 template <class T>
 void launch_grad_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s) {
     with_star<T>(m, [&](const star::Plan& pl, auto w, auto pw, const auto& g) {
-        grad_star_k<T, decltype(w)::value, decltype(pw)::value>
-            <<<star::plan_grid(pl), star::plan_block(pl), 0, s>>>(g, (const T*)phi, (T*)out, mask, wall, pl);
+        constexpr int W = decltype(w)::value;
+        constexpr bool PW = decltype(pw)::value;
+        auto* kern = some_axes<T>(m, mask) ? grad_star_k<T, W, PW, true> : grad_star_k<T, W, PW, false>;
+        kern<<<star::plan_grid(pl), star::plan_block(pl), 0, s>>>(g, (const T*)phi, (T*)out, mask, wall, pl);
     });
 }
 
 template <class T> void launch_lapl_star(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s) {
     with_star<T>(m, [&](const star::Plan& pl, auto w, auto pw, const auto& g) {
-        lapl_star_k<T, decltype(w)::value, decltype(pw)::value>
-            <<<star::plan_grid(pl), star::plan_block(pl), 0, s>>>(g, (const T*)phi, (T*)out, mask, pl);
+        constexpr int W = decltype(w)::value;
+        constexpr bool PW = decltype(pw)::value;
+        auto* kern = some_axes<T>(m, mask) ? lapl_star_k<T, W, PW, true> : lapl_star_k<T, W, PW, false>;
+        kern<<<star::plan_grid(pl), star::plan_block(pl), 0, s>>>(g, (const T*)phi, (T*)out, mask, pl);
     });
 }
 

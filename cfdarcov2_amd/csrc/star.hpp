@@ -225,6 +225,40 @@ __device__ inline Star7<T, W> load7(const T* __restrict__ f, const Offsets<W, O>
     return s;
 }
 
+// The same for an operator over the axes of `mask`: the others' neighbours are
+// not loaded and read as the cell itself.
+template <class T, int W, class O>
+__device__ inline Star7<T, W> load_axes(const T* __restrict__ f, const Offsets<W, O>& o, int mask) {
+    Star7<T, W> s;
+    T c[W];
+    const T* const f0 = f + o.x0;
+    const bool x = mask & 1, y = mask & 2, z = mask & 4;
+    load<T, W>(f0, o.o0, c);
+    if (x) {
+        load<T, W>(f + o.xm1, o.o0, s.xm);
+        load<T, W>(f + o.xp1, o.o0, s.xp);
+    }
+    if (y) {
+        load<T, W>(f0, o.ym1, s.ym);
+        load<T, W>(f0, o.yp1, s.yp);
+    }
+    if (z) {
+        s.r[0] = load1(f0, o.zm1);
+        s.r[W + 1] = load1(f0, o.zp1);
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        s.r[i + 1] = c[i];
+        if (!x) s.xm[i] = s.xp[i] = c[i];
+        if (!y) s.ym[i] = s.yp[i] = c[i];
+    }
+    if (!z) {
+        s.r[0] = c[0];
+        s.r[W + 1] = c[W - 1];
+    }
+    return s;
+}
+
 // Value across the lower or upper face of cell i along axis a
 template <class T, int W> __device__ inline T face_nb(const Star7<T, W>& s, int a, bool upper, int i) {
     if (a == 0) return upper ? s.xp[i] : s.xm[i];

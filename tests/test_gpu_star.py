@@ -239,6 +239,33 @@ def test_launch_geometries(hip_ctx, oracle_lib, n, kind, dtype):
     _check_against_oracle(*_mesh(hip_ctx, oracle_lib, n, kind, dtype), dtype)
 
 
+@pytest.mark.parametrize("dtype,n", [(np.float64, (258, 257, 254)), (np.float32, (323, 322, 323))], ids=["f64", "f32"])
+def test_some_axes_beyond_the_cache(hip_ctx, n, dtype):
+    """Gradient and Laplacian over some axes on fields beyond the last-level
+    cache, which load those axes' neighbours only, against their definition."""
+    from cfdarcov2_amd import capi
+    h = (0.125, 0.25, 0.5)
+    assert 2 * np.prod(n) * np.dtype(dtype).itemsize > 256 << 20
+    gm = capi.HexMesh(hip_ctx, *n, *h, dtype=dtype)
+    phi = torch.from_numpy(np.random.default_rng(3).standard_normal(n).astype(dtype)).cuda()
+    out = torch.empty(gm.N, dtype=phi.dtype, device="cuda")
+    V = h[0] * h[1] * h[2]
+    for mask in (0, 1, 2, 4, 3, 5, 6):
+        grad, lapl = torch.zeros_like(phi), torch.zeros_like(phi)
+        for a in range(3):
+            if not mask & (1 << a):
+                continue
+            k, A = n[a], V / h[a]
+            lo = torch.cat([phi.narrow(a, 0, 1), phi.narrow(a, 0, k - 1)], a)
+            hi = torch.cat([phi.narrow(a, 1, k - 1), phi.narrow(a, k - 1, 1)], a)
+            grad += (-((phi + lo) * 0.5) * A + (phi + hi) * 0.5 * A) / V
+            lapl += ((-phi + lo) / h[a] * A + (-phi + hi) / h[a] * A) / V
+            del lo, hi
+        assert torch.equal(gm.grad(phi.reshape(-1), mask, -1, out=out), grad.reshape(-1)), mask
+        assert torch.equal(gm.lapl(phi.reshape(-1), mask, out=out), lapl.reshape(-1)), mask
+    gm.close()
+
+
 @pytest.mark.parametrize("dtype,n", [(np.float64, (20, 21, 2400)), (np.float32, (24, 23, 3602))], ids=["f64", "f32"])
 def test_launch_geometry_of_long_perturbed_meshes(hip_ctx, oracle_lib, n, dtype):
     """Runs of columns: face arrays beyond half the last-level cache, z at
