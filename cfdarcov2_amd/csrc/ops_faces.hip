@@ -224,6 +224,12 @@ __global__ void __launch_bounds__(256) fheat_k(typename FaceArg<T, GEO>::type g,
     star::store<T, W>(Tout + o.x0, o.o0, res);
 }
 
+// Kernels of three outputs store them after all loads where the registers
+// allow it, since a store keeps back the loads after it (acoustic step of
+// perturbed 64^3 FP32, one cell per thread 8.8 / 8.4 us; with vectors it costs:
+// lattice 200^3 FP64 199 / 206).
+template <class T, int W> constexpr bool kLateStores = sizeof(T) == 4 && W == 1;
+
 // StabVar, first stage: the three gradient components
 template <class T, int W, int GEO, class O>
 __global__ void __launch_bounds__(256) fgrad3_k(typename FaceArg<T, GEO>::type g, const T* __restrict__ phi,
@@ -238,9 +244,11 @@ __global__ void __launch_bounds__(256) fgrad3_k(typename FaceArg<T, GEO>::type g
     for (int d = 0; d < 3; ++d) {
         c.normals(d, n);
         c.template gauss<true>(fv, n, d, r[d]);
+        if constexpr (!kLateStores<T, W>) star::store<T, W>(out[d] + o.x0, o.o0, r[d]);
     }
+    if constexpr (kLateStores<T, W>)
 #pragma unroll
-    for (int d = 0; d < 3; ++d) star::store<T, W>(out[d] + o.x0, o.o0, r[d]);
+        for (int d = 0; d < 3; ++d) star::store<T, W>(out[d] + o.x0, o.o0, r[d]);
 }
 
 // StabVar, second stage: per selected component d the upwind face value
@@ -327,10 +335,11 @@ __global__ void __launch_bounds__(256) fwave_vel_k(typename FaceArg<T, GEO>::typ
         c.template gauss<true>(fv, n, d, r);
 #pragma unroll
         for (int i = 0; i < W; ++i) vel[d][i] = dt * (-r[i]) + vel[d][i];
+        if constexpr (!kLateStores<T, W>) star::store<T, W>(out[d] + o.x0, o.o0, vel[d]);
     }
-    // (after all loads: a store between them would keep the later ones back)
+    if constexpr (kLateStores<T, W>)
 #pragma unroll
-    for (int d = 0; d < 3; ++d) star::store<T, W>(out[d] + o.x0, o.o0, vel[d]);
+        for (int d = 0; d < 3; ++d) star::store<T, W>(out[d] + o.x0, o.o0, vel[d]);
 }
 
 template <class T, int W, int GEO, class O, bool KF>
@@ -373,9 +382,41 @@ template <class T> const GeneralGeo<T>& gg(const cfd_mesh_s* m) {
     if constexpr (sizeof(T) == 4) return m->gg32; else return m->gg64;
 }
 
+enum class Op { grad, lapl, stab, heat, wave };
+
+// The largest mesh, in cells, on which an operator takes one cell per thread.
+// Small meshes because a launch then lasts about as long as one wavefront's
+// chain of operations, which is W times as long with vectors; in FP32 larger
+// perturbed ones too, because their kernels with vectors hold few wavefronts
+// (three to five per SIMD) while the face arrays stay in the last-level cache.
+// Time with vectors / with one cell per thread, in a captured graph:
+//               40^3  56^3  64^3  80^3  100^3 128^3 160^3
+//   lattice   grad  1.12  1.12  1.02  0.98  0.73  0.74  0.52
+//   FP32      lapl  1.13  1.15  1.06  1.10  0.86  0.90  0.58
+//             stab  1.18  1.17  1.08  1.14  0.95  1.05  0.83
+//             heat  1.11  1.16  1.03  1.06  0.85  0.89  0.66
+//             wave  1.22  1.22  1.11  1.15  0.96  1.07  0.89
+//   perturbed grad  1.29  1.20  1.13  1.07  0.99  1.09  1.09 (200^3 0.97)
+//   FP32      lapl  1.14  1.12  1.01  1.01  0.97  1.03  0.81
+//             stab  1.28  1.16  1.21  1.19  1.03  1.07  0.80
+//             heat  1.15  1.19  1.14  1.21  1.09  1.14  0.89
+//             wave  1.35  1.23  1.27  1.20  1.08  1.16  0.85
+//               16^3  24^3  32^3  36^3  40^3  48^3  56^3
+//   lattice   heat  1.02  0.98  0.98  0.94  0.95  0.97  0.86 (the others within 0.04 but
+//   FP64      wave  1.12  1.08  1.08  1.01  0.96  1.01  0.84  of 16^3 to 20^3, up to 1.07)
+//   perturbed heat  1.10  1.04  1.03  0.99  0.92  0.91  0.79 (grad 1.06 to 0.77, lapl
+//   FP64      wave  1.27  1.21  1.20  1.11  1.01  0.98  0.84  1.05 to 0.78, stab 1.13 to 0.80)
+template <class T> int64_t one_cell_limit(Op op, bool lattice) {
+    int bits;
+    if (sizeof(T) == 8) bits = op == Op::wave && !lattice ? 16 : 15;
+    else if (lattice) bits = op == Op::grad ? 18 : 19;
+    else bits = op == Op::grad ? 22 : 21;
+    return int64_t(1) << bits;
+}
+
 // f(plan, grid, block, width, geometry kind, offset, geometry): width and kind
 // as integral constants, the offset a value of its type
-template <class T, class F> void with_faces(const cfd_mesh_s* m, F f) {
+template <class T, class F> void with_faces(const cfd_mesh_s* m, Op op, F f) {
     auto with_width = [&](auto w, auto off) {
         // Face arrays beyond half the last-level cache on meshes long in z: runs
         // of columns (us, cut in x / z: heat step FP64 40x40x1000 44.8 / 39.4,
@@ -388,16 +429,12 @@ template <class T, class F> void with_faces(const cfd_mesh_s* m, F f) {
         if (m->lattice) f(pl, grid, block, w, std::integral_constant<int, 2>{}, off, lg<T>(m));
         else f(pl, grid, block, w, std::integral_constant<int, 3>{}, off, gg<T>(m));
     };
-    // One cell per thread on small meshes, by the uniform meshes' line (us per
-    // acoustic step with vectors / one cell: perturbed FP32 16^3 6.9 / 5.0, 64^3
-    // 10.6 / 8.8, lattice FP32 48^3 6.1 / 5.2, 80^3 9.7 / 9.0, 100^3 13.0 / 14.5;
-    // lattice FP64 32^3 5.4 / 4.8, 48^3 6.5 / 6.6, 64^3 7.7 / 9.5).
-    // Its offsets: 32 bits in FP32 (us per acoustic step of perturbed meshes with
-    // 64 / 32: 48^3 6.30 / 5.87, 64^3 8.39 / 8.08), 64 in FP64, where 32 cost (48^3
-    // 9.08 / 9.57, 128^3 130 / 140) and 64 save registers.
+    // Offsets of one cell per thread: 32 bits in FP32, 64 in FP64 (us per acoustic
+    // step of perturbed meshes with 64 / 32: FP32 48^3 6.30 / 5.87, 64^3 8.39 /
+    // 8.08; FP64 48^3 9.08 / 9.57, 128^3 130 / 140).
     // (A plane's y- and z-faces are one row or column more than its cells.)
     const bool small = star::small_plane<T>(m->Y + 1, m->Z + 1);
-    if (m->Z >= star::kWidth<T> && small && !star::narrow<T>(m->N)) {
+    if (m->Z >= star::kWidth<T> && small && m->N > one_cell_limit<T>(op, m->lattice)) {
         with_width(std::integral_constant<int, star::kWidth<T>>{}, uint32_t(0));
     } else {
         bool done = false;
@@ -416,15 +453,16 @@ template <class T, class F> void with_faces(const cfd_mesh_s* m, F f) {
 
 template <class T>
 void launch_grad_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, int wall, hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
+    with_faces<T>(m, Op::grad, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
         fgrad_k<T, decltype(w)::value, decltype(geo)::value, decltype(off)>
             <<<gr, bl, 0, s>>>(g, (const T*)phi, (T*)out, mask, wall, pl);
     });
 }
 
 template <class T> void launch_lapl_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask, hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
-        flapl_k<T, decltype(w)::value, decltype(geo)::value, decltype(off)><<<gr, bl, 0, s>>>(g, (const T*)phi, (T*)out, mask, pl);
+    with_faces<T>(m, Op::lapl, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
+        flapl_k<T, decltype(w)::value, decltype(geo)::value, decltype(off)>
+            <<<gr, bl, 0, s>>>(g, (const T*)phi, (T*)out, mask, pl);
     });
 }
 
@@ -433,7 +471,7 @@ void launch_stab_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask
     T* gx = (T*)scratch3;
     T* gy = gx + m->N;
     T* gz = gy + m->N;
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
+    with_faces<T>(m, Op::stab, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
         constexpr int W = decltype(w)::value, GEO = decltype(geo)::value;
         using O = decltype(off);
         fgrad3_k<T, W, GEO, O><<<gr, bl, 0, s>>>(g, (const T*)phi, gx, gy, gz, pl);
@@ -445,7 +483,7 @@ void launch_stab_faces(const cfd_mesh_s* m, const void* phi, void* out, int mask
 template <class T>
 void launch_heat_faces(const cfd_mesh_s* m, const void* in, void* out, double alpha, const void* af, double dt,
                        hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
+    with_faces<T>(m, Op::heat, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
         constexpr int W = decltype(w)::value, GEO = decltype(geo)::value;
         using O = decltype(off);
         auto* kern = af ? fheat_k<T, W, GEO, O, true> : fheat_k<T, W, GEO, O, false>;
@@ -456,7 +494,7 @@ void launch_heat_faces(const cfd_mesh_s* m, const void* in, void* out, double al
 template <class T>
 void launch_wave_faces(const cfd_mesh_s* m, void* const* in, void* const* out, double K, const void* Kf, double dt,
                        hipStream_t s) {
-    with_faces<T>(m, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
+    with_faces<T>(m, Op::wave, [&](const Plan& pl, dim3 gr, dim3 bl, auto w, auto geo, auto off, const auto& g) {
         constexpr int W = decltype(w)::value, GEO = decltype(geo)::value;
         using O = decltype(off);
         fwave_vel_k<T, W, GEO, O><<<gr, bl, 0, s>>>(g, (const T*)in[0], (const T*)in[1], (const T*)in[2],

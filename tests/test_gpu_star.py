@@ -274,6 +274,17 @@ def test_launch_geometry_of_long_perturbed_meshes(hip_ctx, oracle_lib, n, dtype)
     _check_against_oracle(*_mesh(hip_ctx, oracle_lib, n, "skewed", dtype), dtype)
 
 
+# either side of the sizes up to which an operator takes one cell per thread
+# (2^15 and 2^16 cells in FP64; 2^18, 2^19, 2^21 and 2^22 in FP32)
+@pytest.mark.parametrize("kind", ["decimal", "skewed"])
+@pytest.mark.parametrize("dtype,n", [(np.float64, (32, 31, 33)), (np.float64, (32, 33, 33)), (np.float64, (41, 40, 41)),
+                                     (np.float32, (63, 64, 65)), (np.float32, (64, 65, 65)), (np.float32, (81, 80, 82)),
+                                     (np.float32, (130, 128, 127)), (np.float32, (163, 161, 161))],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else np.dtype(v).name)
+def test_widths_of_face_geometry_kernels(hip_ctx, oracle_lib, n, kind, dtype):
+    _check_against_oracle(*_mesh(hip_ctx, oracle_lib, n, kind, dtype), dtype)
+
+
 def _check_against_oracle(gm, gg, om, dtype):
     """Every operator and step of the mesh against the oracle's."""
     gg.close()
