@@ -67,14 +67,14 @@ template <class T, int W, class O> __device__ inline void store(T* base, O off, 
 // reciprocal rounded up to 32 significant bits, exact for these k (the
 // hardware has no integer division, and a workgroup's first loads wait for it).
 struct Div {
-    uint32_t m, s;  // k / n = (k m) >> (32 + s); m = 0 for n = 1
-    __device__ int operator()(int k) const { return m ? int(__umulhi(uint32_t(k), m) >> s) : k; }
+    uint32_t n, m, s;  // k / n = (k m) >> (31 + s)
+    __device__ int operator()(int k) const { return int(__umulhi(uint32_t(k) << 1, m) >> s); }
 };
 inline Div make_div(int64_t n) {
     Div d{};
-    if (n == 1) return d;
-    while ((int64_t(2) << d.s) < n) ++d.s;
-    d.m = uint32_t(((uint64_t(1) << (32 + d.s)) + uint64_t(n) - 1) / uint64_t(n));
+    d.n = uint32_t(n);
+    while ((int64_t(1) << d.s) < n) ++d.s;
+    d.m = uint32_t(((uint64_t(1) << (31 + d.s)) + uint64_t(n) - 1) / uint64_t(n));
     return d;
 }
 
@@ -163,12 +163,16 @@ template <int W> __device__ inline bool place_at(const Plan& p, int b, int padde
     const int lin = (b % 8) * (padded / 8) + b / 8;
     if (lin >= p.blocks) return false;
     // blocks of the run's cut axis outermost: (x, y, z), (y, x, z) or (z, x, y)
-    const int n0 = p.cut == 2 ? p.nyb : p.nzb, n1 = p.cut == 0 ? p.nyb : p.X;
-    const int row = p.d0(lin), in = lin - row * n0;
-    const int out = p.d1(row), mid = row - out * n1;
-    const int zb = p.cut == 2 ? out : in;
-    q.x = p.cut == 0 ? out : mid;
-    q.y = (p.cut == 0 ? mid : p.cut == 1 ? out : in) * p.by + ty;
+    const int row = p.d0(lin), in = lin - row * int(p.d0.n);
+    const int out = p.d1(row), mid = row - out * int(p.d1.n);
+    int zb = in, yb = mid;
+    q.x = out;
+    if (p.cut) {
+        q.x = mid;
+        yb = p.cut == 1 ? out : in;
+        if (p.cut == 2) zb = out;
+    }
+    q.y = yb * p.by + ty;
     const int zi = zb * p.bx + tx;
     if (ty >= p.by || q.y >= p.Y || zi * W >= p.Z) return false;
     q.z0 = min(zi * W, p.Z - W);
