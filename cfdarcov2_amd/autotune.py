@@ -1,8 +1,8 @@
 """Autotuner for the fused kernels' block and tile shapes.
 
 For a given mesh it times every candidate shape of the fused acoustic step
-(per-thread kernel; 2.5D marching kernel over tile rows x x-chunk x XCD
-placement) with HIP events on the launch stream, keeps the fastest, and caches
+(star form; 2.5D marching kernel over tile rows x x-chunk x XCD placement; row
+forms of one and two steps per launch) with HIP events on the launch stream, keeps the fastest, and caches
 the choice per (kernel, dtype, mesh extents) in a JSON file
 (``$CFDARCO_TUNE_CACHE``, default ``~/.cache/cfdarco/tune.json``).  Results are
 state-independent (the kernels do the same work for any data), so tuning runs
@@ -151,7 +151,7 @@ HEAT_CANDIDATES = [(0, 8, 16)] + [(1, w, L) for w in (8, 12, 16) for L in (1, 2,
 
 
 def tune_heat(mesh, alpha, dt, steps=100, candidates=None, verbose=False) -> dict:
-    """Pick the fastest heat-step form for `mesh` (per-thread, two steps per
+    """Pick the fastest heat-step form for `mesh` (star form, two steps per
     launch in row form with its waves and chunk, or several steps per launch
     in LDS boxes) from runs on scratch fields, each timed twice (the faster
     run counts: a step can be as short as a few microseconds); forms the mesh

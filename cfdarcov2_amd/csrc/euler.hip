@@ -508,8 +508,7 @@ template <class T> __device__ inline T at(const T* base, uint32_t boff) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + boff);
 }
 
-
-template <class T, int GEO>
+template <class T>
 __device__ inline void axis_faces(T Ax, T Ay, T Az, T (&f)[6][4]) {
 #pragma unroll
     for (int fc = 0; fc < 6; ++fc) {
@@ -575,7 +574,7 @@ __global__ void __launch_bounds__(B) euler_tile_k(typename TileGeo<T, GEO>::type
 
     T fg[6][4] = {};
     T wyz = T(0), wy = T(0), wz = T(0);
-    if constexpr (GEO == 1) axis_faces<T, GEO>(g.A[0], g.A[1], g.A[2], fg);
+    if constexpr (GEO == 1) axis_faces<T>(g.A[0], g.A[1], g.A[2], fg);
     if constexpr (GEO == 2) {
         wy = g.w[1][y];
         wz = g.w[2][z];
@@ -606,7 +605,7 @@ __global__ void __launch_bounds__(B) euler_tile_k(typename TileGeo<T, GEO>::type
         face4(2, x0 * SX, bc, fg[4]);
     }
     fetch(x0);
-    if constexpr (GEO == 2) axis_faces<T, GEO>(wyz, T(0), T(0), fg);
+    if constexpr (GEO == 2) axis_faces<T>(wyz, T(0), T(0), fg);
     {
         qc = prim(gamma, Uc);
         Prim<T> ql = qc;
@@ -636,7 +635,7 @@ __global__ void __launch_bounds__(B) euler_tile_k(typename TileGeo<T, GEO>::type
         }
         if constexpr (GEO == 2) {
             const T wx = g.w[0][x];
-            axis_faces<T, GEO>(wyz, wx * wz, wx * wy, fg);
+            axis_faces<T>(wyz, wx * wz, wx * wy, fg);
         }
         T Un[5];
 #pragma unroll
@@ -712,11 +711,11 @@ __global__ void __launch_bounds__(256) euler_dt_axis_k(FvAxis<T> g, EIn<T> in, i
 #pragma unroll
         for (int k = 0; k < 5; ++k) U[k] = in.u[k][i];
         if constexpr (GEO == 1) {
-            axis_faces<T, GEO>(g.A[0], g.A[1], g.A[2], fg);
+            axis_faces<T>(g.A[0], g.A[1], g.A[2], fg);
         } else {
             const int y = c / Z, z = c - y * Z;
             const T wx = g.w[0][x], wy = g.w[1][y], wz = g.w[2][z];
-            axis_faces<T, GEO>(wy * wz, wx * wz, wx * wy, fg);
+            axis_faces<T>(wy * wz, wx * wz, wx * wy, fg);
             V = g.vol[i];
         }
         loc = local_dt_faces(V, prim(gamma, U), fg);

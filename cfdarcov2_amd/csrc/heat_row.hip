@@ -7,7 +7,7 @@
 // (256/Z rows per wave, four cells per lane) and marches x over a chunk of
 // planes; the tile code is row::heat_row2_tile (row.hpp).  Two launches of two
 // steps each leave the state where four single steps would, so runs go in
-// pairs and the remaining steps take the per-thread kernel.
+// pairs and the remaining steps take the star form.
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"

@@ -9,13 +9,14 @@
 // Consecutive planes run on one XCD, so both cells of a face find its geometry
 // in one L2.
 //
-// Bound by the face arrays (a general FP64 heat cell reads 144 bytes of them, a
-// lattice's 8).  us before (one cell per thread, 64-bit indices, planes spread
-// over the XCDs) and now, 200^3 FP32: perturbed mesh, gradient 156 / 100,
-// Laplacian 180 / 122, stabilisation 526 / 288; on a decimal lattice 527 / 128;
-// FP64 perturbed 292 / 197, 328 / 241, 994 / 583 and decimal 994 / 278.  Steps on
-// decimal lattices: heat 100^3 FP64 38.4 / 6.7, acoustic 120x100x80 FP32
-// 49.0 / 14.0.
+// Bound by the geometry: beside its 16 bytes of state an FP64 heat cell of a
+// general mesh moves 128 (three faces of normal, area and alpha_d, 120, and the
+// volume), of a lattice 8.  us before (one cell per thread, 64-bit indices,
+// planes spread over the XCDs) and now, 200^3 FP32: perturbed mesh, gradient 156
+// / 99, Laplacian 180 / 122, stabilisation 526 / 288; on a decimal lattice 527 /
+// 128; FP64 perturbed 292 / 194, 328 / 239, 994 / 583 and decimal 994 / 278.
+// Steps on decimal lattices: heat 100^3 FP64 38.4 / 6.6, acoustic 120x100x80
+// FP32 49.0 / 14.0.
 //
 // The arithmetic is the reference's (src/fvm3d.cpp:825-829,902-942 and
 // :690-692 with include/grad_utils.hpp:23-125) in its order, sums over the six

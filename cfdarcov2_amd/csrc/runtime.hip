@@ -269,9 +269,9 @@ template <class T> static void create_mesh(cfd_mesh_s* m, const cfd_hex_desc& d)
         // Acoustic step.  While both states (8 fields) fit the last-level
         // cache the star form is the fastest measured at every size and
         // extent (us/step, star / best row form / best march tiles; FP32
-        // 48^3: 3.3 / 5.2 / 6.5, 128^3: 14.5 / 14.3 / 20.2, 200^3: 42.7 /
-        // 48.6 / 63.7; FP64 128^3: 23.0 / 26.5 / 28.3); its re-read rows cost
-        // it beyond (FP32 256^3: 155 / 71 / 140; FP64 200^3: 149 / 106 / 154).
+        // 48^3: 3.3 / 5.2 / 6.5, 128^3: 13.1 / 14.3 / 20.2, 200^3: 40.7 /
+        // 48.6 / 63.7; FP64 128^3: 22.8 / 26.5 / 28.3); its re-read rows cost
+        // it beyond (FP32 256^3: 155 / 71 / 140; FP64 200^3: 136 / 106 / 154).
         if (8 * d.nx * d.ny * d.nz * int64_t(sizeof(T)) <= kLastLevelCacheBytes) {
             m->wave_variant = 0;
         } else if (wave_row_supported(d.nz)) {

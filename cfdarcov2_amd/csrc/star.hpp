@@ -144,10 +144,12 @@ template <class T> inline bool vector_form(int64_t Y, int64_t Z) { return Z >= k
 
 // Whether a step of a mesh of this size is better with one cell per thread: a
 // launch then lasts about as long as one wavefront's chain of operations, and
-// the chain of W cells is longer than the chip needs to be filled (acoustic
-// step, us with one cell per thread / with vectors: FP32 16^3 2.4 / 2.9, 48^3
-// 2.8 / 3.3, 80^3 5.3 / 5.9, 100^3 8.6 / 8.0; FP64 16^3 2.4 / 3.0, 48^3 3.93 /
-// 3.98, 56^3 5.5 / 4.7).
+// the chain of W cells is longer than the chip needs to be filled.  Kernel times
+// (steps replayed from a graph; a run launched step by step takes the host's 3
+// to 4 us per launch where that is longer), us with one cell per thread / with
+// vectors: acoustic step FP32 16^3 2.5 / 3.0, 48^3 2.9 / 3.3, 80^3 5.3 / 5.9,
+// 100^3 8.5 / 7.9; FP64 16^3 2.5 / 3.2, 48^3 4.1 / 4.1, 56^3 5.7 / 4.8; transposed
+// step FP32 48^3 4.8 / 5.5, 72^3 6.8 / 6.7, FP64 48^3 5.8 / 5.6.
 template <class T> inline bool narrow(int64_t cells) {
     return cells <= (sizeof(T) == 4 ? int64_t(1) << 19 : int64_t(1) << 17);
 }

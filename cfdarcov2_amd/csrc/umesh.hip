@@ -18,9 +18,9 @@
 // Cuthill-McKee numbering keeps the six neighbours of a cell, and so the
 // gathered values, within a few cache lines of the cell's own.
 //
-// Bound by the gathers: 96^3 FP64 moves 186 algorithmic bytes per cell and
-// heat step (ids, records, alpha, volume, state) at 6.5 TB/s from the
-// last-level cache.  us/step at 96^3, heat / acoustic, FP64 (FP32): blocks in
+// Bound by the gathers: 96^3 FP64 moves 193 algorithmic bytes per cell and
+// heat step (ids 48, volume 8, state 16, three faces' records and alpha 121) at
+// 6.7 TB/s from the last-level cache.  us/step at 96^3, heat / acoustic, FP64 (FP32): blocks in
 // launch order, faces by their lowest cell, one array per component 43.6 / 86.6
 // (26.2 / 55.2); contiguous runs of blocks per XCD, so a face's second gather
 // hits that L2, 29.6 / 64.1 (20.9 / 45.3); faces by local index and cell,

@@ -2,9 +2,10 @@
 // star.hpp for the form and star_wave.hpp for the step.
 //
 // Bound by its arithmetic (104 operations per cell against the march's 59) and
-// the launch: 48^3 FP32 2.8 us/step in a captured graph (3.3 launched one by one), 128^3 FP32 14.5 (4.6 TB/s), 90x77x123
-// FP64 12.0 us/step against 167 for the 16-row march tile, whose 30 workgroups
-// left most of the chip idle.
+// the launch: 48^3 FP32 2.9 us of kernel per step (3.3 to 4.2 launched one by
+// one, the host's cost), 128^3 FP32 13.1 (5.1 TB/s), 90x77x123 FP64 12.2 us/step
+// against 167 for the 16-row march tile, whose 30 workgroups left most of the
+// chip idle.
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
