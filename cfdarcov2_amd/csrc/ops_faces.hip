@@ -418,13 +418,17 @@ template <class T> int64_t one_cell_limit(Op op, bool lattice) {
 // f(plan, grid, block, width, geometry kind, offset, geometry): width and kind
 // as integral constants, the offset a value of its type
 template <class T, class F> void with_faces(const cfd_mesh_s* m, Op op, F f) {
+    // Face arrays beyond half the last-level cache on meshes long in z: runs of
+    // columns (us, cut in x / z: heat step FP64 40x40x1000 44.9 / 39.6, 60x60x2000
+    // 246 / 216, FP32 40x40x2000 45.2 / 39.7; below that size FP32 40x40x1000 22.1
+    // / 24.6).  The steps take one cell per thread there (with vectors / one, both
+    // cut in z: acoustic step FP64 40x40x1000 95.5 / 87.8, 60x60x2000 480 / 472,
+    // 64x64x512 130 / 134, FP32 40x40x2000 90.7 / 83.1; heat step FP64 39.6 / 37.1,
+    // 216 / 214, 57.8 / 58.9).
+    const bool long_z = !m->lattice && m->Z >= 8 * std::max(m->X, m->Y) &&
+                        2 * 17 * m->N * int64_t(sizeof(T)) > kLastLevelCacheBytes;
+    const bool one = m->N <= one_cell_limit<T>(op, m->lattice) || (long_z && (op == Op::heat || op == Op::wave));
     auto with_width = [&](auto w, auto off) {
-        // Face arrays beyond half the last-level cache on meshes long in z: runs
-        // of columns (us, cut in x / z: heat step FP64 40x40x1000 44.8 / 39.4,
-        // 60x60x2000 246 / 216, FP32 40x40x2000 45.2 / 39.7; below that size
-        // FP32 40x40x1000 22.1 / 24.6).
-        const bool long_z = !m->lattice && m->Z >= 8 * std::max(m->X, m->Y) &&
-                            2 * 17 * m->N * int64_t(sizeof(T)) > kLastLevelCacheBytes;
         const Plan pl = star::make_plan(m->X, m->Y, m->Z, w(), 0, long_z);
         const dim3 grid = star::plan_grid(pl), block = star::plan_block(pl);
         if (m->lattice) f(pl, grid, block, w, std::integral_constant<int, 2>{}, off, lg<T>(m));
@@ -435,7 +439,7 @@ template <class T, class F> void with_faces(const cfd_mesh_s* m, Op op, F f) {
     // 8.08; FP64 48^3 9.08 / 9.57, 128^3 130 / 140).
     // (A plane's y- and z-faces are one row or column more than its cells.)
     const bool small = star::small_plane<T>(m->Y + 1, m->Z + 1);
-    if (m->Z >= star::kWidth<T> && small && m->N > one_cell_limit<T>(op, m->lattice)) {
+    if (m->Z >= star::kWidth<T> && small && !one) {
         with_width(std::integral_constant<int, star::kWidth<T>>{}, uint32_t(0));
     } else {
         bool done = false;

@@ -119,7 +119,7 @@ inline Plan make_plan(int64_t X, int64_t Y, int64_t Z, int W, int threads = 0, b
     // heat step FP64 31.0 / 26.5).
     if (threads == 256 && p.by == 1 && Y >= 4 && 3 * p.bx < 2 * threads) split(3 * columns);
     if (long_z && units >= 64) {
-        split(std::max(8, (units + 63) / 64));
+        split(std::max(8, columns));  // at least one column per XCD; more have more halo (60x60x2000 FP64 241 / 216)
         p.cut = 2;
     } else {
         p.cut = Y >= 4 * X ? 1 : 0;
